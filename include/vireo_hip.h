@@ -192,7 +192,7 @@ int moe_ffn_forward(const vireo_moe_model *m, int layer, float *x, const float *
 /* moe_ffn_forward for callers that cannot allocate (code under HIP graph
  * capture, serving loops, harnesses that forbid hipMalloc): no counterpart in
  * the reference. The same results as moe_ffn_forward, but every intermediate
- * lives in a fixed 32 MiB region of device memory that the library holds per
+ * lives in a fixed 33 MiB region of device memory that the library holds per
  * device from its first use (vireo_hip_init, or the first call on a device)
  * until the process ends, and the call makes no allocation of any kind.
  * Limits: the layer must already be resident and pinned
@@ -220,11 +220,11 @@ int moe_ffn_forward_noalloc(const vireo_moe_model *m, int layer, float *x, const
  * through tagged records, where it is built for the shapes (d = 2048, k = 8,
  * up to 128 experts, expert width 768 or 1024, Q4_K/Q6_K or Q8_0 experts,
  * 256 CUs); its waits are bounded like plan 3's (vireo_hip_status).
- * Under plans 0 and 2, calls of at least 64 tokens run every group as bf16
- * matrix-core GEMMs (inputs and dequantized weights rounded
- * to bf16, fp32 accumulation; the layer's contribution then agrees with the
- * reference to about 1e-2 of its largest magnitude instead of 2e-3); the
- * routing is unaffected. */
+ * Under plans 0 and 2, calls of at least 64 tokens run every group as fp16
+ * matrix-core GEMMs (inputs, activations and dequantized weights rounded to
+ * fp16's 11 bits under power-of-two scales, fp32 accumulation; a token's
+ * contribution then agrees with the reference to about 4e-3 of its largest
+ * magnitude instead of 1e-5); the routing is unaffected. */
 int vireo_hip_set_path(int path);
 
 /* Decode-batch calls (5 to 63 tokens, or 3 and 4 under plan 2) on a pinned layer with Q4_K gate/up and
@@ -241,9 +241,10 @@ int vireo_hip_set_path(int path);
  * it. expert_store_packed_bytes reports the copies' bytes. A copy is made
  * from the pinned views and freed with the pin (expert_store_unpin_layer) or
  * the store; a caller that rewrites a pinned layer's expert bytes in place
- * must unpin and pin it again. Calls of 64 or more tokens on a pinned Q8_0 layer make
- * and read, the same way, a copy in matrix-operand fragments (each lane's
- * bytes of a 32-row, 64-column step together) for the prefill GEMMs. Results
+ * must unpin and pin it again. Calls of 64 or more tokens on a pinned layer of Q8_0, Q4_K
+ * or Q6_K experts make and read, the same way, a copy in matrix-operand
+ * fragments (each lane's words of a 32-row, 64-column step together; 1.0, 1.1
+ * and 1.07 times the expert bytes) for the prefill GEMMs. Results
  * are the same bit for bit either way. 0 turns both off for later calls
  * (existing copies stay until unpinned). No counterpart in the reference. */
 int vireo_hip_set_packed(int on);

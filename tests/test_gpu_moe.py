@@ -461,6 +461,45 @@ def test_grouped_plan_large_groups(cuda, oracle, path, name, T, zipf, plan):
     m.close()
 
 
+# gate/up and down types; fe = 1152 and 1280 take more than the 32 blocks of h
+# whose factors the down GEMM holds at a time
+EDGE_TYPES = [(W.Q4_K, W.Q6_K, 512), (W.Q8_0, W.Q8_0, 1152), (W.Q6_K, W.Q4_K, 1280)]
+
+
+@pytest.mark.parametrize("tg,td,fe", EDGE_TYPES)
+@pytest.mark.parametrize("T", [64, 67, 200, 700])
+def test_prefill_tiles_and_scales(cuda, oracle, tg, td, fe, T):
+    """The fp16 GEMMs of a call of 64+ tokens at the edges of their token tiles
+    (64 and 128 rows, remainders of 1 to 127) for every weight type, on the
+    fragment copy and on the GGUF rows (the same bits), with tokens whose
+    inputs differ by 2^12 in magnitude and their activations by 2^24. A
+    token's contribution passes seven fp16 roundings (input, scale and weight of
+    both projections, h), each at most 2^-11 of the largest: 4e-3 of it."""
+    lib = _lib.load()
+    shape = W.MoEShape("edge", 512, 8, 2, fe, True, tg, tg, td)
+    bias = np.linspace(0.0, 3.0, 8).astype(np.float32)  # groups of many sizes
+    m = M.DeviceMoE(shape, 1, seed=71, logit_bias=bias)
+    x, hb = W.host_hidden(shape.d, T, 71)
+    hb = hb * np.exp2(np.arange(T) % 13 - 6).astype(np.float32)[:, None]
+    hbt = torch.from_numpy(hb).to(cuda)
+    outs = []
+    try:
+        for packed in (0, 1):
+            _lib.check(lib.vireo_hip_set_packed(packed), "vireo_hip_set_packed")
+            xt = torch.zeros((T, shape.d), device=cuda)
+            idx, _ = m.forward(0, xt, hbt, return_routing=True)
+            outs.append(xt.cpu().numpy())
+    finally:
+        lib.vireo_hip_set_packed(1)
+    np.testing.assert_array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+    xo, io, _, _ = oracle_layer(oracle, m, 0, np.zeros_like(x), hb)
+    np.testing.assert_array_equal(idx.cpu().numpy(), io)
+    rel = np.abs(outs[1] - xo).max(1) / np.abs(xo).max(1)
+    print(f"T={T} fe={fe}: groups {np.bincount(io.ravel(), minlength=8)} max rel {rel.max():.2e}")
+    assert rel.max() <= 4e-3
+    m.close()
+
+
 def test_grouped_plan_large_groups_unregistered(cuda, oracle, path):
     """Unregistered experts among the matrix-core groups contribute nothing."""
     path(0)

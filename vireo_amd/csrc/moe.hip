@@ -10,7 +10,7 @@
 //                        grouped down -> combine + residual      (6 kernels)
 // The grouped plan reads each routed expert's weights once per call however
 // many tokens chose it. In calls of at least kMfmaMinCall tokens every group
-// runs as bf16 matrix-core GEMMs (moe_mfma.hip; 4 more kernels); calls of
+// runs as fp16 matrix-core GEMMs (moe_mfma.hip; 3 more kernels); calls of
 // kMdecMinTokens to kMfmaMinCall - 1 tokens with Q4_K_M experts run their
 // groups on the matrix cores with exact 16-bit operands (moe_mdec.hip), and
 // smaller calls (or other types) on moe_gdec.hip's kernels, which keep a
@@ -91,11 +91,12 @@ struct Ws {
     uint32_t *flags;
     uint32_t *bar;  // decode plan: kFusedBlocks barrier flags, then the token's flag word
     DecodePlan *plan;
-    int32_t *tiles, *small;  // matrix-core plan: token tiles, the other groups
-    void *hs;                // matrix-core plan: bf16 h rows in dispatch order
-    void *xb;                // matrix-core plan: bf16 copy of hb
+    int32_t *tiles;          // matrix-core plan: token tiles
+    void *hs;                // matrix-core plan: fp16 h rows in dispatch order
+    int8_t *he;              // and their block exponents [P x fe / 32]
+    void *xb;                // matrix-core plan: fp16 copy of hb
     void *xp;                // decode-batch matrix-core plan: split inputs [T x d x 4 bytes]
-    float *xsc;              // and their per-token scales [T]
+    float *xsc;              // either matrix-core plan's per-token scales [T]
     uint32_t *ctr;           // and the down kernel's arrival counters (vh_mdec_ctr_words)
     const void **tab;        // paged plan: [E + 1] expert tables [3 E] (one per batch, then the combine's)
     int32_t *act;            // paged plan: [E] active lists [E + 1] (one per batch)
@@ -117,7 +118,11 @@ int get_ws(int T, int E, int k, int d, int fe, bool experts, bool grouped, Ws *w
     const size_t P = size_t(T) * k;
     size_t off = 0;
     auto take = [&](size_t bytes) { const size_t o = off; off += al256(bytes); return o; };
-    const size_t o_parts = take(size_t(T) * E * sizeof(RoutePart));
+    // the matrix-core plan's exponents and scales take the router parts' place
+    // once the routing is done with them
+    const size_t parts_bytes = size_t(T) * E * sizeof(RoutePart);
+    const size_t he_bytes = mfma ? al256(P * (fe / 32)) : 0, side_bytes = mfma ? he_bytes + size_t(T) * 4 : 0;
+    const size_t o_parts = take(parts_bytes > side_bytes ? parts_bytes : side_bytes);
     const size_t o_idx = take(P * 4), o_w = take(P * 4), o_flags = take(size_t(T) * 4);
     const size_t o_plan = take(sizeof(DecodePlan));
     const size_t o_bar = take((kFusedBlocks + 1) * 4);
@@ -126,14 +131,13 @@ int get_ws(int T, int E, int k, int d, int fe, bool experts, bool grouped, Ws *w
     const size_t o_h = (experts && !mfma) ? take(P * fe * 4) : 0;  // the matrix cores keep h in hs
     const size_t o_y = (experts && grouped) ? take(P * d * 4) : 0;
     const size_t o_tiles = mfma ? take(size_t(vh_mfma_plan_words(int(P), E)) * 4) : 0;
-    const size_t o_small = mfma ? take(size_t(E + 1) * 4) : 0;
     const size_t o_hs = mfma ? take(P * fe * 2) : 0;
     const size_t o_xb = mfma ? take(size_t(T) * d * 2) : 0;
     const bool small = experts && grouped && T < kMfmaMinCall;
     const size_t o_xp = small ? take(vh_mdec_xp_bytes(T, d)) : 0, o_xsc = small ? take(size_t(T) * 4) : 0;
     const size_t o_ctr = small ? take(size_t(vh_mdec_ctr_words(d)) * 4) : 0;
-    const size_t ntab = paged ? size_t(E + 1) : 1, nact = paged ? size_t(E) : 1;
-    const size_t o_tab = take(ntab * 3 * E * sizeof(void *)), o_act = take(nact * (E + 1) * 4);
+    const size_t o_tab = paged ? take(size_t(E + 1) * 3 * E * sizeof(void *)) : 0,
+                 o_act = paged ? take(size_t(E) * (E + 1) * 4) : 0;
     const size_t o_pidx = paged ? take(P * 4) : 0, o_pw = paged ? take(P * 4) : 0,
                  o_pflags = paged ? take(size_t(T) * 4) : 0;
     void *base;
@@ -157,14 +161,16 @@ int get_ws(int T, int E, int k, int d, int fe, bool experts, bool grouped, Ws *w
     ws->h = (experts && !mfma) ? reinterpret_cast<float *>(b + o_h) : nullptr;
     ws->ybuf = (experts && grouped) ? reinterpret_cast<float *>(b + o_y) : nullptr;
     ws->tiles = mfma ? reinterpret_cast<int32_t *>(b + o_tiles) : nullptr;
-    ws->small = mfma ? reinterpret_cast<int32_t *>(b + o_small) : nullptr;
     ws->hs = mfma ? b + o_hs : nullptr;
+    ws->he = mfma ? reinterpret_cast<int8_t *>(b + o_parts) : nullptr;
     ws->xb = mfma ? b + o_xb : nullptr;
     ws->xp = small ? b + o_xp : nullptr;
-    ws->xsc = small ? reinterpret_cast<float *>(b + o_xsc) : nullptr;
+    ws->xsc = small  ? reinterpret_cast<float *>(b + o_xsc)
+              : mfma ? reinterpret_cast<float *>(b + o_parts + he_bytes)
+                     : nullptr;
     ws->ctr = small ? reinterpret_cast<uint32_t *>(b + o_ctr) : nullptr;
-    ws->tab = reinterpret_cast<const void **>(b + o_tab);
-    ws->act = reinterpret_cast<int32_t *>(b + o_act);
+    ws->tab = paged ? reinterpret_cast<const void **>(b + o_tab) : nullptr;
+    ws->act = paged ? reinterpret_cast<int32_t *>(b + o_act) : nullptr;
     ws->pidx = paged ? reinterpret_cast<int32_t *>(b + o_pidx) : nullptr;
     ws->pw = paged ? reinterpret_cast<float *>(b + o_pw) : nullptr;
     ws->pflags = paged ? reinterpret_cast<uint32_t *>(b + o_pflags) : nullptr;
@@ -453,18 +459,21 @@ extern "C" int moe_decode_phases(const vireo_moe_model *m, int n, const int *lay
 // made on the first call that may allocate (never under graph capture) and
 // held by the store with the pin; NULL: read the GGUF rows.
 // kind 0: the decode batch's tiles (vh_mdec_pack_layer), 1: the prefill
-// GEMMs' Q8_0 row octets (vh_mfma_pack_q8).
+// GEMMs' fragments (vh_mfma_pack).
 const void *const *packed_table(const vireo_moe_model *m, int layer, const void *const *table, bool may_alloc,
                                 hipStream_t s, int kind = 0) {
     if (!g_packed) return nullptr;
     const void *const *pt = vh_store_packed_table(m->es, layer, kind);
     if (pt || !may_alloc) return pt;
     const int E = m->n_experts, d = m->dim, fe = m->ffn_exp;
-    const uint64_t bytes = kind ? vh_mfma_pack_bytes(E, d, fe) : vh_mdec_pack_bytes(E, d, fe);
+    const vireo_moe_layer &L = m->layers[layer];
+    const uint32_t tg = L.gate_exps->ggml_type, td = L.down_exps->ggml_type;
+    const uint64_t bytes = kind ? vh_mfma_pack_bytes(tg, td, E, d, fe) : vh_mdec_pack_bytes(E, d, fe);
     void *buf = vh_store_packed_begin(m->es, layer, kind, bytes);
     if (!buf) return nullptr;  // over the store's capacity: read the GGUF rows
     void *tab = nullptr;
-    int rc = kind ? vh_mfma_pack_q8(table, E, d, fe, buf, &tab, s) : vh_mdec_pack_layer(table, E, d, fe, buf, &tab, s);
+    int rc = kind ? vh_mfma_pack(table, tg, td, E, d, fe, buf, &tab, s)
+                  : vh_mdec_pack_layer(table, E, d, fe, buf, &tab, s);
     if (!rc) rc = vh_store_set_packed(m->es, layer, kind, tab);
     if (rc) {
         (void)hipGetLastError();
@@ -789,19 +798,16 @@ int ffn_forward(const vireo_moe_model *m, int layer, float *x, const float *hb, 
     if (!rc && !mdec) rc = vh_dispatch(idx, P, E, ws.counts, ws.offs, ws.perm, mfma ? nullptr : ws.active, s);
     if (!rc && flags_out)
         rc = vh_check(hipMemcpyAsync(flags_out, ws.flags, size_t(n_tokens) * 4, hipMemcpyDeviceToDevice, s));
-    if (mfma) {  // every group on the matrix cores (its small list stays empty)
-        const int mt = vh_mfma_max_tiles(P, E);
-        // Q8_0 experts of a pinned layer: the fragment copy (made on the first such call that may allocate)
-        const void *const *pt =
-            (!rc && tg == VT_Q8_0 && td == VT_Q8_0) ? packed_table(m, layer, table, !src, s, 1) : nullptr;
-        // the tile plan and the GEMMs' bf16 inputs in one launch
-        if (!rc) rc = vh_mfma_plan(ws.counts, E, P, 1, tg, td, d, fe, ws.tiles, ws.small, hb, ws.xb,
-                                   int64_t(n_tokens) * d, s);
+    if (mfma) {  // every group on the matrix cores
+        // experts of a pinned layer: the fragment copy (made on the first such call that may allocate)
+        const void *const *pt = rc ? nullptr : packed_table(m, layer, table, !src, s, 1);
+        // the tile plan and the GEMMs' fp16 inputs in one launch
+        if (!rc) rc = vh_mfma_plan(ws.counts, ws.offs, E, n_tokens, k, tg, td, d, fe, ws.tiles, hb, ws.xb, ws.xsc, s);
         const void *const *tb = pt ? pt : table;
-        if (!rc) rc = vh_mfma_gateup(tg, ws.tiles, mt, ws.counts, ws.offs, ws.perm, tb, pt != nullptr, ws.xb, d, fe, k,
-                                     ws.hs, s);
-        if (!rc) rc = vh_mfma_down(td, ws.tiles, mt, ws.counts, ws.offs, ws.perm, tb, pt != nullptr, ws.hs, d, fe,
-                                   ws.ybuf, s);
+        if (!rc) rc = vh_mfma_gateup(tg, ws.tiles, P, E, ws.perm, tb, pt != nullptr, ws.xb, ws.xsc,
+                                     d, fe, k, ws.hs, ws.he, s);
+        if (!rc) rc = vh_mfma_down(td, ws.tiles, P, E, ws.perm, tb, pt != nullptr, ws.hs, ws.he,
+                                   d, fe, ws.ybuf, s);
     } else if (mdec) {
         // calls of a decode batch's size, Q4_K_M experts: the matrix cores
         if (!rc && !prepped) rc = vh_mdec_prep(hb, n_tokens, d, ws.xp, ws.xsc, s);
@@ -829,8 +835,10 @@ int ffn_forward(const vireo_moe_model *m, int layer, float *x, const float *hb, 
 
 // The workspace of moe_ffn_forward_noalloc: a fixed region of device memory
 // in the library's code object (each device holds its own copy until the
-// process ends), shared by every such call on a device.
-constexpr size_t kNoAllocScratchBytes = size_t(32) << 20;
+// process ends), shared by every such call on a device. 33 MiB: the calls whose
+// other intermediates fit 32 fit with the prefill GEMMs' block exponents of h
+// (a byte per 32 activations, at most a 64th of the rest).
+constexpr size_t kNoAllocScratchBytes = size_t(33) << 20;
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 void *g_scratch_dev[64];  // per device: scratch's device address (host code never uses the symbol itself)
 

@@ -1,26 +1,39 @@
-// bf16 matrix-core (MFMA) grouped GEMMs for the groups of large calls.
+// fp16 matrix-core (MFMA) grouped GEMMs for the groups of large calls.
 //
 // moe_ffn (src/gguf_run.c:193-213) runs every (token, expert) pair as two
 // matvecs; when a call carries many tokens, an expert's tokens form a group
 // and its projections become GEMMs: H_e = silu(X_e G_e^T) * (X_e U_e^T) and
 // Y_e = H_e D_e^T, with X_e the group's rows of hb gathered through the
 // dispatch permutation. Every group of a call of at least kMfmaMinCall
-// tokens runs here on v_mfma_f32_32x32x16_bf16 (a group smaller than a token
-// tile leaves the tile's other rows unused; the tile's cost is staging its
-// weights either way): the inputs are rounded to bf16, the weights are
-// dequantized exactly (src/gguf_compute.c:52-120) and then rounded to bf16
-// while they are staged, and products are accumulated in fp32.
+// tokens runs here on v_mfma_f32_32x32x16_f16 with fp32 accumulation.
 //
-// Tiles: a workgroup (512 threads) owns a token tile of 32, 64 or 128 rows of
-// one group (whole 128-row tiles, the remainder in the smallest that holds
-// it) and kBRows = 256 weight rows (gate/up: 128 rows of gate and the same
-// 128 rows of up; down: 256 rows), and steps over K in kBK = 64 columns. The
-// inputs pass through LDS as 16-byte chunks of 8 consecutive K values laid
+// Numbers: both operands are fp16 (11 significant bits) under power-of-two
+// scales, which cost nothing in precision and take fp16's narrow range out of
+// play: a token's inputs by its largest magnitude (to below 2^14), a weight
+// row by a bound on its largest magnitude (row_exponent), the activations h
+// per (pair, 32 columns) by the block's largest. A weight is formed from its
+// exact quant by packed fp16 operations: Q8_0 and Q6_K (q - 32) times the
+// rounded scale, Q4_K one fused d1 q - m1 on the rounded d1 and m1. On the
+// benchmark's shapes the layer's output lies 5 to 8 times closer to a 64-bit
+// evaluation than with both operands rounded to bf16, and a weight costs 1.5
+// (Q8_0), 1.6 (Q4_K) or 2.4 (Q6_K) vector instructions where bf16 rounding
+// through fp32 took 2.8 to 4.
+//
+// Tiles: a workgroup of four waves owns a token tile of 32, 64 or 128 rows of
+// one group and 256 weight rows, 64 per wave (gate/up: 32 of gate and the same
+// 32 of up; down: 64), and steps over K in kBK = 64 columns. Each wave
+// dequantizes its own 64 rows in registers and multiplies all of the tile's
+// rows by them, so a weight is converted once per workgroup and an input
+// fragment read from LDS feeds two multiplies (with 32 rows per wave the
+// operand reads alone took all of the LDS bandwidth). Only the inputs pass
+// through LDS, double buffered, as 16-byte chunks of 8 consecutive K values laid
 // out [K/8][row] (row index XOR-swizzled by the chunk), so a 32-lane group's
-// operand read is one contiguous 512-byte run. GGUF-row experts: four waves
-// multiply and four stage the weights through LDS too (mfma_proj_kernel);
-// pinned Q8_0 experts come from a copy in the operand order and every wave
-// multiplies, reading its own weights (mfma_frag_kernel).
+// operand read is one contiguous 512-byte run. Two workgroups share a CU:
+// 256 registers, two waves per SIMD, one converting while the other multiplies.
+//
+// Weights: the experts of a pinned layer come from a copy in the operand order
+// (Frag, vh_mfma_pack); others are read from their GGUF rows and rearranged in
+// registers into the same words, so the results do not depend on the source.
 //
 // Order: the workgroups are numbered so that each XCD (hardware dispatch sends
 // workgroup b to XCD b mod 8) takes a contiguous run of (token tile, column
@@ -28,9 +41,10 @@
 // the consecutive token tiles of one expert that share its weight tiles, meet
 // in the same L2. The runs are cut at equal shares of the staged bytes.
 //
-// Outputs: gate/up writes h as bf16 rows in dispatch order (hs[offs[e] + i]),
-// so the down GEMM reads its A operand contiguously; down writes the fp32 row
-// y[pair] that the combine kernel reads, as on the fp32 plan.
+// Outputs: gate/up writes h as fp16 rows in dispatch order (hs[offs[e] + i])
+// with their block exponents (he), so the down GEMM reads its A operand
+// contiguously; down writes the fp32 row y[pair] that the combine kernel reads,
+// as on the fp32 plan.
 #include <hip/hip_runtime.h>
 #include <vector>
 #include <algorithm>
@@ -41,665 +55,777 @@
 
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int kBM = 128, kBK = 64, kBRows = 256, kThreads = 512, kXcds = 8;
+constexpr int kBK = 64, kBRows = 256, kWaves = 4, kThreads = 64 * kWaves, kXcds = 8;
 constexpr int kChunks = kBK / 8;  // 16-byte chunks per row and K step
-#ifndef VH_MFMA_SETS
-#define VH_MFMA_SETS 2
-#endif
-// register sets of the staging waves: a step's global loads are issued
-// sets<T>() - 1 K steps before its words are dequantized into LDS (a Q4_K
-// set holds 64 registers, a Q6_K set 96: two fit)
+constexpr int kBufs = 3;          // LDS buffers of the inputs: the step's, the next one's, and the one being written
+constexpr int kBigTile = 128, kSmallTile = 64;  // the largest token tile of the two kernels (tile_rows)
+
+VH_DEV f16x2 as_h2(uint32_t v) { return __builtin_bit_cast(f16x2, v); }
+VH_DEV f16x2 splat(_Float16 v) { return f16x2{v, v}; }
+VH_DEV uint32_t h_bits(float v) { return __builtin_bit_cast(uint16_t, _Float16(v)); }
+
+// (a & m) | e with the operands in registers: the compiler's own form takes at
+// most one constant from outside the vector registers and splits in two
+VH_DEV uint32_t and_or(uint32_t a, uint32_t m, uint32_t e) {
+    uint32_t r;
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(m), "v"(e));
+    return r;
+}
+// constants that and_or and v_perm_b32 take from vector registers
+struct Consts {
+    uint32_t lo = 0x000f000fu, hi = 0x00f000f0u, e = 0x64006400u, h0 = 0x00300030u, h1 = 0x03000300u,
+             b = 0x64646464u;
+    VH_DEV Consts() { asm volatile("" : "+v"(lo), "+v"(hi), "+v"(e), "+v"(h0), "+v"(h1), "+v"(b)); }
+};
+
+// ---- operand words --------------------------------------------------------------
+// What a lane holds of one weight row r = lane % 32 of a 32-row fragment over
+// K step s (64 columns): the 32 weights of its half h = lane / 32 of the step,
+// columns 64 s + 32 h + 8 ks + j, of which it supplies j = 0..7 to sub-step ks =
+// 0..3 - NW words of quants and a word of their fp16 scales, under the row's
+// power of two. (The columns a multiply takes together are free as long as the
+// inputs' operand takes the same: the lanes of half h read input chunk 4 h + ks.)
+// get() forms sub-step ks's B operand.
 template <int T>
-constexpr int sets() { return (T & 0xff) == VT_Q8_0 ? VH_MFMA_SETS : 2; }
-
-// The raw bytes of 8 consecutive weights of one row - K chunk kc (columns
-// 64 s + 8 kc .. + 7) of K step s - and their dequantization to fp32 with the
-// reference's arithmetic (every value is that of gguf_dequant_row). Pos holds
-// what does not change with s (setup() takes the row's byte offset ro in the
-// 4-aligned tensor, under 4 GiB); Raw holds one step's words (load()); the
-// step enters the addresses only through uniform base pointers.
-template <int T>
-struct Chunk;
+struct Op;
 
 template <>
-struct Chunk<VT_Q8_0> {  // src/gguf_compute.c:112-120: y = qs * d, exact
-    // block (2 s + kc / 4) starts at ob + 68 s and the thread's 8 quant bytes
-    // at oq + 68 s, an even offset: one 8-byte load (global memory accepts any
-    // alignment), one 16-bit load of the scale
-    struct Pos {
-        uint32_t ob, oq;
-    };
-    struct Raw {
-        uint32_t d;
-        uint2 q;
-    };
-    static VH_DEV void setup(Pos &p, uint32_t ro, int kc) {
-        p.ob = ro + 34u * uint32_t(kc >> 2);
-        p.oq = p.ob + 2u + 8u * uint32_t(kc & 3);
-    }
-    static VH_DEV void load(const Pos &p, Raw &r, gbyte *m, int s) {
-        gbyte *ms = m + 68 * s;
-        r.d = ld_u16(ms + p.ob);
-        r.q = ld_u64(ms + p.oq);
-    }
-    static VH_DEV void values(const Pos &, const Raw &r, int, float (&v)[8]) {
-        // q + 128 as an unsigned byte, converted with v_cvt_f32_ubyte*; then
-        // (q + 128) * s - 128 * s is q * s exactly (at most 19 significant bits)
-        const float sc = h2f(r.d), off = -128.0f * sc;
-        uint32_t u0 = r.q.x ^ 0x80808080u, u1 = r.q.y ^ 0x80808080u;
-        asm volatile("" : "+v"(u0), "+v"(u1));
-        const uint32_t w[2] = {u0, u1};
+struct Op<VT_Q8_0> {  // src/gguf_compute.c:112-120: y = q d
+    // words 2 ks, 2 ks + 1: bytes q_j + 128; scale: the block's d
+    static constexpr int NW = 8, scale_bytes = 2;
+    static VH_DEV f16x8 get(const uint32_t (&w)[NW], uint32_t sc, int ks, const Consts &c) {
+        const f16x2 d = splat(as_h2(sc)[0]);
+        f16x8 o;
 #pragma unroll
-        for (int i = 0; i < 8; i++) v[i] = fmaf(float((w[i >> 2] >> (8 * (i & 3))) & 0xffu), sc, off);
+        for (int p = 0; p < 4; p++) {  // fp16 1024 + u is the byte u under the byte 0x64
+            const uint32_t v = __builtin_amdgcn_perm(w[2 * ks + (p >> 1)], c.b, (p & 1) ? 0x00070006u : 0x00050004u);
+            const f16x2 y = (as_h2(v) - splat(_Float16(1152.0f))) * d;
+            o[2 * p] = y[0];
+            o[2 * p + 1] = y[1];
+        }
+        return o;
     }
 };
 
 template <>
-struct Chunk<VT_Q4_K> {  // src/gguf_compute.c:52-66: y = (d*sc)*q - dmin*m
-    // step s lies in super-block s / 4 and its chunk pair s % 4 (both
-    // uniform); the thread's 8 nibbles are bytes 8 (kc % 4) .. + 7 of the
-    // pair's 32: low nibbles (sub-block 2 (s % 4)) for kc < 4, else high
-    struct Pos {
-        uint32_t ro, oq, hi;
-    };
-    struct Raw {
-        uint4 hdr;
-        uint2 q;
-    };
-    static VH_DEV void setup(Pos &p, uint32_t ro, int kc) {
-        p.ro = ro;
-        p.oq = ro + 16u + 8u * uint32_t(kc & 3);
-        p.hi = uint32_t(kc >> 2);
+struct Op<VT_Q4_K> {  // src/gguf_compute.c:52-66: y = d1 q - m1 (d1 = d sc, m1 = dmin m)
+    // word ks: nibble j at bit 16 (j % 2) + 4 (j / 2); scales: the sub-block's d1, m1
+    static constexpr int NW = 4, scale_bytes = 4;
+    static VH_DEV f16x8 get(const uint32_t (&w)[NW], uint32_t sc, int ks, const Consts &c) {
+        const f16x2 s = as_h2(sc), d = splat(s[0]), m = splat(s[1]), d16 = d * splat(_Float16(0.0625f));
+        const f16x2 k = splat(_Float16(1024.0f));
+        const uint32_t a = w[ks], b = a >> 8;
+        // bits 0-3 of each half give 1024 + q, bits 4-7 give 1024 + 16 q; both less 1024 are exact
+        const f16x2 p0 = __builtin_elementwise_fma(as_h2(and_or(a, c.lo, c.e)) - k, d, -m);
+        const f16x2 p1 = __builtin_elementwise_fma(as_h2(and_or(a, c.hi, c.e)) - k, d16, -m);
+        const f16x2 p2 = __builtin_elementwise_fma(as_h2(and_or(b, c.lo, c.e)) - k, d, -m);
+        const f16x2 p3 = __builtin_elementwise_fma(as_h2(and_or(b, c.hi, c.e)) - k, d16, -m);
+        return f16x8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
     }
-    static VH_DEV void load(const Pos &p, Raw &r, gbyte *m, int s) {
-        gbyte *ms = m + 144 * (s >> 2);
-        r.hdr = ld_u128(ms + p.ro);
-        r.q = ld_u64(ms + 32 * (s & 3) + p.oq);
-    }
-    static VH_DEV void values(const Pos &p, const Raw &r, int s, float (&v)[8]) {
-        int sc, mn;
-        q4k_scale_min(2 * (s & 3) + int(p.hi), r.hdr.y, r.hdr.z, r.hdr.w, sc, mn);
-        const float d1 = h2f(r.hdr.x & 0xffffu) * float(sc), m1 = h2f(r.hdr.x >> 16) * float(mn);
-        const uint32_t sh = 4u * p.hi;
-        uint32_t w0 = (r.q.x >> sh) & 0x0f0f0f0fu, w1 = (r.q.y >> sh) & 0x0f0f0f0fu;
-        asm volatile("" : "+v"(w0), "+v"(w1));
-        const uint32_t w[2] = {w0, w1};
-#pragma unroll
-        for (int i = 0; i < 8; i++)  // d1 * q is exact: one rounding, as in the reference
-            v[i] = fmaf(d1, float((w[i >> 2] >> (8 * (i & 3))) & 0xffu), -m1);
-    }
-};
-
-// 8 bytes at even byte offset c of a 4-aligned tensor, read as aligned words
-// that stay in [c - 2, c + 8) and shifted into place (by sh = c & 3 bytes)
-// when used. p points at c.
-struct Even8 {
-    uint32_t w0, w1, w2, sh;
-    VH_DEV void load(gbyte *p, uint32_t shift) {
-        sh = shift;
-        gbyte *a = p - sh;
-        w0 = ld_u32(a);
-        w1 = ld_u32(a + 4);
-        w2 = ld_u16(a + (sh ? 8 : 6));  // bytes c+6, c+7 (unused when sh == 0)
-    }
-    VH_DEV uint32_t lo() const { return align2(w1, w0, sh); }
-    VH_DEV uint32_t hi() const { return align2(w2, w1, sh); }
 };
 
 template <>
-struct Chunk<VT_Q6_K> {  // src/gguf_compute.c:83-103: y = (d*sc)*(q - 32)
-    // step s: super-block b = s / 4 at byte U = 210 b of the row, half
-    // h = (s % 4) / 2, both uniform. The thread's 8 elements are l = 8 (kc % 4)
-    // .. + 7 of group g = 2 (s % 2) + kc / 4: the low (g < 2) or high nibbles
-    // of ql[64 h + 32 (g % 2) + l], bits 2g of qh[32 h + l], scale
-    // [8 h + l / 16 + 2 g]. U is even, so a field's alignment is that of its
-    // offset within the row's first super-block plus 2 (b % 2).
-    struct Pos {
-        uint32_t oql, oqh, osc, od, gl;
-    };
-    struct Raw {
-        Even8 ql, qh;
-        uint32_t d, sc;
-    };
-    static VH_DEV void setup(Pos &p, uint32_t ro, int kc) {
-        const uint32_t l = 8u * uint32_t(kc & 3);
-        p.oql = ro + 32u * uint32_t(kc >> 2) + l;
-        p.oqh = ro + 128u + l;
-        p.osc = ro + 192u + (l >> 4) + 2u * uint32_t(kc >> 2);
-        p.od = ro + 208u;
-        p.gl = uint32_t(kc >> 2);
+struct Op<VT_Q6_K> {  // src/gguf_compute.c:83-103: y = (d sc) (q - 32)
+    // word ks: the low nibbles as Q4_K's; words 4, 5: the high 2 bits of
+    // sub-steps 0, 1 and 2, 3 - weight j of an even sub-step at bit 16 (j % 2)
+    // + {4, 8, 6, 10}[j / 2], of an odd one at 16 (j % 2) + {12, 0, 14, 2}[j / 2];
+    // scales: d sc of the two 16-weight sub-blocks (sub-steps 0, 1 and 2, 3)
+    static constexpr int NW = 6, scale_bytes = 4;
+    static VH_DEV int hi_bit(int ks, int j) {
+        const int p = j >> 1;
+        return 16 * (j & 1) + ((ks & 1) ? (p == 0 ? 12 : p == 1 ? 0 : p == 2 ? 14 : 2)
+                                        : (p == 0 ? 4 : p == 1 ? 8 : p == 2 ? 6 : 10));
     }
-    static VH_DEV void load(const Pos &p, Raw &r, gbyte *m, int s) {
-        const int b = s >> 2, h = (s & 3) >> 1;
-        gbyte *ms = m + 210 * b;
-        const uint32_t odd = 2u * uint32_t(b & 1);
-        r.ql.load(ms + 64 * h + p.oql, (p.oql + odd) & 3u);
-        r.qh.load(ms + 32 * h + p.oqh, (p.oqh + odd) & 3u);
-        r.sc = ld_u8(ms + 8 * h + 4 * (s & 1) + p.osc);
-        r.d = ld_u16(ms + p.od);
-    }
-    static VH_DEV void values(const Pos &p, const Raw &r, int s, float (&v)[8]) {
-        const uint32_t g = 2u * uint32_t(s & 1) + p.gl;
-        const float sc = h2f(r.d) * float(int(int8_t(r.sc)));
-        const uint32_t lsh = g >= 2 ? 4u : 0u, hsh = 2u * g;
-        uint32_t w0 = ((r.ql.lo() >> lsh) & 0x0f0f0f0fu) | (((r.qh.lo() >> hsh) & 0x03030303u) << 4);
-        uint32_t w1 = ((r.ql.hi() >> lsh) & 0x0f0f0f0fu) | (((r.qh.hi() >> hsh) & 0x03030303u) << 4);
-        asm volatile("" : "+v"(w0), "+v"(w1));
-        const uint32_t w[2] = {w0, w1};
-        // sc * q - 32 sc is sc * (q - 32) exactly before its one rounding, as
-        // in the reference's (d * sc) * (q - 32)
-#pragma unroll
-        for (int i = 0; i < 8; i++) v[i] = fmaf(sc, float((w[i >> 2] >> (8 * (i & 3))) & 0xffu), -32.0f * sc);
+    static VH_DEV f16x8 get(const uint32_t (&w)[NW], uint32_t sc, int ks, const Consts &c) {
+        const f16x2 d = splat(as_h2(sc)[ks >> 1]), d16 = d * splat(_Float16(0.0625f));
+        const f16x2 k0 = splat(_Float16(1056.0f)), k1 = splat(_Float16(1536.0f));
+        uint32_t h = w[4 + (ks >> 1)];
+        if (ks & 1) h = __builtin_amdgcn_perm(h, h, 0x02030001u);  // the bytes of each half swapped
+        const uint32_t a = w[ks], b = a >> 8, g = h >> 2;
+        // the 6-bit quant in place: 1024 + q, or 1024 + 16 q from bit 4
+        const f16x2 p0 = (as_h2(and_or(h, c.h0, and_or(a, c.lo, c.e))) - k0) * d;
+        const f16x2 p1 = (as_h2(and_or(h, c.h1, and_or(a, c.hi, c.e))) - k1) * d16;
+        const f16x2 p2 = (as_h2(and_or(g, c.h0, and_or(b, c.lo, c.e))) - k0) * d;
+        const f16x2 p3 = (as_h2(and_or(g, c.h1, and_or(b, c.hi, c.e))) - k1) * d16;
+        return f16x8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
     }
 };
 
-VH_DEV bf16x8 to_bf16(const float (&v)[8]) {
-    f32x8 f;
-#pragma unroll
-    for (int i = 0; i < 8; i++) f[i] = v[i];
-    return __builtin_convertvector(f, bf16x8);
+// The power of two a weight row's scales are multiplied by, as its exponent:
+// bound * 2^e lies in [2^13, 2^14) for a bound on the row's magnitudes (0 for
+// a row of zeros or with a scale that is not finite).
+VH_DEV int exponent_for(float bound) {
+    if (!(bound > 0.0f) || !(bound <= 3.4028234663852886e38f)) return 0;
+    int ex;
+    frexpf(bound, &ex);
+    return max(-100, min(100, 14 - ex));
 }
 
-// One token tile of BM rows (32, 64 or 128) against kBRows weight rows, by
-// the 512 threads of mfma_proj_kernel. A is bf16: GATEUP: xb [T x K], row
-// perm[i] / k; else hs [P x K], row i. GATEUP: B = gate and up rows, out = hs
-// (bf16 [P x rows], row i); else B = down rows, out = y (fp32 [P x rows], row
-// perm[i]). i runs over base + m0 .. + mcnt - 1 (mcnt <= BM) within the
-// group; rows of the tile past mcnt repeat the group's last row and are not
-// stored.
-//
-// Waves 0-3 only multiply: WM x WN of them share the tile (BM = 128 and 64:
-// 2 x 2, BM = 32: 1 x 4), wave c owning rows (BM / WM) (c / WN) .. + BM / WM - 1
-// and kBRows / WN of the weight rows (gate/up: as many columns of gate as of
-// up), FI x FJ 32 x 32 accumulator fragments. Waves 4-7 only stage: their
-// global loads run sets<T>() K steps ahead in register sets, and each step
-// they dequantize the set that arrived a step ago into the LDS buffer the
-// multiplying waves will read next. Every SIMD holds one wave of each kind,
-// so the matrix cores and the vector ALUs work at the same time; one barrier
-// per K step. A tile of fewer rows stages fewer input bytes per step for the
-// same weight bytes: small groups cost less than a full tile.
-template <int T, bool GATEUP, int BM>
-VH_DEV void mfma_tile(bf16x8 (&As)[2][kChunks][kBM], bf16x8 (&Bs)[2][kChunks][kBRows], int (&prow)[kBM], gbyte *M0,
-                      gbyte *M1, const int32_t *__restrict__ perm, const __bf16 *__restrict__ src, int K, int rows,
-                      int k, int64_t row_bytes, void *__restrict__ out, int base, int m0, int mcnt, int n0) {
-    static_assert(BM == 32 || BM == 64 || BM == 128, "token tiles of 32, 64 or 128 rows");
-    constexpr int NCOL = GATEUP ? kBRows / 2 : kBRows;  // output columns per workgroup
-    constexpr int WM = BM >= 64 ? 2 : 1, WN = 4 / WM;    // multiplying waves along rows, columns
-    constexpr int FI = BM / 32 / WM, FJ = kBRows / WN / 32;  // fragments per wave
-    constexpr int AQ = BM / 32;                          // input rows staged per staging thread
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int nk = K / kBK;
-    // down: the y row of each tile row (the dispatch permutation) in LDS for
-    // the epilogue, read once here (threads of the multiplying waves; the
-    // first barrier below publishes it): loaded under the epilogue's row
-    // condition, each store waited for its own load
-    if (!GATEUP && tid < BM) prow[tid] = perm[base + m0 + min(tid, mcnt - 1)];
+// GGUF rows: the loads of one lane and step (raw), their rearrangement into
+// operand words, and the row's blocks with the magnitude bound of one.
+template <int T>
+struct Rows;
 
-    if (wv >= 4) {
-        // ---- staging waves: thread p stages K chunk kc = p & 7 of A rows
-        // (p >> 3) + 32 q (q < AQ) and of B rows (p >> 3) + 32 q (q < 8).
-        // In LDS, chunk kc of row r sits at [kc][r ^ kc]: the 8 lanes of a row
-        // write 8 different bank groups, and a 32-lane operand read stays
-        // conflict-free. The K step enters the global addresses only through
-        // uniform base pointers.
-        const int p = tid - 256, kc = p & 7, rx = (p >> 3) ^ kc;
-        gbyte *abase = gmem(src);
-        uint32_t aoff[AQ];
-#pragma unroll
-        for (int q = 0; q < AQ; q++) {
-            const int i = base + m0 + min((p >> 3) + 32 * q, mcnt - 1);
-            aoff[q] = uint32_t((GATEUP ? size_t(perm[i] / k) : size_t(i)) * K * 2) + 16u * uint32_t(kc);
-        }
-        // B rows (p >> 3) + 32 q lie 32 q rows (gate/up: 32 (q % 4) rows of
-        // gate or up) past row p >> 3: one set of offsets, and per q a uniform
-        // base pointer (32 rows are a multiple of 4 bytes, so alignments agree)
-        using C = Chunk<T>;
-        constexpr int kSets = sets<T>();
-        typename C::Pos bp;
-        C::setup(bp, uint32_t(n0 + (p >> 3)) * uint32_t(row_bytes), kc);
-        gbyte *bm[8];
-#pragma unroll
-        for (int q = 0; q < 8; q++) bm[q] = (GATEUP && q >= 4 ? M1 : M0) + (GATEUP ? q & 3 : q) * 32 * row_bytes;
+// nibbles j = 0..7 (bytes of a, then of b, each below 16) in the order of Op<VT_Q4_K>
+VH_DEV uint32_t nibble_word(uint32_t a, uint32_t b) {
+    const uint32_t t = a | (b << 4);
+    const uint32_t u = __builtin_amdgcn_perm(t, t, 0x01010000u), v = __builtin_amdgcn_perm(t, t, 0x03030202u);
+    return (u & 0x000f000fu) | ((u >> 4) & 0x0f000f00u) | ((v << 4) & 0x00f000f0u) | (v & 0xf000f000u);
+}
 
-        struct Stage {
-            uint4 ah[AQ];
-            typename C::Raw bw[8];
-        } st[kSets];
-        auto load = [&](Stage &g, int step) {
-            gbyte *as = abase + 128 * step;
-#pragma unroll
-            for (int q = 0; q < AQ; q++) g.ah[q] = ld_u128(as + aoff[q]);
-#pragma unroll
-            for (int q = 0; q < 8; q++) C::load(bp, g.bw[q], bm[q], step);
-        };
-        auto store = [&](const Stage &g, int buf, int step) {
-#pragma unroll
-            for (int q = 0; q < AQ; q++) As[buf][kc][rx + 32 * q] = __builtin_bit_cast(bf16x8, g.ah[q]);
-#pragma unroll
-            for (int q = 0; q < 8; q++) {
-                float w[8];
-                C::values(bp, g.bw[q], step, w);
-                Bs[buf][kc][rx + 32 * q] = to_bf16(w);
-            }
-        };
-        // step t's words live in register set t % kSets: issued at step
-        // t - kSets, dequantized into LDS at step t - 1
-#pragma unroll
-        for (int j = 0; j < kSets; j++) load(st[j], min(j, nk - 1));
-        store(st[0], 0, 0);
-        lds_barrier();
-        for (int s0 = 0; s0 < nk; s0 += kSets) {
-#pragma unroll
-            for (int j = 0; j < kSets; j++) {
-                // step s: the multiplying waves read buffer s & 1
-                const int s = s0 + j;
-                if (s >= nk) break;
-                load(st[j], min(s + kSets, nk - 1));  // unconditional: the waits count only older loads
-                if (s + 1 < nk) store(st[(j + 1) % kSets], (s + 1) & 1, s + 1);
-                lds_barrier();  // LDS only: the loads in flight stay in flight
-            }
-        }
-        return;
+VH_DEV uint32_t u4_at(const uint4 &v, int i) { return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w; }
+
+template <>
+struct Rows<VT_Q8_0> {
+    struct Raw {
+        uint4 q[2];
+        uint32_t d;
+    };
+    static VH_DEV int blocks(int K) { return K / 32; }
+    static VH_DEV float bound(gbyte *row, int b) { return fabsf(h2f(ld_u16(row + 34 * b))) * 128.0f; }
+    static VH_DEV float step_bound(const Raw &r) { return fabsf(h2f(r.d)) * 128.0f; }
+    static VH_DEV void load(gbyte *row, int s, int half, Raw &r) {  // block 2 s + half
+        gbyte *p = row + 68 * s + 34 * half;
+        r.q[0] = ld_u128(p + 2);
+        r.q[1] = ld_u128(p + 18);
+        r.d = ld_u16(p);
     }
+    static VH_DEV void words(const Raw &r, int, int, float up, uint32_t (&w)[8], uint32_t &sc) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) w[i] = u4_at(r.q[i >> 2], i & 3) ^ 0x80808080u;
+        sc = h_bits(h2f(r.d) * up);
+    }
+};
 
-    // ---- multiplying waves: v_mfma_f32_32x32x16_bf16 (lane l supplies row
-    // l % 32, K values 8 (l / 32) .. + 7 of each operand; it holds column
-    // l % 32, rows 8 (r / 4) + 4 (l / 32) + r % 4 of the 32 x 32 result)
-    const int wm = wv / WN, wn = wv % WN;
-    // B rows of the wave's FJ 32-column fragments (gate/up: FJ / 2 of gate,
-    // the same FJ / 2 of up)
-    int bfr[FJ];
+template <>
+struct Rows<VT_Q4_K> {
+    struct Raw {
+        uint4 hdr, q[2];
+    };
+    static VH_DEV int blocks(int K) { return K / 256; }
+    static VH_DEV float bound_of(uint32_t h) {
+        return fmaxf(fabsf(h2f(h & 0xffffu)) * (63.0f * 15.0f), fabsf(h2f(h >> 16)) * 63.0f);
+    }
+    static VH_DEV float bound(gbyte *row, int b) { return bound_of(ld_u32(row + 144 * b)); }
+    static VH_DEV float step_bound(const Raw &r) { return bound_of(r.hdr.x); }
+    // step s: the 32 bytes s % 4 of super-block s / 4, low nibbles (sub-block 2 (s % 4)) for half 0, high for 1
+    static VH_DEV void load(gbyte *row, int s, int, Raw &r) {
+        gbyte *p = row + 144 * (s >> 2);
+        r.hdr = ld_u128(p);
+        r.q[0] = ld_u128(p + 16 + 32 * (s & 3));
+        r.q[1] = ld_u128(p + 32 + 32 * (s & 3));
+    }
+    static VH_DEV void words(const Raw &r, int s, int half, float up, uint32_t (&w)[4], uint32_t &sc) {
+        const int sh = 4 * half;
 #pragma unroll
-    for (int j = 0; j < FJ; j++)
-        bfr[j] = GATEUP ? (j < FJ / 2 ? 0 : NCOL) + (NCOL / WN) * wn + 32 * (j % (FJ / 2)) : (kBRows / WN) * wn + 32 * j;
-    f32x16 acc[FI][FJ];
+        for (int ks = 0; ks < 4; ks++)
+            w[ks] = nibble_word((u4_at(r.q[ks >> 1], 2 * (ks & 1)) >> sh) & 0x0f0f0f0fu,
+                                (u4_at(r.q[ks >> 1], 2 * (ks & 1) + 1) >> sh) & 0x0f0f0f0fu);
+        int a0, m0, a1, m1;
+        q4k_scale_min(2 * (s & 3), r.hdr.y, r.hdr.z, r.hdr.w, a0, m0);
+        q4k_scale_min(2 * (s & 3) + 1, r.hdr.y, r.hdr.z, r.hdr.w, a1, m1);
+        sc = h_bits(h2f(r.hdr.x & 0xffffu) * up * float(half ? a1 : a0)) |
+             h_bits(h2f(r.hdr.x >> 16) * up * float(half ? m1 : m0)) << 16;
+    }
+};
+
+template <>
+struct Rows<VT_Q6_K> {
+    struct Raw {
+        uint4 ql[2], qh[2];
+        uint32_t sc, d;
+    };
+    static VH_DEV int blocks(int K) { return K / 256; }
+    static VH_DEV float bound(gbyte *row, int b) { return fabsf(h2f(ld_u16(row + 210 * b + 208))) * (128.0f * 32.0f); }
+    static VH_DEV float step_bound(const Raw &r) { return fabsf(h2f(r.d)) * (128.0f * 32.0f); }
+    // step s: half h = (s % 4) / 2 of super-block s / 4, group g = 2 (s % 2) +
+    // `half`: weight l has its low bits in ql[64 h + 32 (g % 2) + l] (low nibbles
+    // for g < 2), its high bits 2 g of qh[32 h + l], its scale in scales[8 h + 2 g + l / 16]
+    static VH_DEV void load(gbyte *row, int s, int half, Raw &r) {
+        gbyte *p = row + 210 * (s >> 2);
+        const int h = (s & 3) >> 1;
 #pragma unroll
-    for (int i = 0; i < FI; i++)
-#pragma unroll
-        for (int j = 0; j < FJ; j++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
-    lds_barrier();  // buffer 0 staged
-    for (int s = 0; s < nk; s++) {
-        const int buf = s & 1;
+        for (int i = 0; i < 2; i++) {
+            r.ql[i] = ld_u128(p + 64 * h + 32 * half + 16 * i);
+            r.qh[i] = ld_u128(p + 128 + 32 * h + 16 * i);
+        }
+        r.sc = ld_u16(p + 192 + 8 * h + 2 * (2 * (s & 1) + half));
+        r.d = ld_u16(p + 208);
+    }
+    static VH_DEV void words(const Raw &r, int s, int half, float up, uint32_t (&w)[6], uint32_t &sc) {
+        const int sh = (s & 1) ? 4 : 0, g2 = 2 * (2 * (s & 1) + half);
+        w[4] = w[5] = 0;
 #pragma unroll
         for (int ks = 0; ks < 4; ks++) {
-            const int kg = 2 * ks + (lane >> 5), lx = (lane & 31) ^ kg;
-            bf16x8 a[FI], b[FJ];
+            const int i = 2 * (ks & 1);
+            w[ks] = nibble_word((u4_at(r.ql[ks >> 1], i) >> sh) & 0x0f0f0f0fu,
+                                (u4_at(r.ql[ks >> 1], i + 1) >> sh) & 0x0f0f0f0fu);
+            const uint32_t h0 = u4_at(r.qh[ks >> 1], i) >> g2, h1 = u4_at(r.qh[ks >> 1], i + 1) >> g2;
 #pragma unroll
-            for (int i = 0; i < FI; i++) a[i] = As[buf][kg][lx + (BM / WM) * wm + 32 * i];
-#pragma unroll
-            for (int j = 0; j < FJ; j++) b[j] = Bs[buf][kg][lx + bfr[j]];
-#pragma unroll
-            for (int i = 0; i < FI; i++)
-#pragma unroll
-                for (int j = 0; j < FJ; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+            for (int j = 0; j < 8; j++)
+                w[4 + (ks >> 1)] |= (((j < 4 ? h0 : h1) >> (8 * (j & 3))) & 3u) << Op<VT_Q6_K>::hi_bit(ks, j);
         }
-        lds_barrier();
+        const float d = h2f(r.d) * up;
+        sc = h_bits(d * float(int(int8_t(r.sc)))) | h_bits(d * float(int(int8_t(r.sc >> 8)))) << 16;
     }
+};
 
-    // epilogue
+// Fragment (group c, step s, j) of a packed matrix: a lane's words together,
+// 16 bytes of a lane at a time, then the lanes' scales. Group c of gate/up: rows
+// 32 c .. + 31 of gate (j = 0) and of up (j = 1); of down: rows 64 c + 32 j ..
+// + 31. It sits at ((c * nk + s) * 2 + j) * bytes; the rows' scales 2^-e follow
+// the fragments (gate's rows, then up's).
+template <int T>
+struct Frag {
+    static constexpr int NW = Op<T>::NW, SB = Op<T>::scale_bytes, bytes = 64 * (4 * NW + SB);
+    static VH_DEV void load(gbyte *p, int lane, uint32_t (&w)[NW], uint32_t &sc) {
+        const uint4 a = ld_u128(p + 16 * lane);
+        w[0] = a.x;
+        w[1] = a.y;
+        w[2] = a.z;
+        w[3] = a.w;
+        if constexpr (NW == 8) {
+            const uint4 b = ld_u128(p + 1024 + 16 * lane);
+            w[4] = b.x;
+            w[5] = b.y;
+            w[6] = b.z;
+            w[7] = b.w;
+        } else if constexpr (NW == 6) {
+            const uint2 b = ld_u64(p + 1024 + 8 * lane);
+            w[4] = b.x;
+            w[5] = b.y;
+        }
+        if constexpr (SB == 4) sc = ld_u32(p + 256 * NW + 4 * lane);
+        else sc = ld_u16(p + 256 * NW + 2 * lane);
+    }
+    static VH_DEV void store(uint8_t *p, int lane, const uint32_t (&w)[NW], uint32_t sc) {
+        *reinterpret_cast<uint4 *>(p + 16 * lane) = make_uint4(w[0], w[1], w[2], w[3]);
+        if constexpr (NW == 8) *reinterpret_cast<uint4 *>(p + 1024 + 16 * lane) = make_uint4(w[4], w[5], w[6], w[7]);
+        if constexpr (NW == 6) *reinterpret_cast<uint2 *>(p + 1024 + 8 * lane) = make_uint2(w[4], w[5]);
+        if constexpr (SB == 4) *reinterpret_cast<uint32_t *>(p + 256 * NW + 4 * lane) = sc;
+        else *reinterpret_cast<uint16_t *>(p + 256 * NW + 2 * lane) = uint16_t(sc);
+    }
+};
+
+struct GemmArgs {
+    const int32_t *tiles, *perm;
+    const void *const *table;
+    const uint8_t *src;   // A: gate/up: xb [T x K] fp16; down: hs [P x K] fp16
+    const float *xsc;     // gate/up: the tokens' scales [T]
+    int8_t *he;           // block exponents of hs [P x fe / 32] (gate/up writes, down reads)
+    void *out;            // gate/up: hs; down: y [P x rows]
+    int K, rows, k;
+    int64_t row_bytes;    // GGUF rows
+};
+
+// Half of a max-reduction of N pairs of values over lanes: lanes with `hi` set
+// keep m[r + N], the others m[r], each the larger of its own and of the lane
+// that CTRL reads (one whose `hi` is the other way).
+template <int CTRL, int N>
+VH_DEV void fold(float (&m)[16], bool hi) {
+#pragma unroll
+    for (int r = 0; r < N; r++) {
+        const float own = hi ? m[r + N] : m[r], other = hi ? m[r] : m[r + N];
+        m[r] = fmaxf(own, dpp_keep<CTRL>(other));
+    }
+}
+
+// 2^n as fp16 bits, n <= 0 (0 below 2^-24)
+VH_DEV uint32_t h_pow2(int n) { return n >= -14 ? uint32_t(15 + n) << 10 : n >= -24 ? 1u << (24 + n) : 0u; }
+
+constexpr int kFacBlocks = 32;  // blocks of h whose factors are in LDS at a time
+
+template <bool GATEUP, int LDB>
+struct TileLds {
+    f16x8 As[kBufs][kChunks][LDB];
+    float rsc[LDB];                                  // the rows' scales in the epilogue
+    float hsc[GATEUP ? kWaves : 1][32];              // gate/up: a wave's 32 row scales of h
+    int prow[GATEUP ? 1 : LDB];                      // down: the rows' y rows
+    uint16_t fac[GATEUP ? 1 : kFacBlocks][GATEUP ? 1 : LDB];  // and the factors of their blocks of h (fp16)
+};
+
+// One token tile of BM rows against the wave's two 32-row fragments, by the
+// kWaves waves of mfma_gemm_kernel. GATEUP: A row i is xb row perm[i] / k, the
+// weights gate and up, out = hs row i and its block exponents; else A row i is
+// hs row i, scaled to the row's largest block as it is staged, out = y row
+// perm[i]. i runs over base + m0 .. + mcnt - 1 (mcnt <= BM) within the group;
+// rows of the tile past mcnt repeat the group's last row and are not stored.
+//
+// K step s: the inputs of step s + 2 go from registers into LDS and those of s
+// + 3 are requested; the wave multiplies step s, forming its operands from the
+// weights requested two steps ago, and requests those of step s + 2. Every load
+// is unconditional (steps past the end repeat the last one), so the waits count
+// exactly the loads issued after the one needed, and the barrier is LDS-only:
+// loads stay in flight across it.
+template <int T, bool GATEUP, int BM, int LDB, bool PK>
+VH_DEV void gemm_tile(TileLds<GATEUP, LDB> &L, const GemmArgs &a, gbyte *M0, gbyte *M1, int base, int m0, int mcnt,
+                      int n0) {
+    using O = Op<T>;
+    constexpr int FI = BM / 32, AQ = BM * kChunks / kThreads;
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), half = lane >> 5;
+    const int K = a.K, nk = K / kBK;
+    const Consts cst;
+    // input staging: slot tid + 256 q holds K chunk kc = tid % 8 of tile row tid / 8 + 32 q
+    const int kc = tid & 7, rq = tid >> 3, nblk = K / 32;
+    gbyte *abase = gmem(a.src);
+    uint32_t aoff[AQ];
+#pragma unroll
+    for (int q = 0; q < AQ; q++) {
+        const int r = rq + 32 * q, i = base + m0 + min(r, mcnt - 1);
+        const int t = GATEUP ? a.perm[i] / a.k : i;
+        aoff[q] = uint32_t(size_t(t) * K * 2) + 16u * uint32_t(kc);
+        if constexpr (GATEUP) {
+            if (kc == 0) L.rsc[r] = a.xsc[t];
+        }
+    }
+    // down: the factors 2^(block exponent - row exponent) of kFacBlocks blocks of
+    // h, from block b0 on: two threads per row, half of the blocks each
+    auto factors = [&](int b0, int e) {
+        if (tid < 2 * BM) {
+            const int r = tid >> 1;
+            gbyte *he = gmem(a.he) + size_t(base + m0 + min(r, mcnt - 1)) * nblk;
+            uint32_t w[kFacBlocks / 8];
+#pragma unroll
+            for (int x = 0; x < kFacBlocks / 8; x++)  // nblk is a multiple of 4; words past the end repeat the last
+                w[x] = ld_u32(he + min(b0 + 4 * (kFacBlocks / 8 * (tid & 1) + x), nblk - 4));
+            if (b0 == 0) {  // the row's exponent: its largest block's
+                e = -128;
+#pragma unroll
+                for (int x = 0; x < kFacBlocks / 2; x++) e = max(e, int(int8_t(w[x >> 2] >> (8 * (x & 3)))));
+                for (int b = kFacBlocks + 4 * (tid & 1); b < nblk; b += 8) {
+                    const uint32_t v = ld_u32(he + b);
+#pragma unroll
+                    for (int x = 0; x < 4; x++) e = max(e, int(int8_t(v >> (8 * x))));
+                }
+                e = max(e, int(dpp_u<0xB1>(uint32_t(e))));
+                if (!(tid & 1)) {
+                    L.rsc[r] = ldexpf(1.0f, e - 14);
+                    L.prow[r] = a.perm[base + m0 + min(r, mcnt - 1)];
+                }
+            }
+#pragma unroll
+            for (int x = 0; x < kFacBlocks / 2; x++)
+                L.fac[kFacBlocks / 2 * (tid & 1) + x][r] = uint16_t(h_pow2(int(int8_t(w[x >> 2] >> (8 * (x & 3)))) - e));
+        }
+        return e;
+    };
+    uint4 av[AQ];
+    auto loadA = [&](int step) {
+#pragma unroll
+        for (int q = 0; q < AQ; q++) av[q] = ld_u128(abase + 128 * step + aoff[q]);
+    };
+    auto storeA = [&](int buf, int step) {
+#pragma unroll
+        for (int q = 0; q < AQ; q++) {
+            f16x8 v = __builtin_bit_cast(f16x8, av[q]);
+            if constexpr (!GATEUP) {
+                const _Float16 f = __builtin_bit_cast(_Float16, L.fac[(2 * step + (kc >> 2)) % kFacBlocks][rq + 32 * q]);
+                v = v * f16x8{f, f, f, f, f, f, f, f};
+            }
+            L.As[buf][kc][(rq ^ kc) + 32 * q] = v;
+        }
+    };
+
+    // the wave's weights: fragment group c of the packed matrix, or the lane's two GGUF rows
+    const int c = n0 / (GATEUP ? 32 : 64) + wv, col = lane & 31;
+    gbyte *fb = M0 + size_t(c) * nk * 2 * Frag<T>::bytes;
+    gbyte *row[2];
+    float up[2], rs[2];  // the rows' powers of two (GGUF rows) and, for the epilogue, their inverses
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const int r = GATEUP ? 32 * c + col : 64 * c + 32 * j + col;
+        if constexpr (PK) {
+            const size_t frags = size_t(GATEUP ? 2 : 1) * a.rows / 32 * nk * Frag<T>::bytes;
+            rs[j] = __uint_as_float(ld_u32(M0 + frags + 4 * (GATEUP ? j * a.rows + r : r)));
+        } else {
+            row[j] = (GATEUP && j ? M1 : M0) + int64_t(r) * a.row_bytes;
+        }
+    }
+    struct Words {
+        uint32_t w[O::NW], sc;
+    };
+    struct Raw {
+        typename Rows<T>::Raw g;
+    };
+    using Set = std::conditional_t<PK, Words, Raw>;
+    // GGUF rows are rearranged into words a step ahead, so one set of them is in flight
+    Set st[PK ? 2 : 1][2];
+    auto loadB = [&](Set (&g)[2], int step) {
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            if constexpr (PK) Frag<T>::load(fb + (size_t(step) * 2 + j) * Frag<T>::bytes, lane, g[j].w, g[j].sc);
+            else Rows<T>::load(row[j], step, half, g[j].g);
+        }
+    };
+
+    f32x16 acc[FI][2];
 #pragma unroll
     for (int i = 0; i < FI; i++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int row = (BM / WM) * wm + 32 * i + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-            if (row >= mcnt) continue;
-            const int pos = base + m0 + row;
-            if (GATEUP) {
-                __bf16 *hs = static_cast<__bf16 *>(out) + size_t(pos) * rows;
+        for (int j = 0; j < 2; j++)
 #pragma unroll
-                for (int jj = 0; jj < FJ / 2; jj++)
-                    hs[n0 + (NCOL / WN) * wn + 32 * jj + (lane & 31)] = __bf16(swiglu(acc[i][jj][r], acc[i][FJ / 2 + jj][r]));
-            } else {
-                float *y = static_cast<float *>(out) + size_t(prow[row]) * rows;
+            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
+
+    // The operands of sub-step ks + 1 are formed, and its input fragments read,
+    // between the multiplies of sub-step ks (across the step's barrier too: the
+    // inputs of step s + 1 have been in LDS since the barrier before), so a
+    // wave's vector instructions run in the shadow of its own multiplies.
+    int rowe = 0;  // down, threads 2 r and 2 r + 1: row r's exponent
+    f16x8 af[FI], b[2];
+    Words wd[2];
+    auto words = [&](Set (&g)[2], int s) {
 #pragma unroll
-                for (int j = 0; j < FJ; j++) y[n0 + (kBRows / WN) * wn + 32 * j + (lane & 31)] = acc[i][j][r];
+        for (int j = 0; j < 2; j++) {
+            if constexpr (PK) wd[j] = g[j];
+            else Rows<T>::words(g[j].g, s, half, up[j], wd[j].w, wd[j].sc);
+        }
+    };
+    // GGUF rows: a row's power of two follows from its first step's bound (below
+    // 2^11 under it) and is lowered, with what the row has accumulated, where a
+    // later bound would pass 2^15 under it: no pass over the row's scales ahead.
+    // Powers of two are exact, so the results are those of the packed copy's.
+    float fix[2];
+    auto row_bound = [&](Set &g) {  // of the row's step: both halves' (a finite bound, or 0)
+        if constexpr (PK) {
+            return 0.0f;
+        } else {
+            const float b = Rows<T>::step_bound(g.g), o = T == VT_Q8_0 ? __shfl_xor(b, 32, 64) : b;
+            return fmaxf(b, o);
+        }
+    };
+    auto rescale = [&](Set (&g)[2]) {
+        if constexpr (!PK) {
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const float bnd = row_bound(g[j]);
+                const float to = bnd * up[j] >= 32768.0f ? ldexpf(1.0f, exponent_for(bnd) - 3) : up[j];
+                fix[j] = to / up[j];
+                up[j] = to;
             }
         }
+    };
+    auto readA = [&](int buf, int ks, int i) {
+        const int kg = 4 * half + ks;
+        af[i] = L.As[buf][kg][(col ^ kg) + 32 * i];
+    };
+    auto step = [&](int s, int b0, int b1, int b2, Set (&cur)[2], Set (&nxt)[2]) {
+        if constexpr (!GATEUP)
+            if ((s + 2) % (kFacBlocks / 2) == 0 && s + 2 < nk) {  // the next blocks' factors (every 16 steps)
+                lds_barrier();
+                factors(2 * (s + 2), rowe);
+                lds_barrier();
+            }
+        storeA(b2, s + 2);
+        loadA(min(s + 3, nk - 1));
+        __builtin_amdgcn_sched_barrier(0);  // the loads stay where they are issued
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++) {
+            if (ks == 3) {
+                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (PK) loadB(cur, min(s + 2, nk - 1));
+                __builtin_amdgcn_sched_barrier(0);
+                rescale(nxt);
+                words(nxt, min(s + 1, nk - 1));
+                if constexpr (!PK) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    loadB(nxt, min(s + 2, nk - 1));
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            f16x8 bn[2];
+#pragma unroll
+            for (int j = 0; j < 2; j++) bn[j] = O::get(wd[j].w, wd[j].sc, (ks + 1) & 3, cst);
+#pragma unroll
+            for (int i = 0; i < FI; i++) {
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], b[j], acc[i][j], 0, 0, 0);
+                readA(ks < 3 ? b0 : b1, (ks + 1) & 3, i);
+            }
+            b[0] = bn[0];
+            b[1] = bn[1];
+#pragma unroll
+            for (int i = 0; i < 2 * FI; i++) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                    // a multiply
+                __builtin_amdgcn_sched_group_barrier(0x002, 20 / FI, 0);      // vector instructions
+                if (i & 1) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);         // an LDS read
+            }
+        }
+        if constexpr (!PK) {
+            if (__any(fix[0] != 1.0f || fix[1] != 1.0f))
+#pragma unroll
+                for (int i = 0; i < FI; i++)
+#pragma unroll
+                    for (int j = 0; j < 2; j++)
+#pragma unroll
+                        for (int r = 0; r < 16; r++) acc[i][j][r] *= fix[j];
+        }
+        lds_barrier();
+    };
+    loadB(st[0], 0);
+    if constexpr (PK) loadB(st[1], min(1, nk - 1));
+    loadA(0);
+    if constexpr (!GATEUP) {
+        rowe = factors(0, 0);
+        lds_barrier();
+    }
+    storeA(0, 0);
+    loadA(min(1, nk - 1));
+    storeA(1, 1);
+    loadA(min(2, nk - 1));
+    lds_barrier();
+    if constexpr (!PK)
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const float bnd = row_bound(st[0][j]);
+            up[j] = ldexpf(1.0f, bnd > 0.0f ? exponent_for(bnd) - 3 : 14);
+        }
+    words(st[0], 0);
+    if constexpr (!PK) loadB(st[0], min(1, nk - 1));
+#pragma unroll
+    for (int i = 0; i < FI; i++) readA(0, 0, i);
+#pragma unroll
+    for (int j = 0; j < 2; j++) b[j] = O::get(wd[j].w, wd[j].sc, 0, cst);
+    // K is a multiple of 128 (vh_mfma_supported): an even number of steps
+    for (int s = 0, b0 = 0; s < nk; s += 2) {
+        const int b1 = b0 == 2 ? 0 : b0 + 1, b2 = b1 == 2 ? 0 : b1 + 1;
+        step(s, b0, b1, b2, st[0], st[PK ? 1 : 0]);
+        step(s + 1, b1, b2, b0, st[PK ? 1 : 0], st[0]);
+        b0 = b2;
+    }
+
+    if constexpr (!PK) {
+        rs[0] = 1.0f / up[0];
+        rs[1] = 1.0f / up[1];
+    }
+    // epilogue: the lane holds column `col` of each fragment, rows 8 (r / 4) +
+    // 4 half + r % 4 of each 32-row block
+    const int r0 = base + m0;
+    auto row_of = [&](int r) { return 8 * (r >> 2) + (r & 3); };  // + 4 half
+#pragma unroll
+    for (int i = 0; i < FI; i++) {
+        float sc[16];
+#pragma unroll
+        for (int r = 0; r < 16; r++) sc[r] = L.rsc[32 * i + row_of(r) + 4 * half];
+        if constexpr (GATEUP) {
+            float h[16], m[16];
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const float g = acc[i][0][r] * (rs[0] * sc[r]), u = acc[i][1][r] * (rs[1] * sc[r]);
+                h[r] = g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) * u;  // kept to 11 bits below
+                m[r] = fabsf(h[r]);
+            }
+            // each row's largest |h| over the half wave's 32 columns: the rows are
+            // folded over the lanes, so that after the steps below lane l holds row
+            // r(l) = 8 b4 + 4 b3 + 2 b2 + b1 of the 16 (b: the bits of l)
+#pragma unroll
+            for (int r = 0; r < 8; r++) {
+                const auto v = __builtin_amdgcn_permlane16_swap(__float_as_uint(m[r]), __float_as_uint(m[r + 8]), false, false);
+                m[r] = fmaxf(__uint_as_float(v[0]), __uint_as_float(v[1]));
+            }
+            fold<0x128, 4>(m, (lane & 8) != 0);  // row_ror:8
+            fold<0x141, 2>(m, (lane & 4) != 0);  // row_half_mirror: the other four of eight lanes
+            fold<0x4E, 1>(m, (lane & 2) != 0);
+            m[0] = fmaxf(m[0], dpp_keep<0xB1>(m[0]));
+            // the block's exponent: |h| < 2^e, stored as h 2^(14 - e) in fp16
+            const uint32_t mb = __float_as_uint(m[0]);
+            const int e = mb ? max(-100, min(127, int(mb >> 23) - 126)) : -128;
+            const int rl = row_of((lane >> 1) & 15) + 4 * half;
+            if (!(lane & 1)) {
+                L.hsc[wv][rl] = __uint_as_float(uint32_t(127 + 14 - max(e, -100)) << 23);
+                if (32 * i + rl < mcnt) a.he[size_t(r0 + 32 * i + rl) * (a.rows / 32) + c] = int8_t(e);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            auto *hs = (__attribute__((address_space(1))) char *)a.out + (size_t(r0 + 32 * i) * a.rows + 32 * c) * 2;
+            const uint32_t ho = uint32_t(4 * half * a.rows + col) * 2u;
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const _Float16 v = _Float16(h[r] * L.hsc[wv][row_of(r) + 4 * half]);
+                if (32 * i + row_of(r) + 4 * half < mcnt)
+                    *(__attribute__((address_space(1))) _Float16 *)(hs + size_t(row_of(r)) * a.rows * 2 + ho) = v;
+            }
+            __builtin_amdgcn_wave_barrier();
+        } else {
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int tr = 32 * i + row_of(r) + 4 * half;
+                if (tr < mcnt) {
+                    float *y = static_cast<float *>(a.out) + size_t(L.prow[tr]) * a.rows + 64 * c + col;
+                    y[0] = acc[i][0][r] * (rs[0] * sc[r]);
+                    y[32] = acc[i][1][r] * (rs[1] * sc[r]);
+                }
+            }
+        }
+    }
 }
 
-// kXcds x slots workgroups of 512 threads (slots from tile_cost). The plan
+// kXcds x slots workgroups (slots from tile_cost). The plan
 // (mfma_plan_kernel) holds n tiles (expert, size, first row of its group)
 // and, per launch, where each XCD's run of (tile, column tile) pairs starts:
 // workgroup b runs on XCD b mod 8 (hardware dispatch) and takes pair
-// start[b mod 8] + b / 8 of that XCD's contiguous run, column tiles fastest,
-// so the workgroups sharing a token tile, and the consecutive token tiles of
-// one expert that share its weight tiles, meet in the same L2. The runs are
-// cut at equal shares of the staged bytes (tiles of fewer rows cost less).
-template <int T, bool GATEUP>
-__global__ void __launch_bounds__(kThreads) mfma_proj_kernel(const int32_t *__restrict__ tiles,
-                                                             const int32_t *__restrict__ counts,
-                                                             const int32_t *__restrict__ offs,
-                                                             const int32_t *__restrict__ perm,
-                                                             const void *const *__restrict__ table,
-                                                             const __bf16 *__restrict__ src, int K, int rows, int k,
-                                                             int64_t row_bytes, void *__restrict__ out) {
+// start[b mod 8] + b / 8 of that XCD's contiguous run, column tiles fastest.
+// BMAX: the plan's largest tile. What bounds it (Qwen3 Q4_K_M, 4093 tokens,
+// 128-row tiles): a K step takes 1.5 us of a CU's two workgroups where its
+// multiplies need 1.0 at the clock it runs at (2.0 GHz), and a workgroup spends
+// 6 us before its first step (a chain of four loads) and 8 (gate/up) or 6
+// (down) after its last; gate/up 514 -> 250 us, down 381 -> 180 us against the
+// kernel whose waves were split into staging and multiplying ones.
+template <int T, bool GATEUP, int BMAX, bool PK>
+__global__ void __launch_bounds__(kThreads, BMAX == kBigTile || !PK ? 2 : 3) mfma_gemm_kernel(GemmArgs a) {
     constexpr int NCOL = GATEUP ? kBRows / 2 : kBRows;  // output columns per workgroup
-    __shared__ bf16x8 As[2][kChunks][kBM];
-    __shared__ bf16x8 Bs[2][kChunks][kBRows];
-    __shared__ int prow[kBM];
-    const int nct = rows / NCOL, xcd = blockIdx.x % kXcds, slot = blockIdx.x / kXcds;
-    const int32_t *run = tiles + (GATEUP ? kPlanRunsGU : kPlanRunsDN);
-    const int L = run[xcd] + slot;
-    if (L >= run[xcd + 1]) return;
-    const int t = L / nct, n0 = (L % nct) * NCOL;
-    const int code = tiles[kPlanHead + 2 * t], m0 = tiles[kPlanHead + 2 * t + 1];
-    const int e = code & 0xffff, bmt = code >> 16;
-    const int base = offs[e], mcnt = min(bmt, counts[e] - m0);
-    const int tid = threadIdx.x;
-
-    gbyte *M0 = gmem(table[3 * e + (GATEUP ? 0 : 2)]);
-    gbyte *M1 = GATEUP ? gmem(table[3 * e + 1]) : M0;
+    __shared__ TileLds<GATEUP, BMAX> lds;
+    const int nct = a.rows / NCOL, xcd = blockIdx.x % kXcds, slot = blockIdx.x / kXcds;
+    const int32_t *run = a.tiles + (GATEUP ? kPlanRunsGU : kPlanRunsDN);
+    const int at = run[xcd] + slot;
+    if (at >= run[xcd + 1]) return;
+    const int t = at / nct, n0 = (at % nct) * NCOL;
+    const int32_t *rec = a.tiles + kPlanHead + 4 * t;
+    const int e = rec[0] & 0xffff, bmt = rec[0] >> 16, m0 = rec[1], base = rec[2], mcnt = rec[3];
+    gbyte *M0 = gmem(a.table[3 * e + (GATEUP ? 0 : 2)]);
+    gbyte *M1 = GATEUP ? gmem(a.table[3 * e + 1]) : M0;
     if (!M0 || !M1) {
         // an unregistered expert contributes nothing (src/gguf_run.c:201): its
         // h rows are zero, and the combine skips its y rows
         if (GATEUP)
-            for (int i = tid; i < mcnt * NCOL; i += kThreads)
-                static_cast<__bf16 *>(out)[size_t(base + m0 + i / NCOL) * rows + n0 + i % NCOL] = __bf16(0.0f);
-        return;
-    }
-    if (bmt == 32)
-        mfma_tile<T, GATEUP, 32>(As, Bs, prow, M0, M1, perm, src, K, rows, k, row_bytes, out, base, m0, mcnt, n0);
-    else if (bmt == 64)
-        mfma_tile<T, GATEUP, 64>(As, Bs, prow, M0, M1, perm, src, K, rows, k, row_bytes, out, base, m0, mcnt, n0);
-    else
-        mfma_tile<T, GATEUP, 128>(As, Bs, prow, M0, M1, perm, src, K, rows, k, row_bytes, out, base, m0, mcnt, n0);
-}
-
-// ---- Q8_0 experts packed in the matrix cores' operand order (kQ8Frag) ----
-//
-// A pinned Q8_0 layer's experts are copied once (vh_mfma_pack_q8) into
-// fragments: fragment (g, s) of a matrix is the 32 weight rows one
-// v_mfma_f32_32x32x16_bf16 B operand takes (gate/up: rows 16 g .. 16 g + 15 of
-// gate, then the same rows of up; down: rows 32 g .. 32 g + 31) over K step s
-// (64 columns), kFragBytes bytes: first, lane l's 32 quant bytes - row l % 32,
-// columns 64 s + 16 ks + 8 (l / 32) .. + 7 for ks = 0..3, the 8 bytes it
-// supplies to sub-step ks - then the rows' two block scales (2 x fp16 per row,
-// blocks 2 s and 2 s + 1). A wave reads its B operand for a K step with two
-// 1 KB and one 128 B load instructions of consecutive bytes and dequantizes
-// it in its own registers; only the activations pass through LDS.
-constexpr int kFragBytes = 2176;
-
-// One token tile of BM rows against 8 fragments (gate/up: 128 output columns;
-// down: 256), 512 threads: wave w multiplies all BM rows by fragment w, FI =
-// BM / 32 accumulators. Per K step every thread dequantizes its wave's B
-// operand loaded two steps earlier (the values of Chunk<VT_Q8_0>, rounded to
-// bf16 the same way, in the same K order: the results equal mfma_tile's bit for
-// bit), issues the loads of two steps ahead, multiplies, and stores the
-// inputs of the next step into the other LDS buffer. The barrier is LDS-only:
-// global loads stay in flight across it.
-template <bool GATEUP, int BM>
-VH_DEV void frag_tile(bf16x8 (&As)[2][kChunks][kBM], int (&prow)[kBM], gbyte *F, const int32_t *__restrict__ perm,
-                      const __bf16 *__restrict__ src, int K, int rows, int k, void *__restrict__ out, int base, int m0,
-                      int mcnt, int n0) {
-    constexpr int FI = BM / 32, AQ = (BM * kChunks + kThreads - 1) / kThreads;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nk = K / kBK;
-    // down: the y row of each tile row in LDS for the epilogue (as mfma_tile;
-    // the first barrier below publishes it)
-    if (!GATEUP && tid < BM) prow[tid] = perm[base + m0 + min(tid, mcnt - 1)];
-    // this wave's fragments: g = n0 / 16 + wv (gate/up) or n0 / 32 + wv (down)
-    gbyte *fb = F + size_t((GATEUP ? n0 / 16 : n0 / 32) + wv) * nk * kFragBytes;
-    gbyte *fq = fb + 32 * lane, *fs = fb + 2048 + 4 * (lane & 31);
-    // input staging: chunk slot c = tid + 512 q holds K chunk c & 7 of tile row
-    // c >> 3 (rows past the group repeat its last row; slots past the tile
-    // fill LDS rows that are not read). Every load is unconditional (steps
-    // past the end repeat the last one), so the waits before each use count
-    // exactly the loads issued after it.
-    gbyte *abase = gmem(src);
-    uint32_t aoff[AQ];
-    int arow[AQ];
-#pragma unroll
-    for (int q = 0; q < AQ; q++) {
-        const int c = tid + kThreads * q, r = c >> 3, kc = c & 7;
-        const int i = base + m0 + min(r, mcnt - 1);
-        aoff[q] = uint32_t((GATEUP ? size_t(perm[i] / k) : size_t(i)) * K * 2) + 16u * uint32_t(kc);
-        arow[q] = r ^ kc;
-    }
-    uint4 av[2][AQ], bq[2][2];
-    uint32_t bs[2];
-    auto loadA = [&](int set, int step) {
-#pragma unroll
-        for (int q = 0; q < AQ; q++) av[set][q] = ld_u128(abase + 128 * step + aoff[q]);
-    };
-    auto storeA = [&](int set, int buf) {
-#pragma unroll
-        for (int q = 0; q < AQ; q++)
-            As[buf][(tid + kThreads * q) & 7][arow[q]] = __builtin_bit_cast(bf16x8, av[set][q]);
-    };
-    auto loadB = [&](int set, int step) {
-        bq[set][0] = ld_u128(fq + size_t(step) * kFragBytes);
-        bq[set][1] = ld_u128(fq + size_t(step) * kFragBytes + 16);
-        bs[set] = ld_u32(fs + size_t(step) * kFragBytes);
-    };
-    f32x16 acc[FI];
-#pragma unroll
-    for (int i = 0; i < FI; i++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) acc[i][r] = 0.0f;
-
-    // K step s: B(s) in register set s % 2, A(s + 1) in set (s + 1) % 2, LDS
-    // buffer s % 2 holds A(s)
-    auto step = [&](int s, auto SET) {
-        constexpr int set = decltype(SET)::value, nset = 1 - set;
-        // B(s): (q + 128) * d - 128 * d = q * d exactly, then bf16
-        bf16x8 b[4];
-        const uint32_t w[8] = {bq[set][0].x, bq[set][0].y, bq[set][0].z, bq[set][0].w,
-                               bq[set][1].x, bq[set][1].y, bq[set][1].z, bq[set][1].w};
-#pragma unroll
-        for (int ks = 0; ks < 4; ks++) {
-            const float sc = h2f(ks < 2 ? bs[set] & 0xffffu : bs[set] >> 16), off = -128.0f * sc;
-            uint32_t u0 = w[2 * ks] ^ 0x80808080u, u1 = w[2 * ks + 1] ^ 0x80808080u;
-            asm volatile("" : "+v"(u0), "+v"(u1));
-            const uint32_t uu[2] = {u0, u1};
-            float v[8];
-#pragma unroll
-            for (int i = 0; i < 8; i++) v[i] = fmaf(float((uu[i >> 2] >> (8 * (i & 3))) & 0xffu), sc, off);
-            b[ks] = to_bf16(v);
-        }
-        loadB(set, min(s + 2, nk - 1));
-#pragma unroll
-        for (int ks = 0; ks < 4; ks++) {
-            const int kg = 2 * ks + (lane >> 5), lx = (lane & 31) ^ kg;
-#pragma unroll
-            for (int i = 0; i < FI; i++)
-                acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(As[set][kg][lx + 32 * i], b[ks], acc[i], 0, 0, 0);
-        }
-        storeA(nset, nset);
-        loadA(nset, min(s + 3, nk - 1));
-        lds_barrier();
-    };
-    loadA(0, 0);
-    loadB(0, 0);
-    loadA(1, min(1, nk - 1));
-    loadB(1, min(1, nk - 1));
-    storeA(0, 0);
-    loadA(0, min(2, nk - 1));
-    lds_barrier();
-    int s = 0;
-    for (; s + 1 < nk; s += 2) {
-        step(s, std::integral_constant<int, 0>());
-        step(s + 1, std::integral_constant<int, 1>());
-    }
-    if (s < nk) step(s, std::integral_constant<int, 0>());
-
-    // epilogue: lane l holds column l % 32 of the fragment (gate/up: gate
-    // column l % 16 in lanes l % 32 < 16, up in the others)
-#pragma unroll
-    for (int i = 0; i < FI; i++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int row = 32 * i + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-            if (GATEUP) {
-                const float g = acc[i][r], u = __shfl_xor(g, 16, 64);
-                if (row < mcnt && !(lane & 16))
-                    static_cast<__bf16 *>(out)[size_t(base + m0 + row) * rows + n0 + 16 * wv + (lane & 15)] =
-                        __bf16(swiglu(g, u));
-            } else if (row < mcnt) {
-                static_cast<float *>(out)[size_t(prow[row]) * rows + n0 + 32 * wv + (lane & 31)] = acc[i][r];
+            for (int i = threadIdx.x; i < mcnt * NCOL; i += kThreads) {
+                const size_t pos = size_t(base + m0 + i / NCOL);
+                const int cc = n0 + i % NCOL;
+                static_cast<_Float16 *>(a.out)[pos * a.rows + cc] = _Float16(0.0f);
+                if (cc % 32 == 0) a.he[pos * (a.rows / 32) + cc / 32] = int8_t(-128);
             }
-        }
-}
-
-// mfma_proj_kernel's grid, plan and outputs on kQ8Frag experts: table[3 e] =
-// the expert's gate/up fragments, table[3 e + 2] its down fragments. Held to
-// 128 registers (four waves per SIMD): two workgroups share a CU, one
-// multiplying while the other waits at its barrier.
-template <bool GATEUP>
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) mfma_frag_kernel(const int32_t *__restrict__ tiles,
-                                                             const int32_t *__restrict__ counts,
-                                                             const int32_t *__restrict__ offs,
-                                                             const int32_t *__restrict__ perm,
-                                                             const void *const *__restrict__ table,
-                                                             const __bf16 *__restrict__ src, int K, int rows, int k,
-                                                             void *__restrict__ out) {
-    constexpr int NCOL = GATEUP ? kBRows / 2 : kBRows;
-    __shared__ bf16x8 As[2][kChunks][kBM];
-    __shared__ int prow[kBM];
-    const int nct = rows / NCOL, xcd = blockIdx.x % kXcds, slot = blockIdx.x / kXcds;
-    const int32_t *run = tiles + (GATEUP ? kPlanRunsGU : kPlanRunsDN);
-    const int L = run[xcd] + slot;
-    if (L >= run[xcd + 1]) return;
-    const int t = L / nct, n0 = (L % nct) * NCOL;
-    const int code = tiles[kPlanHead + 2 * t], m0 = tiles[kPlanHead + 2 * t + 1];
-    const int e = code & 0xffff, bmt = code >> 16;
-    const int base = offs[e], mcnt = min(bmt, counts[e] - m0);
-    gbyte *F = gmem(table[3 * e + (GATEUP ? 0 : 2)]);
-    if (!F) {
-        // an unregistered expert contributes nothing (src/gguf_run.c:201)
-        if (GATEUP)
-            for (int i = threadIdx.x; i < mcnt * NCOL; i += kThreads)
-                static_cast<__bf16 *>(out)[size_t(base + m0 + i / NCOL) * rows + n0 + i % NCOL] = __bf16(0.0f);
         return;
     }
-    if (bmt == 32)
-        frag_tile<GATEUP, 32>(As, prow, F, perm, src, K, rows, k, out, base, m0, mcnt, n0);
-    else if (bmt == 64)
-        frag_tile<GATEUP, 64>(As, prow, F, perm, src, K, rows, k, out, base, m0, mcnt, n0);
-    else
-        frag_tile<GATEUP, 128>(As, prow, F, perm, src, K, rows, k, out, base, m0, mcnt, n0);
+    if (bmt == 32) gemm_tile<T, GATEUP, 32, BMAX, PK>(lds, a, M0, M1, base, m0, mcnt, n0);
+    else if (bmt == 64) gemm_tile<T, GATEUP, 64, BMAX, PK>(lds, a, M0, M1, base, m0, mcnt, n0);
+    else if constexpr (BMAX == 128) gemm_tile<T, GATEUP, 128, BMAX, PK>(lds, a, M0, M1, base, m0, mcnt, n0);
 }
 
-// bf16 copy of n4 x 4 fp32 values (both 16-byte aligned) by workgroup blk of nblk
-VH_DEV void bf16_copy(const float4 *__restrict__ x, uint2 *__restrict__ y, int64_t n4, int blk, int nblk) {
-    for (int64_t i = blk * int64_t(256) + threadIdx.x; i < n4; i += int64_t(nblk) * 256) {
+// The fp16 copy of hb [T x d] under each token's power of two (its largest
+// magnitude brought below 2^14; 1 where that is not finite), a wave per
+// token, and the inverse scales xsc [T]; workgroup blk of 256 threads.
+VH_DEV void f16_rows(const float *__restrict__ hb, _Float16 *__restrict__ xb, float *__restrict__ xsc, int T, int d,
+                     int blk) {
+    const int t = blk * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (t >= T) return;
+    const float4 *x = reinterpret_cast<const float4 *>(hb + size_t(t) * d);
+    f16x4 *y = reinterpret_cast<f16x4 *>(xb + size_t(t) * d);
+    float m = 0.0f;
+    for (int i = lane; i < d / 4; i += 64) {
         const float4 v = x[i];
-        typedef float f32x4_ __attribute__((ext_vector_type(4)));
-        typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-        const bf16x4 b = __builtin_convertvector(f32x4_{v.x, v.y, v.z, v.w}, bf16x4);
-        y[i] = __builtin_bit_cast(uint2, b);
+        m = fmaxf(m, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
     }
-}
-
-__global__ void __launch_bounds__(256) to_bf16_kernel(const float4 *__restrict__ x, uint2 *__restrict__ y, int64_t n4) {
-    bf16_copy(x, y, n4, blockIdx.x, gridDim.x);
+    const int e = exponent_for(wave_max_f(m));
+    const float up = ldexpf(1.0f, e);
+    if (lane == 0) xsc[t] = ldexpf(1.0f, -e);
+    for (int i = lane; i < d / 4; i += 64) {
+        const float4 v = x[i];
+        y[i] = f16x4{_Float16(v.x * up), _Float16(v.y * up), _Float16(v.z * up), _Float16(v.w * up)};
+    }
 }
 
 // The bytes a token tile of bm rows stages per K step (the weights' wb and
 // the inputs), in 64-byte units: the cost by which the XCDs' runs are cut.
 __host__ __device__ constexpr int tile_step_cost(int wb, int bm) { return (wb + bm * kBK * 2) / 64; }
 
-// A group's token tiles: n128 of 128 rows, then one of rbm (32 or 64) rows if
-// rbm != 0 - the remainder in the smallest tile that holds it (above 64 rows,
-// a whole tile).
+// A group's token tiles under the largest tile of bm rows (128 or 64): n whole
+// ones, then one of rbm (32 or 64) rows if rbm != 0 - the remainder in the
+// smallest tile that holds it (above bm / 2 rows, a whole tile).
 struct GroupTiles {
-    int n128, rbm;
-    __host__ __device__ explicit GroupTiles(int cnt) {
-        n128 = cnt / 128;
-        int r = cnt - 128 * n128;
-        if (r > 64) {
-            n128++;
+    int bm, n, rbm;
+    __host__ __device__ GroupTiles(int cnt, int bmax) : bm(bmax), n(cnt / bmax) {
+        int r = cnt - bm * n;
+        if (2 * r > bm) {
+            n++;
             r = 0;
         }
         rbm = r == 0 ? 0 : r <= 32 ? 32 : 64;
     }
-    __host__ __device__ int count() const { return n128 + (rbm ? 1 : 0); }
-    __host__ __device__ int rows(int i) const { return i < n128 ? 128 : rbm; }
+    __host__ __device__ int count() const { return n + (rbm ? 1 : 0); }
+    __host__ __device__ int rows(int i) const { return i < n ? bm : rbm; }
 };
 
-// One workgroup of 256 threads (thread e = expert e, E <= 256). The plan:
+// Workgroup 0 of 256 threads (thread e = expert e, E <= 256): the plan,
 //   tiles[0]               n, the number of token tiles
 //   tiles[kPlanRunsGU + x]  x = 0..8: where XCD x's run of gate/up (tile,
 //                           column tile) pairs starts (x = 8: the end)
 //   tiles[kPlanRunsDN + x]  the same for the down launch
-//   tiles[kPlanHead + 2 t]  tile t: expert | rows << 16 (32, 64 or 128), then
-//                           the tile's first row within its group
-// for the groups of at least min_tokens tokens (experts ascending, tiles as
-// GroupTiles), and the list of the other non-empty groups in the dispatch
-// kernel's `active` format (small[0 .. n), n at small[E]). The runs are cut
-// at equal shares of the launch's staged bytes (tile_step_cost per pair); a
-// cut that would give an XCD more pairs than the launch has slots per XCD
-// falls back to equal shares of pairs.
-__global__ void __launch_bounds__(256) mfma_plan_kernel(const int32_t *__restrict__ counts, int E, int min_tokens,
+//   tiles[kPlanHead + 4 t]  tile t: expert | rows << 16 (32, 64 or 128), the
+//                           tile's first row within its group, the group's
+//                           first pair (offs), the tile's pairs
+// (experts ascending, tiles as GroupTiles). The runs are cut at equal shares
+// of the launch's staged bytes (tile_step_cost per pair); a cut that would
+// give an XCD more pairs than the launch has slots per XCD falls back to equal
+// shares of pairs. The other workgroups: the GEMMs' inputs (f16_rows).
+__global__ void __launch_bounds__(256) mfma_plan_kernel(const int32_t *__restrict__ counts,
+                                                        const int32_t *__restrict__ offs, int E, int bmax,
                                                         int nct_gu, int wb_gu, int slots_gu, int nct_dn,
                                                         int wb_dn, int slots_dn, int32_t *__restrict__ tiles,
-                                                        int32_t *__restrict__ small, const float4 *__restrict__ x,
-                                                        uint2 *__restrict__ y, int64_t n4) {
-    if (blockIdx.x > 0) {  // the other workgroups: the bf16 copy of the inputs (to_bf16_kernel)
-        bf16_copy(x, y, n4, blockIdx.x - 1, gridDim.x - 1);
+                                                        const float *__restrict__ hb, _Float16 *__restrict__ xb,
+                                                        float *__restrict__ xsc, int T, int d) {
+    if (blockIdx.x > 0) {
+        f16_rows(hb, xb, xsc, T, d, blockIdx.x - 1);
         return;
     }
-    __shared__ int wsum[4][2];
+    __shared__ int wsum[4];
     __shared__ int wcost[4][2];
     __shared__ int runs[2][kXcds + 1];
     __shared__ int total[2];
     __shared__ int ntiles;
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
     const int cnt = t < E ? counts[t] : 0;
-    const bool on = cnt > 0 && cnt >= min_tokens;
-    const GroupTiles gt(on ? cnt : 0);
-    const int nt = gt.count(), sm = (!on && cnt > 0) ? 1 : 0;
+    const GroupTiles gt(cnt, bmax);
+    const int nt = gt.count();
     const int ncts[2] = {nct_gu, nct_dn};
     const int wbs[2] = {wb_gu, wb_dn};
     int c[2];
 #pragma unroll
     for (int l = 0; l < 2; l++)
-        c[l] = ncts[l] * (gt.n128 * tile_step_cost(wbs[l], kBM) + (gt.rbm ? tile_step_cost(wbs[l], gt.rbm) : 0));
-    int it = nt, is = sm;
+        c[l] = ncts[l] * (gt.n * tile_step_cost(wbs[l], bmax) + (gt.rbm ? tile_step_cost(wbs[l], gt.rbm) : 0));
+    int it = nt;
     int ic[2] = {c[0], c[1]};
 #pragma unroll
     for (int sh = 1; sh < 64; sh <<= 1) {
-        const int ot = __shfl_up(it, sh, 64), os = __shfl_up(is, sh, 64);
+        const int ot = __shfl_up(it, sh, 64);
         const int o0 = __shfl_up(ic[0], sh, 64), o1 = __shfl_up(ic[1], sh, 64);
         if (lane >= sh) {
             it += ot;
-            is += os;
             ic[0] += o0;
             ic[1] += o1;
         }
     }
     if (lane == 63) {
-        wsum[wv][0] = it;
-        wsum[wv][1] = is;
+        wsum[wv] = it;
         wcost[wv][0] = ic[0];
         wcost[wv][1] = ic[1];
     }
     __syncthreads();
-    int bt = 0, bs = 0;
+    int bt = 0;
     int bc[2] = {0, 0};
     for (int w = 0; w < wv; w++) {
-        bt += wsum[w][0];
-        bs += wsum[w][1];
+        bt += wsum[w];
         bc[0] += wcost[w][0];
         bc[1] += wcost[w][1];
     }
-    const int ex_t = bt + it - nt, ex_s = bs + is - sm;
+    const int ex_t = bt + it - nt;
     for (int i = 0; i < nt; i++) {
-        tiles[kPlanHead + 2 * (ex_t + i)] = t | (gt.rows(i) << 16);
-        tiles[kPlanHead + 2 * (ex_t + i) + 1] = kBM * i;
+        int32_t *rec = tiles + kPlanHead + 4 * (ex_t + i);
+        rec[0] = t | (gt.rows(i) << 16);
+        rec[1] = bmax * i;
+        rec[2] = offs[t];
+        rec[3] = min(gt.rows(i), cnt - bmax * i);
     }
-    if (sm) small[ex_s] = t;
     if (t == 255) {
         ntiles = ex_t + nt;
         total[0] = bc[0] + ic[0];
         total[1] = bc[1] + ic[1];
         tiles[0] = ex_t + nt;
-        small[E] = ex_s + sm;
     }
     __syncthreads();
     // the cuts: XCD x's run starts at the pair holding staged byte x * total / 8
@@ -709,10 +835,10 @@ __global__ void __launch_bounds__(256) mfma_plan_kernel(const int32_t *__restric
         for (int x = 1; x < kXcds; x++) {
             const int target = int(int64_t(x) * total[l] / kXcds);
             if (c[l] > 0 && ex_c <= target && target < ex_c + c[l]) {
-                // the tile holding the target (a whole 128-row tile or the last), then its column
-                const int off = target - ex_c, c128 = tile_step_cost(wbs[l], kBM), full = gt.n128 * ncts[l] * c128;
-                const int i = off < full ? off / (ncts[l] * c128) : gt.n128;
-                const int rest = off - i * ncts[l] * c128;
+                // the tile holding the target (a whole tile or the last), then its column
+                const int off = target - ex_c, cw = tile_step_cost(wbs[l], bmax), full = gt.n * ncts[l] * cw;
+                const int i = off < full ? off / (ncts[l] * cw) : gt.n;
+                const int rest = off - i * ncts[l] * cw;
                 runs[l][x] = (ex_t + i) * ncts[l] + min(rest / tile_step_cost(wbs[l], gt.rows(i)), ncts[l] - 1);
             }
         }
@@ -736,45 +862,48 @@ __global__ void __launch_bounds__(256) mfma_plan_kernel(const int32_t *__restric
     }
 }
 
+// The largest token tile of a call of P pairs over E experts: 128 rows where
+// the average group has at least kBigAverage, else 64, whose kernel keeps three
+// waves per SIMD instead of two to hide the weights' loads, which bound small
+// groups. Measured per layer with tiles of up to 64 / 128 rows: OLMoE Q4_K_M 512
+// tokens (64 per expert) 205 / 236 us, Qwen3 Q8_0 2048 tokens (128 per expert,
+// Zipf) 424 / 421 us, Qwen3 Q4_K_M 4093 tokens (256 per expert) 705 / 667 us.
+constexpr int kBigAverage = 100;
+int tile_rows(int P, int E) { return P >= kBigAverage * E ? kBigTile : kSmallTile; }
+
 // The column tiles, weight bytes per K step and workgroup slots per XCD of a
-// launch: enough slots for any cut mfma_plan_kernel makes (an XCD's share of
-// the staged bytes plus one pair, at the cheapest pair's cost).
+// launch: an eighth more than an XCD's share of the most pairs there can be
+// (mfma_plan_kernel cuts into equal shares of pairs where an XCD would get
+// more; a workgroup past its XCD's run costs a round trip).
 struct TileCost {
     int nct, wb, slots;
 };
-TileCost tile_cost(uint32_t type, int K, int rows, bool gateup, int max_tiles) {
+TileCost tile_cost(uint32_t type, int K, int rows, bool gateup, int P, int E) {
     TileCost c;
     c.nct = rows / (gateup ? kBRows / 2 : kBRows);
     c.wb = int(int64_t(kBRows) * vh_row_bytes(type, K) * kBK / K);  // a multiple of 64 for these types
-    const int64_t cmax = tile_step_cost(c.wb, kBM), cmin = tile_step_cost(c.wb, 32);
-    c.slots = int((int64_t(max_tiles) * c.nct * cmax / kXcds + cmax) / cmin + 1);
+    const int64_t per = (int64_t(vh_mfma_max_tiles(P, E)) * c.nct + kXcds - 1) / kXcds;
+    c.slots = int(per + per / 8 + 1);
     return c;
 }
 
+template <int T, bool GATEUP>
+void launch_gemm(const GemmArgs &a, const dim3 &g, bool big, bool packed, hipStream_t s) {
+    const dim3 b(kThreads);
+    if (big && packed) hipLaunchKernelGGL((mfma_gemm_kernel<T, GATEUP, kBigTile, true>), g, b, 0, s, a);
+    else if (big) hipLaunchKernelGGL((mfma_gemm_kernel<T, GATEUP, kBigTile, false>), g, b, 0, s, a);
+    else if (packed) hipLaunchKernelGGL((mfma_gemm_kernel<T, GATEUP, kSmallTile, true>), g, b, 0, s, a);
+    else hipLaunchKernelGGL((mfma_gemm_kernel<T, GATEUP, kSmallTile, false>), g, b, 0, s, a);
+}
+
 template <bool GATEUP>
-int mfma_launch(uint32_t type, const int32_t *tiles, int max_tiles, const int32_t *counts, const int32_t *offs,
-                const int32_t *perm, const void *const *table, bool packed, const __bf16 *src, int K, int rows, int k,
-                void *out, hipStream_t s) {
-    if (packed && type != VT_Q8_0) return -EINVAL;
-    const TileCost tc = tile_cost(type, K, rows, GATEUP, max_tiles);
-    const dim3 g(unsigned(tc.slots) * kXcds);
+int gemm(uint32_t type, int P, int E, bool packed, const GemmArgs &a, hipStream_t s) {
+    const dim3 g(unsigned(tile_cost(type, a.K, a.rows, GATEUP, P, E).slots) * kXcds);
+    const bool big = tile_rows(P, E) == kBigTile;
     switch (type) {
-    case VT_Q8_0:
-        if (packed)
-            hipLaunchKernelGGL((mfma_frag_kernel<GATEUP>), g, dim3(kThreads), 0, s, tiles, counts, offs, perm, table,
-                               src, K, rows, k, out);
-        else
-            hipLaunchKernelGGL((mfma_proj_kernel<VT_Q8_0, GATEUP>), g, dim3(kThreads), 0, s, tiles, counts, offs,
-                               perm, table, src, K, rows, k, vh_row_bytes(type, K), out);
-        break;
-    case VT_Q4_K:
-        hipLaunchKernelGGL((mfma_proj_kernel<VT_Q4_K, GATEUP>), g, dim3(kThreads), 0, s, tiles, counts, offs, perm,
-                           table, src, K, rows, k, vh_row_bytes(type, K), out);
-        break;
-    case VT_Q6_K:
-        hipLaunchKernelGGL((mfma_proj_kernel<VT_Q6_K, GATEUP>), g, dim3(kThreads), 0, s, tiles, counts, offs, perm,
-                           table, src, K, rows, k, vh_row_bytes(type, K), out);
-        break;
+    case VT_Q8_0: launch_gemm<VT_Q8_0, GATEUP>(a, g, big, packed, s); break;
+    case VT_Q4_K: launch_gemm<VT_Q4_K, GATEUP>(a, g, big, packed, s); break;
+    case VT_Q6_K: launch_gemm<VT_Q6_K, GATEUP>(a, g, big, packed, s); break;
     default: return -EINVAL;
     }
     return vh_check(hipGetLastError());
@@ -789,93 +918,122 @@ bool vh_mfma_supported(uint32_t tg, uint32_t td, int d, int fe, int E) {
            d % kBK == 0 && fe % kBK == 0 && E <= 256;
 }
 
-int vh_mfma_max_tiles(int P, int E) { return P / kBM + E; }
+int vh_mfma_max_tiles(int P, int E) { return P / tile_rows(P, E) + E; }
 
-int vh_mfma_plan_words(int P, int E) { return kPlanHead + 2 * vh_mfma_max_tiles(P, E); }
+int vh_mfma_plan_words(int P, int E) { return kPlanHead + 4 * vh_mfma_max_tiles(P, E); }
 
-int vh_mfma_plan(const int32_t *counts, int E, int P, int min_tokens, uint32_t tg, uint32_t td, int d, int fe,
-                 int32_t *tiles, int32_t *small, const float *hb, void *xb, int64_t n, hipStream_t s) {
-    if (E > 256 || (hb && (n % 4 || ((reinterpret_cast<uintptr_t>(hb) | reinterpret_cast<uintptr_t>(xb)) & 15u))))
-        return -EINVAL;
-    const int64_t n4 = hb ? n / 4 : 0;
-    const unsigned copy_blocks = unsigned(std::min<int64_t>((n4 + 255) / 256, 4096));
-    const int mt = vh_mfma_max_tiles(P, E);
-    const TileCost gu = tile_cost(tg, d, fe, true, mt), dn = tile_cost(td, fe, d, false, mt);
+int vh_mfma_plan(const int32_t *counts, const int32_t *offs, int E, int T, int k, uint32_t tg, uint32_t td, int d, int fe, int32_t *tiles,
+                 const float *hb, void *xb, float *xsc, hipStream_t s) {
+    if (E > 256 || d % 4 || ((reinterpret_cast<uintptr_t>(hb) | reinterpret_cast<uintptr_t>(xb)) & 15u)) return -EINVAL;
+    const int P = T * k, mt = vh_mfma_max_tiles(P, E);
+    const TileCost gu = tile_cost(tg, d, fe, true, P, E), dn = tile_cost(td, fe, d, false, P, E);
     // the plan's costs are 32-bit sums over every (tile, column tile) pair
-    if (int64_t(mt) * std::max(gu.nct, dn.nct) * tile_step_cost(std::max(gu.wb, dn.wb), kBM) > INT32_MAX)
+    if (int64_t(mt) * std::max(gu.nct, dn.nct) * tile_step_cost(std::max(gu.wb, dn.wb), kBigTile) > INT32_MAX)
         return -E2BIG;
-    hipLaunchKernelGGL(mfma_plan_kernel, dim3(1 + copy_blocks), dim3(256), 0, s, counts, E, min_tokens, gu.nct,
-                       gu.wb, gu.slots, dn.nct, dn.wb, dn.slots, tiles, small,
-                       reinterpret_cast<const float4 *>(hb), static_cast<uint2 *>(xb), n4);
+    hipLaunchKernelGGL(mfma_plan_kernel, dim3(1 + unsigned((T + 3) / 4)), dim3(256), 0, s, counts, offs, E, tile_rows(P, E),
+                       gu.nct, gu.wb, gu.slots, dn.nct, dn.wb, dn.slots, tiles, hb, static_cast<_Float16 *>(xb), xsc,
+                       T, d);
     return vh_check(hipGetLastError());
 }
 
-int vh_to_bf16(const float *x, void *y, int64_t n, hipStream_t s) {
-    if (n % 4 || (reinterpret_cast<uintptr_t>(x) & 15u) || (reinterpret_cast<uintptr_t>(y) & 15u)) return -EINVAL;
-    const int64_t n4 = n / 4;
-    const unsigned blocks = unsigned(std::min<int64_t>((n4 + 255) / 256, 4096));
-    hipLaunchKernelGGL(to_bf16_kernel, dim3(blocks), dim3(256), 0, s, reinterpret_cast<const float4 *>(x),
-                       static_cast<uint2 *>(y), n4);
-    return vh_check(hipGetLastError());
+int vh_mfma_gateup(uint32_t type, const int32_t *tiles, int P, int E, const int32_t *perm,
+                   const void *const *table, bool packed, const void *xb, const float *xsc, int d,
+                   int fe, int k, void *hs, int8_t *he, hipStream_t s) {
+    return gemm<true>(type, P, E, packed,
+                      GemmArgs{tiles, perm, table, static_cast<const uint8_t *>(xb), xsc, he, hs, d, fe,
+                               k, vh_row_bytes(type, d)},
+                      s);
 }
 
-int vh_mfma_gateup(uint32_t type, const int32_t *tiles, int max_tiles, const int32_t *counts, const int32_t *offs,
-                   const int32_t *perm, const void *const *table, bool packed, const void *xb, int d, int fe, int k,
-                   void *hs, hipStream_t s) {
-    return mfma_launch<true>(type, tiles, max_tiles, counts, offs, perm, table, packed,
-                             static_cast<const __bf16 *>(xb), d, fe, k, hs, s);
-}
-
-int vh_mfma_down(uint32_t type, const int32_t *tiles, int max_tiles, const int32_t *counts, const int32_t *offs,
-                 const int32_t *perm, const void *const *table, bool packed, const void *hs, int d, int fe,
-                 float *ybuf, hipStream_t s) {
-    return mfma_launch<false>(type, tiles, max_tiles, counts, offs, perm, table, packed,
-                              static_cast<const __bf16 *>(hs), fe, d, 1, ybuf, s);
+int vh_mfma_down(uint32_t type, const int32_t *tiles, int P, int E, const int32_t *perm,
+                 const void *const *table, bool packed, const void *hs, const int8_t *he, int d,
+                 int fe, float *ybuf, hipStream_t s) {
+    return gemm<false>(type, P, E, packed,
+                       GemmArgs{tiles, perm, table, static_cast<const uint8_t *>(hs), nullptr,
+                                const_cast<int8_t *>(he), ybuf, fe, d, 1, vh_row_bytes(type, fe)},
+                       s);
 }
 
 namespace {
-// One workgroup per (fragment, expert), 544 threads: thread w writes word w
-// of the fragment's kFragBytes (kQ8Frag layout, above) from the expert's
-// GGUF rows. gateup: fragments of gate and up (rows 16 g + r % 16 of gate for
-// r < 16, of up above), else of down (rows 32 g + r); nk K steps per row.
-__global__ void __launch_bounds__(576) q8_frag_pack_kernel(const void *const *__restrict__ src_tab,
-                                                           void *const *__restrict__ dst_tab, int gateup, int nk,
-                                                           int64_t row_bytes) {
-    const int e = blockIdx.y, f = blockIdx.x, g = f / nk, st = f - g * nk, w = threadIdx.x;
-    uint8_t *dst = static_cast<uint8_t *>(dst_tab[3 * e + (gateup ? 0 : 2)]);
-    if (!dst || w >= kFragBytes / 4) return;
-    const int r = w < 512 ? (w >> 3) & 31 : w - 512;  // the fragment row this word belongs to
-    const uint8_t *row = gateup ? static_cast<const uint8_t *>(src_tab[3 * e + (r < 16 ? 0 : 1)]) +
-                                      int64_t(16 * g + (r & 15)) * row_bytes
-                                : static_cast<const uint8_t *>(src_tab[3 * e + 2]) + int64_t(32 * g + r) * row_bytes;
-    uint32_t v;
-    if (w < 512) {
-        // lane w / 8, bytes 4 (w % 8) .. + 3 of its 32: sub-step (w % 8) / 2, half w % 2
-        const int lane = w >> 3, ks = (w & 7) >> 1, K0 = 64 * st + 16 * ks + 8 * (lane >> 5) + 4 * (w & 1);
-        const uint8_t *q = row + 34 * (K0 >> 5) + 2 + (K0 & 31);  // even: two 16-bit loads
-        v = uint32_t(*reinterpret_cast<const uint16_t *>(q)) | uint32_t(*reinterpret_cast<const uint16_t *>(q + 2)) << 16;
-    } else {
-        v = uint32_t(*reinterpret_cast<const uint16_t *>(row + 68 * st)) |
-            uint32_t(*reinterpret_cast<const uint16_t *>(row + 68 * st + 34)) << 16;
+// One workgroup per (fragment row set, expert): the 32 rows of fragment index
+// blockIdx.x = 2 c + j (Frag) of the expert's gate/up or down matrix, every K
+// step. First the rows' exponents (8 threads scan a row's scales) and their
+// scales behind the fragments, then a wave per K step.
+template <int T, bool GATEUP>
+__global__ void __launch_bounds__(256) frag_pack_kernel(const void *const *__restrict__ src_tab,
+                                                        void *const *__restrict__ dst_tab, int K, int rows,
+                                                        int64_t row_bytes) {
+    __shared__ float up[32];
+    const int e = blockIdx.y, c = blockIdx.x >> 1, j = blockIdx.x & 1, tid = threadIdx.x, nk = K / kBK;
+    uint8_t *dst = static_cast<uint8_t *>(dst_tab[3 * e + (GATEUP ? 0 : 2)]);
+    if (!dst) return;
+    gbyte *m = gmem(src_tab[3 * e + (GATEUP ? j : 2)]);
+    const int r0 = GATEUP ? 32 * c : 64 * c + 32 * j;
+    {
+        gbyte *row = m + int64_t(r0 + (tid >> 3)) * row_bytes;
+        float b = 0.0f;
+        for (int i = tid & 7; i < Rows<T>::blocks(K); i += 8) {
+            const float v = Rows<T>::bound(row, i);
+            b = v > b || !(v <= 3.4028234663852886e38f) ? v : b;
+        }
+#pragma unroll
+        for (int sh = 1; sh < 8; sh <<= 1) {
+            const float o = __shfl_xor(b, sh, 64);
+            b = o > b || !(o <= 3.4028234663852886e38f) ? o : b;
+        }
+        if ((tid & 7) == 0) {
+            const int ex = exponent_for(b);
+            up[tid >> 3] = ldexpf(1.0f, ex);
+            float *rs = reinterpret_cast<float *>(dst + size_t(GATEUP ? 2 : 1) * rows / 32 * nk * Frag<T>::bytes);
+            rs[(GATEUP ? j * rows : 0) + r0 + (tid >> 3)] = ldexpf(1.0f, -ex);
+        }
     }
-    *reinterpret_cast<uint32_t *>(dst + int64_t(f) * kFragBytes + 4 * w) = v;
+    __syncthreads();
+    const int lane = tid & 63;
+    gbyte *row = m + int64_t(r0 + (lane & 31)) * row_bytes;
+    for (int s = tid >> 6; s < nk; s += 4) {
+        typename Rows<T>::Raw raw;
+        uint32_t w[Op<T>::NW], sc;
+        Rows<T>::load(row, s, lane >> 5, raw);
+        Rows<T>::words(raw, s, lane >> 5, up[lane & 31], w, sc);
+        Frag<T>::store(dst + ((size_t(c) * nk + s) * 2 + j) * Frag<T>::bytes, lane, w, sc);
+    }
+}
+
+size_t frag_bytes(uint32_t t) {
+    return t == VT_Q8_0 ? Frag<VT_Q8_0>::bytes : t == VT_Q4_K ? Frag<VT_Q4_K>::bytes : Frag<VT_Q6_K>::bytes;
+}
+// an expert's gate/up and down fragments with their rows' scales
+size_t pack_gu_bytes(uint32_t tg, int d, int fe) {
+    return (size_t(2) * fe / 32 * (d / kBK) * frag_bytes(tg) + size_t(2) * fe * 4 + 255) & ~size_t(255);
+}
+size_t pack_dn_bytes(uint32_t td, int d, int fe) {
+    return (size_t(d) / 32 * (fe / kBK) * frag_bytes(td) + size_t(d) * 4 + 255) & ~size_t(255);
+}
+
+template <bool GATEUP>
+void pack_launch(uint32_t type, const void *const *table, void *const *dt, int E, int K, int rows, hipStream_t s) {
+    const dim3 g(unsigned((GATEUP ? 2 : 1) * rows / 32), unsigned(E)), b(256);
+    const int64_t rb = vh_row_bytes(type, K);
+    if (type == VT_Q8_0) hipLaunchKernelGGL((frag_pack_kernel<VT_Q8_0, GATEUP>), g, b, 0, s, table, dt, K, rows, rb);
+    else if (type == VT_Q4_K) hipLaunchKernelGGL((frag_pack_kernel<VT_Q4_K, GATEUP>), g, b, 0, s, table, dt, K, rows, rb);
+    else hipLaunchKernelGGL((frag_pack_kernel<VT_Q6_K, GATEUP>), g, b, 0, s, table, dt, K, rows, rb);
 }
 }  // namespace
 
-uint64_t vh_mfma_pack_bytes(int E, int d, int fe) {
-    if (E < 1 || d < kBRows || fe < kBK || d % kBRows || fe % (kBRows / 2) || d % kBK || fe % kBK) return 0;
-    const uint64_t gb = uint64_t(fe) * vh_row_bytes(VT_Q8_0, d), db = uint64_t(d) * vh_row_bytes(VT_Q8_0, fe);
-    return (2 * gb + db) * E;
+uint64_t vh_mfma_pack_bytes(uint32_t tg, uint32_t td, int E, int d, int fe) {
+    if (E < 1 || d < kBRows || fe < kBK || !vh_mfma_supported(tg, td, d, fe, E)) return 0;
+    return uint64_t(E) * (pack_gu_bytes(tg, d, fe) + pack_dn_bytes(td, d, fe));
 }
 
-int vh_mfma_pack_q8(const void *const *table, int E, int d, int fe, void *buf, void **tab_out, hipStream_t s) {
+int vh_mfma_pack(const void *const *table, uint32_t tg, uint32_t td, int E, int d, int fe, void *buf, void **tab_out,
+                 hipStream_t s) {
     *tab_out = nullptr;
-    if (!buf || !vh_mfma_pack_bytes(E, d, fe)) return -EINVAL;
+    if (!buf || !vh_mfma_pack_bytes(tg, td, E, d, fe)) return -EINVAL;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (int rc = vh_check(hipStreamIsCapturing(s, &cap))) return rc;
     if (cap != hipStreamCaptureStatusNone) return -EBUSY;  // no allocation under capture
-    const int64_t rg = vh_row_bytes(VT_Q8_0, d), rd = vh_row_bytes(VT_Q8_0, fe);
-    const size_t gb = size_t(fe) * rg, db = size_t(d) * rd, per = 2 * gb + db;
+    const size_t gb = pack_gu_bytes(tg, d, fe), per = gb + pack_dn_bytes(td, d, fe);
     std::vector<const void *> src(size_t(3) * E), dst(size_t(3) * E, nullptr);
     if (int rc = vh_check(hipMemcpyAsync(src.data(), table, src.size() * sizeof(void *), hipMemcpyDeviceToHost, s)))
         return rc;
@@ -886,14 +1044,13 @@ int vh_mfma_pack_q8(const void *const *table, int E, int d, int fe, void *buf, v
     for (int e = 0; e < E; e++) {
         if (!src[3 * e] || !src[3 * e + 1] || !src[3 * e + 2]) continue;  // unregistered: stays NULL
         dst[3 * e] = dst[3 * e + 1] = b + per * e;  // gate/up fragments
-        dst[3 * e + 2] = b + per * e + 2 * gb;       // down fragments
+        dst[3 * e + 2] = b + per * e + gb;           // down fragments
     }
     int rc = vh_check(hipMemcpy(tab, dst.data(), dst.size() * sizeof(void *), hipMemcpyHostToDevice));
     if (!rc) {
         void *const *dt = static_cast<void *const *>(tab);
-        const dim3 gg(fe / 16 * (d / kBK), E), gd(d / 32 * (fe / kBK), E);
-        hipLaunchKernelGGL(q8_frag_pack_kernel, gg, dim3(576), 0, s, table, dt, 1, d / kBK, rg);
-        hipLaunchKernelGGL(q8_frag_pack_kernel, gd, dim3(576), 0, s, table, dt, 0, fe / kBK, rd);
+        pack_launch<true>(tg, table, dt, E, d, fe, s);
+        pack_launch<false>(td, table, dt, E, fe, d, s);
         rc = vh_check(hipGetLastError());
     }
     if (rc) {
