@@ -223,3 +223,48 @@ def test_contiguous_store_equals_dense(cuda, d, G):
     del before
     for s in (dense, cont, devp):
         s.close()
+
+
+# (kv_dim, block tokens, query heads, kv heads, context): the edges of the
+# attention kernel's 32-token tiles and of its 128 chunks (one tile each up to
+# 4096 tokens), blocks that do not divide a tile, every group size; three heads
+# per kv head take the per-head kernel (2100 blocks: more than 256 chunks)
+EDGES = [(128, 32, 32, 4, 1), (128, 32, 32, 4, 31), (128, 32, 8, 4, 64), (64, 24, 4, 2, 65), (256, 64, 8, 1, 129),
+         (64, 1, 4, 1, 200), (128, 16, 4, 4, 4096), (64, 32, 8, 1, 4097), (128, 64, 8, 2, 16500),
+         (64, 1, 3, 1, 2100), (128, 16, 6, 2, 300)]
+
+
+@pytest.mark.parametrize("d,G,heads,kv_heads,ctx", EDGES)
+def test_attention_tile_edges(cuda, d, G, heads, kv_heads, ctx):
+    """Attention over a dense store (listed blocks) and, where the group size
+    has a grouped kernel, a contiguous one at a device position, against torch
+    in fp64. A score is a sum of d products in fp32, off by at most 2^-24 d of
+    their magnitudes' sum (below 2e-5 of a unit here), and so are the weights:
+    2e-5 of the largest output."""
+    from vireo_amd import kv as KV
+    gen = torch.Generator(device=cuda)
+    gen.manual_seed(d + ctx)
+    k, v = (torch.randn((ctx, kv_heads, d), generator=gen, device=cuda) for _ in range(2))
+    q = torch.randn((heads, d), generator=gen, device=cuda)
+    s = torch.softmax((q.double().view(kv_heads, -1, d) @ k.double().permute(1, 2, 0).contiguous()) / d ** 0.5, -1)
+    want = (s @ v.double().permute(1, 0, 2).contiguous()).reshape(heads, d)
+    outs = []
+    for max_tokens in (0, ctx + 70):
+        st = KV.DeviceKV(kv_heads, d, G, dense=True, max_tokens=max_tokens)
+        out = torch.empty((heads, d), device=cuda)
+        for t in range(ctx):
+            st.append(0, t, k[t], v[t])
+        if max_tokens == 0:
+            st.attend_gqa(0, heads, kv_heads, q, out)
+        elif heads // kv_heads in (1, 2, 4, 8):
+            pos = torch.full((1,), ctx - 1, dtype=torch.int32, device=cuda)
+            st.attend_gqa_pos(0, heads, kv_heads, pos, q, out)
+        else:
+            st.attend_gqa(0, heads, kv_heads, q, out)
+        outs.append(out.clone())
+        torch.cuda.synchronize()
+        st.close()
+    err = float((outs[0].double() - want).abs().max() / want.abs().max())
+    print(f"d={d} G={G} {heads}/{kv_heads} ctx={ctx}: max rel {err:.2e}")
+    assert err <= 2e-5
+    assert torch.equal(outs[0], outs[1])

@@ -23,7 +23,9 @@
 //                      the scores, lane = output dimension for the weighted
 //                      sum), then the four waves merge in order into the
 //                      chunk's partial (m, l, acc);
-//   kv_merge_kernel    per head, the chunks' partials in order: out = acc / l.
+//   kv_attend_group_kernel  the same for the query heads of a kv head at once,
+//                      where they attend the same blocks;
+//   kv_merge_kernel    per head, the chunks' partials in a fixed order: out = acc / l.
 // The work split depends only on the selected token sequence, so a block
 // gives the same bits resident, spilled or paged back.
 #include <hip/hip_runtime.h>
@@ -71,13 +73,6 @@ struct AppendArgs {
     float inv[kMaxAppend];   // 1 / (tokens in the block after this one)
 };
 
-// sum of v over the 64 lanes in lane order (the same on every lane)
-VH_DEV float wave_sum_ordered(float v) {
-    float s = 0.0f;
-    for (int u = 0; u < 64; u++) s += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), u));
-    return s;
-}
-
 // grid n, 64 * DPL threads... (any multiple of 64): row i of k and v into its block
 __global__ void __launch_bounds__(256) kv_append_kernel(AppendArgs a, const float *__restrict__ k,
                                                         const float *__restrict__ v, int d, int gd) {
@@ -106,21 +101,19 @@ __global__ void __launch_bounds__(256) kv_score_kernel(const float *const *__res
     scores[size_t(h) * stride + c] = s;
 }
 
-// partial of chunk c of head h: part[(h * nchunk + c) * (2 + d)] = {m, l, acc[d]}
+// partial of chunk c of head h: the accumulator part[(h * nchunk + c) * d ..], {m, l} in ml[h * nchunk + c]
 template <int DPL>
 __global__ void __launch_bounds__(256) kv_attend_kernel(const KvDesc *__restrict__ desc, const int *__restrict__ off,
                                                         const int *__restrict__ cnt, const float *__restrict__ q,
-                                                        int G, float scale, int nchunk, float *__restrict__ part) {
+                                                        int G, float scale, int nchunk, float *__restrict__ part,
+                                                        float2 *__restrict__ ml) {
     constexpr int D = 64 * DPL;
     __shared__ float qs[D];
     __shared__ float wm[4], wl[4], wacc[4][D];
     const int h = blockIdx.y, c = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int n = cnt[h], e0 = c * kChunkBlocks, e1 = min(n, e0 + kChunkBlocks);
-    float *pout = part + (size_t(h) * nchunk + c) * (2 + D);
-    if (e0 >= n) {  // an empty chunk (heads with fewer entries than others)
-        if (tid == 0) { pout[0] = -INFINITY; pout[1] = 0.0f; }
-        return;
-    }
+    float *pout = part + (size_t(h) * nchunk + c) * D;
+    if (e0 >= n) return;  // past the head's entries: the merge does not read it
     for (int j = tid; j < D; j += 256) qs[j] = q[size_t(h) * D + j];
     __syncthreads();
     float m = -INFINITY, l = 0.0f, acc[DPL];
@@ -183,253 +176,295 @@ __global__ void __launch_bounds__(256) kv_attend_kernel(const KvDesc *__restrict
 #pragma unroll
             for (int i = 0; i < DPL; i++) A[i] = fmaf(wacc[w][lane + 64 * i], f, A[i]);
         }
-        if (lane == 0) { pout[0] = M; pout[1] = L; }
+        if (lane == 0) ml[size_t(h) * nchunk + c] = make_float2(M, L);
 #pragma unroll
-        for (int i = 0; i < DPL; i++) pout[2 + lane + 64 * i] = A[i];
+        for (int i = 0; i < DPL; i++) pout[lane + 64 * i] = A[i];
     }
 }
 
-// out[h] = (sum_c acc_c e^(m_c - M)) / (sum_c l_c e^(m_c - M)), chunks in
-// order: lane c takes chunk c's (m, l) for the maximum and the weights
-// e^(m_c - M) (64 chunks at a time), then every lane adds its columns'
-// accumulators over the chunks in order
-// counts.count(h): the blocks query head h attended
+// out[h] = (sum_c acc_c e^(m_c - M)) / (sum_c l_c e^(m_c - M)). 256 threads per
+// head: thread c % 256 forms chunk c's weight e^(m_c - M) (256 chunks at a
+// time), then group g of D / 4 threads adds the accumulators of chunks g, g + NG,
+// ..., a float4 per thread, and the groups' sums are added in order. One wave
+// per head, 16 chunks' loads in flight, took 22.7 us for 469 chunks and 5.3 us
+// for 64; this takes 4.6 us for up to 128. counts.chunks(h): head h's chunks.
 struct HeadCounts {
     const int *cnt;
-    VH_DEV int count(int h) const { return cnt[h]; }
+    VH_DEV int chunks(int h) const { return (cnt[h] + kChunkBlocks - 1) / kChunkBlocks; }
 };
 template <int DPL, class Counts>
-__global__ void __launch_bounds__(64) kv_merge_kernel(const float *__restrict__ part, Counts counts, int nchunk, int cb,
-                                                      float *__restrict__ out) {
-    constexpr int D = 64 * DPL;
-    __shared__ float fs[64];
-    const int h = blockIdx.x, lane = threadIdx.x;
-    const int nc = (counts.count(h) + cb - 1) / cb;
-    const float *p = part + size_t(h) * nchunk * (2 + D);
+__global__ void __launch_bounds__(256) kv_merge_kernel(const float *__restrict__ part, const float2 *__restrict__ ml,
+                                                       Counts counts, int nchunk, float *__restrict__ out) {
+    constexpr int D = 64 * DPL, NDQ = D / 4, NG = 256 / NDQ, U = 16;
+    __shared__ float fs[256];
+    __shared__ float4 red[NG][NDQ];
+    __shared__ float wm[4], wl[4];
+    const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, dq = tid % NDQ, grp = tid / NDQ;
+    const int nc = counts.chunks(h);
+    const float4 *p = reinterpret_cast<const float4 *>(part + size_t(h) * nchunk * D) + dq;
+    ml += size_t(h) * nchunk;
     float M = -INFINITY;
-    for (int c = lane; c < nc; c += 64) M = fmaxf(M, p[size_t(c) * (2 + D)]);
+    for (int c = tid; c < nc; c += 256) M = fmaxf(M, ml[c].x);
     M = wave_max_f(M);
-    float L = 0.0f, A[DPL];
-#pragma unroll
-    for (int i = 0; i < DPL; i++) A[i] = 0.0f;
-    for (int c0 = 0; c0 < nc; c0 += 64) {
-        const int c = c0 + lane;
+    if (lane == 0) wm[wv] = M;
+    __syncthreads();
+    M = fmaxf(fmaxf(wm[0], wm[1]), fmaxf(wm[2], wm[3]));
+    float L = 0.0f;
+    float4 A = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (int c0 = 0; c0 < nc; c0 += 256) {
+        const int n = min(256, nc - c0);
         float f = 0.0f, lw = 0.0f;
-        if (c < nc) {
-            const float lc = p[size_t(c) * (2 + D) + 1];
-            if (lc != 0.0f) {  // an empty chunk adds nothing
-                f = expf(p[size_t(c) * (2 + D)] - M);
-                lw = lc * f;
+        if (tid < n) {
+            const float2 v = ml[c0 + tid];
+            if (v.y != 0.0f) {  // an empty chunk adds nothing
+                f = expf(v.x - M);
+                lw = v.y * f;
             }
         }
-        fs[lane] = f;
-        // l summed in chunk order: lane 0 adds the 64 weights in turn
+        fs[tid] = f;
+        lw = wave_sum_f(lw);
+        if (lane == 0) wl[wv] = lw;
         __syncthreads();
-        const float lsum = wave_sum_ordered(lw);
-        L += lsum;
-        const int n = min(64, nc - c0);
-        // 16 chunks' loads in flight: the loop is bound by their latency (the
-        // accumulation order, and so the result, does not depend on it; 998 ->
-        // 1 146 tok/s for 48 layers at context 4096 against 4 in flight)
-#pragma unroll 16
-        for (int u = 0; u < n; u++) {
-            const float fu = fs[u];
-            const float *pc = p + size_t(c0 + u) * (2 + D) + 2;
+        L += (wl[0] + wl[1]) + (wl[2] + wl[3]);
+        for (int u0 = grp; u0 < n; u0 += NG * U) {
+            float4 v[U];
 #pragma unroll
-            for (int i = 0; i < DPL; i++) A[i] = fmaf(pc[lane + 64 * i], fu, A[i]);
+            for (int u = 0; u < U; u++) v[u] = p[size_t(c0 + min(u0 + NG * u, n - 1)) * NDQ];
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                if (u0 + NG * u < n) {
+                    const float fu = fs[u0 + NG * u];
+                    A.x = fmaf(v[u].x, fu, A.x);
+                    A.y = fmaf(v[u].y, fu, A.y);
+                    A.z = fmaf(v[u].z, fu, A.z);
+                    A.w = fmaf(v[u].w, fu, A.w);
+                }
         }
         __syncthreads();
     }
-    const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+    red[grp][dq] = A;
+    __syncthreads();
+    if (tid < NDQ) {
+        float4 a = red[0][tid];
 #pragma unroll
-    for (int i = 0; i < DPL; i++) out[size_t(h) * D + lane + 64 * i] = A[i] * inv;
+        for (int u = 1; u < NG; u++) {
+            a.x += red[u][tid].x;
+            a.y += red[u][tid].y;
+            a.z += red[u][tid].z;
+            a.w += red[u][tid].w;
+        }
+        const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+        float *o = out + size_t(h) * D + 4 * tid;  // any 4-byte alignment
+        o[0] = a.x * inv;
+        o[1] = a.y * inv;
+        o[2] = a.z * inv;
+        o[3] = a.w * inv;
+    }
 }
 
-constexpr int kGroupBlocks = 2;  // list entries per workgroup of the grouped-query kernel
-
 // Grouped-query attention when every query head of a group attends the same
-// blocks (selections that do not depend on the query): grid (chunks, kv
-// heads), 256 threads. Chunk c of kv head g covers entries c CB .. c CB + CB - 1
-// of g's list; its keys and values are read once for the HPG query heads
-// g HPG .. g HPG + HPG - 1, whose partials {m, l, acc} it writes as
-// kv_attend_kernel does (chunk size CB). Phases: the scores of every token
-// and head (a quad of lanes per token, a quarter of the dimensions each), the
-// per-head softmax over the chunk (a wave per head), then the weighted sum of
-// the values (a thread per column of 4 dimensions and group of tokens),
-// reduced over the token groups in order.
-// The blocks of kv head g's list: count(g), and entry(g, e) = (block, tokens).
+// blocks (selections that do not depend on the query): grid (chunks, kv heads),
+// 256 threads. The list's tokens are taken in tiles of kTileTok, a chunk's
+// workgroup in tiles c S .. c S + S - 1 with S the least that gives at most
+// kMaxChunks chunks; each tile's keys and values are read once for the HPG query
+// heads g HPG .. g HPG + HPG - 1. Per tile: the scores (eight lanes per token: a
+// load instruction reads eight tokens' 128 consecutive bytes), an online softmax (a wave per head), and the weighted sum
+// of the values (a thread per column of 4 dimensions and group of tokens, over
+// every tile; the groups are added once at the end). The next tile's keys are
+// requested once the scores are formed and its values once they are weighed, so
+// a workgroup's loads stay in flight across its phases. Bound by the read of the
+// keys and values at long contexts and by the load's round trip and the phases
+// at short ones. Per layer of 4 kv heads of 128 with the append and the merge,
+// against one 64-token tile per workgroup with four lanes per token (whose loads
+// each touched 64 lines): 30 001 tokens (123 MB) 63.7 -> 36.5 us, 4096 tokens (17 MB)
+// 19.5 -> 16.9 us. 64-token tiles: 37.5 and 17.8; of those, 64, 96 and 256 chunks at
+// 30 001 tokens: 44, 39.5 and 44 us.
+constexpr int kTileTok = 32, kMaxChunks = 128;
+
+// The blocks of kv head g's list: tokens(g) - every block but the last is full -
+// and block(g, e).
 struct ListedBlocks {  // lists uploaded by the host
     const KvDesc *desc;
     const int *off, *cnt;
-    VH_DEV int count(int g) const { return cnt[g]; }
-    VH_DEV KvDesc entry(int g, int e) const { return desc[off[g] + e]; }
+    int G;
+    VH_DEV int tokens(int g) const {
+        const int n = cnt[g];
+        return n == 0 ? 0 : (n - 1) * G + desc[off[g] + n - 1].ntok;
+    }
+    VH_DEV const float *block(int g, int e) const { return desc[off[g] + e].blk; }
 };
 struct ContiguousBlocks {  // a contiguous store at the position *pos (every block attended)
     const float *base;  // block b of layer l at base + (l * max_blocks + b) * 2 G D
     const int *pos;
     int layer0, max_blocks, G, D;
-    VH_DEV int count(int) const {
-        const int p = *pos;
-        return p < 0 ? 0 : min(p / G + 1, max_blocks);
-    }
-    VH_DEV KvDesc entry(int g, int e) const {
-        const int p = *pos, last = p / G;
-        KvDesc k;
-        k.blk = base + (size_t(layer0 + g) * max_blocks + e) * size_t(2 * G * D);
-        k.ntok = e < last ? G : p % G + 1;
-        k.pad = 0;
-        return k;
+    VH_DEV int tokens(int) const { return min(max(*pos + 1, 0), max_blocks * G); }
+    VH_DEV const float *block(int g, int e) const {
+        return base + (size_t(layer0 + g) * max_blocks + e) * size_t(2 * G * D);
     }
 };
 
-// a query head's count is its kv head's list's (the heads of a group attend
+VH_DEV int tiles_per_chunk(int tiles) { return (tiles + kMaxChunks - 1) / kMaxChunks; }
+
+// a query head's chunks are its kv head's list's (the heads of a group attend
 // the same blocks)
 template <class Lists>
 struct GroupCounts {
     Lists lists;
     int hpg;
-    VH_DEV int count(int h) const { return lists.count(h / hpg); }
+    VH_DEV int chunks(int h) const {
+        const int tiles = (lists.tokens(h / hpg) + kTileTok - 1) / kTileTok, s = tiles_per_chunk(tiles);
+        return s ? (tiles + s - 1) / s : 0;
+    }
 };
 
 template <int D, int HPG, class Lists>
-__global__ void __launch_bounds__(256) kv_attend_group_kernel(Lists lists, const float *__restrict__ q, int G,
-                                                              float scale, int nchunk, float *__restrict__ part) {
-    constexpr int CB = kGroupBlocks, TMAX = CB * 64, QD = D / 4, NDQ = D / 4, NTG = 256 / NDQ;
-    __shared__ float4 qs[HPG][D / 4];
-    __shared__ float ps[HPG][TMAX];
-    __shared__ float hm[HPG], hl[HPG];
+__global__ void __launch_bounds__(256, D <= 128 ? 3 : 2) kv_attend_group_kernel(Lists lists, const float *__restrict__ q, int G,
+                                                              float scale, int nchunk, float *__restrict__ part,
+                                                              float2 *__restrict__ ml) {
+    constexpr int KF = D / 32, NDQ = D / 4, NTG = 256 / NDQ, MT = kTileTok / NTG;
+    __shared__ float4 qs[HPG][NDQ];
+    __shared__ float ps[2][HPG][kTileTok], cf[2][HPG];
     __shared__ float4 red[NTG][HPG][NDQ];
     const int g = blockIdx.y, c = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int n = lists.count(g), e0 = c * CB, e1 = min(n, e0 + CB);
-    if (e0 >= n) {  // an empty chunk: its heads' partials are empty
-        if (tid < HPG) {
-            float *po = part + (size_t(g * HPG + tid) * nchunk + c) * (2 + D);
-            po[0] = -INFINITY;
-            po[1] = 0.0f;
-        }
-        return;
-    }
-    for (int i = tid; i < HPG * (D / 4); i += 256)
-        qs[i / (D / 4)][i % (D / 4)] = reinterpret_cast<const float4 *>(q + size_t(g) * HPG * D)[i];
-    const KvDesc d0 = lists.entry(g, e0), d1 = e0 + 1 < e1 ? lists.entry(g, e0 + 1) : KvDesc{d0.blk, 0, 0};
-    const float *B0 = d0.blk, *B1 = d1.blk;
-    const int n0 = d0.ntok, T = n0 + d1.ntok;
-    auto krow = [&](int t) { return t < n0 ? B0 + size_t(t) * D : B1 + size_t(t - n0) * D; };  // V at + G D
-    // the values this thread weighs in the last phase, loaded before the scores
-    // are formed (D <= 128: at most 16 float4 per thread)
-    const int dq = tid % NDQ, tg = tid / NDQ;
-    constexpr int MT = D <= 128 ? TMAX / NTG : 1;
-    float4 vv[MT];
-    if constexpr (D <= 128) {
+    for (int i = tid; i < HPG * NDQ; i += 256)
+        qs[i / NDQ][i % NDQ] = reinterpret_cast<const float4 *>(q + size_t(g) * HPG * D)[i];
+    const int T = lists.tokens(g), tiles = (T + kTileTok - 1) / kTileTok, S = tiles_per_chunk(tiles);
+    const int i0 = c * S, i1 = min(tiles, i0 + S);
+    if (i0 >= i1) return;  // past the list's chunks: the merge does not read it
+    // row tt of tile i (a row past the list repeats its last one); keys at 0, values at G D
+    const int mg = (65536 + G - 1) / G;  // x / G = x mg >> 16 for x < 96, G <= 64
+    auto row = [&](int i, int tt) {
+        const int t0 = i * kTileTok, e0 = t0 / G, x = t0 - e0 * G + min(tt, T - 1 - t0), e = (x * mg) >> 16;
+        return lists.block(g, e0 + e) + size_t(x - e * G) * D;
+    };
+    const int o = tid & 7, ta = tid >> 3;           // scores: token ta, float4s 8 j + o
+    const int dq = tid % NDQ, tg = tid / NDQ;        // values: column dq of tokens tg + NTG m
+    float4 kk[KF], vv[MT];
+    auto load_k = [&](int i) {
+        const float4 *r = reinterpret_cast<const float4 *>(row(i, ta)) + o;
 #pragma unroll
-        for (int m = 0; m < MT; m++) {
-            const int t = tg + NTG * m;
-            vv[m] = t < T ? reinterpret_cast<const float4 *>(krow(t) + size_t(G) * D)[dq] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        }
-    }
-    __syncthreads();
-    // scores: lanes 4m .. 4m + 3 take token t = tid / 4 (+ 64 j), quarter tid % 4
-    const int qd = tid & 3;
+        for (int j = 0; j < KF; j++) kk[j] = r[8 * j];
+    };
+    auto load_v = [&](int i) {
 #pragma unroll
-    for (int t0 = 0; t0 < TMAX; t0 += 64) {
-        const int t = t0 + (tid >> 2);
-        float sc[HPG];
-#pragma unroll
-        for (int i = 0; i < HPG; i++) sc[i] = 0.0f;
-        if (t < T) {
-            const float4 *kr = reinterpret_cast<const float4 *>(krow(t) + qd * QD);
-#pragma unroll
-            for (int j = 0; j < QD / 4; j++) {
-                const float4 kk = kr[j];
-#pragma unroll
-                for (int i = 0; i < HPG; i++) {
-                    const float4 qq = qs[i][qd * (QD / 4) + j];
-                    sc[i] = fmaf(qq.x, kk.x, fmaf(qq.y, kk.y, fmaf(qq.z, kk.z, fmaf(qq.w, kk.w, sc[i]))));
-                }
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < HPG; i++) {
-            sc[i] += dpp_f<0xB1>(sc[i]);
-            sc[i] += dpp_f<0x4E>(sc[i]);
-        }
-        if (qd == 0 && t < T)
-#pragma unroll
-            for (int i = 0; i < HPG; i++) ps[i][t] = sc[i] * scale;
-    }
-    __syncthreads();
-    // softmax of each head over the chunk's tokens: wave w takes heads w, w + 4, ...
-    for (int i = wv; i < HPG; i += 4) {
-        const float a = lane < T ? ps[i][lane] : -INFINITY, b = lane + 64 < T ? ps[i][lane + 64] : -INFINITY;
-        const float mx = wave_max_f(fmaxf(a, b));
-        const float pa = lane < T ? expf(a - mx) : 0.0f, pb = lane + 64 < T ? expf(b - mx) : 0.0f;
-        const float l = wave_sum_f(pa + pb);
-        if (lane < T) ps[i][lane] = pa;
-        if (lane + 64 < T) ps[i][lane + 64] = pb;
-        if (lane == 0) {
-            hm[i] = mx;
-            hl[i] = l;
-        }
-    }
-    __syncthreads();
-    // weighted values: thread (token group tg, column dq) sums tokens tg, tg + NTG, ...
+        for (int m = 0; m < MT; m++) vv[m] = reinterpret_cast<const float4 *>(row(i, tg + NTG * m) + size_t(G) * D)[dq];
+    };
+    load_k(i0);
+    load_v(i0);
+    float rm[2] = {-INFINITY, -INFINITY}, rl[2] = {0.0f, 0.0f};  // the wave's heads wv, wv + 4
     float4 acc[HPG];
 #pragma unroll
     for (int i = 0; i < HPG; i++) acc[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    auto weigh = [&](const float4 &v, int t) {
+    lds_barrier();  // qs
+    for (int it = i0; it < i1; it++) {
+        const int b = (it - i0) & 1, lim = T - it * kTileTok;  // tokens of the tile (lim >= kTileTok: all)
+        float sc[HPG];
+        int oq = o;
+        asm volatile("" : "+v"(oq));  // the queries are read again in every tile, not held in registers
 #pragma unroll
         for (int i = 0; i < HPG; i++) {
-            const float pt = ps[i][t];
-            acc[i].x = fmaf(pt, v.x, acc[i].x);
-            acc[i].y = fmaf(pt, v.y, acc[i].y);
-            acc[i].z = fmaf(pt, v.z, acc[i].z);
-            acc[i].w = fmaf(pt, v.w, acc[i].w);
+            sc[i] = 0.0f;
+#pragma unroll
+            for (int j = 0; j < KF; j++) {
+                const float4 qq = qs[i][8 * j + oq];
+                sc[i] = fmaf(qq.x, kk[j].x, fmaf(qq.y, kk[j].y, fmaf(qq.z, kk[j].z, fmaf(qq.w, kk[j].w, sc[i]))));
+            }
+            // formed here: sunk past the next loads, the products would hold both
+            // tiles' keys and every head's queries in registers
+            asm volatile("" : "+v"(sc[i]));
+            if (i & 1) __builtin_amdgcn_sched_barrier(0);
         }
-    };
-    if constexpr (D <= 128) {
+        __builtin_amdgcn_sched_barrier(0);
+        load_k(min(it + 1, i1 - 1));
+#pragma unroll
+        for (int i = 0; i < HPG; i++) {
+            float v = sc[i];
+            v += dpp_f<0xB1>(v);
+            v += dpp_f<0x4E>(v);
+            v += dpp_f<0x141>(v);
+            if (o == i) ps[b][i][ta] = ta < lim ? v * scale : -INFINITY;
+        }
+        lds_barrier();
+        // online softmax: wave w takes heads w, w + 4
+#pragma unroll
+        for (int x = 0; x < (HPG + 3) / 4; x++) {
+            const int i = wv + 4 * x;
+            if (i >= HPG) break;
+            const float a = lane < kTileTok ? ps[b][i][lane] : -INFINITY, mn = fmaxf(rm[x], wave_max_f(a));
+            const float corr = expf(rm[x] - mn), pa = lane < lim ? expf(a - mn) : 0.0f;
+            rl[x] = rl[x] * corr + wave_sum_f(pa);
+            rm[x] = mn;
+            if (lane < kTileTok) ps[b][i][lane] = pa;
+            if (lane == 0) cf[b][i] = corr;
+        }
+        lds_barrier();
+#pragma unroll
+        for (int i = 0; i < HPG; i++) {
+            const float f = cf[b][i];
+            acc[i].x *= f;
+            acc[i].y *= f;
+            acc[i].z *= f;
+            acc[i].w *= f;
+        }
 #pragma unroll
         for (int m = 0; m < MT; m++)
-            if (tg + NTG * m < T) weigh(vv[m], tg + NTG * m);
-    } else {
-        for (int t = tg; t < T; t += NTG) weigh(reinterpret_cast<const float4 *>(krow(t) + size_t(G) * D)[dq], t);
+            if (tg + NTG * m < lim)
+#pragma unroll
+                for (int i = 0; i < HPG; i++) {
+                    const float pt = ps[b][i][tg + NTG * m];
+                    acc[i].x = fmaf(pt, vv[m].x, acc[i].x);
+                    acc[i].y = fmaf(pt, vv[m].y, acc[i].y);
+                    acc[i].z = fmaf(pt, vv[m].z, acc[i].z);
+                    acc[i].w = fmaf(pt, vv[m].w, acc[i].w);
+                }
+#pragma unroll
+        for (int i = 0; i < HPG; i++) asm volatile("" : "+v"(acc[i].x), "+v"(acc[i].y), "+v"(acc[i].z), "+v"(acc[i].w));
+        __builtin_amdgcn_sched_barrier(0);
+        load_v(min(it + 1, i1 - 1));
     }
 #pragma unroll
     for (int i = 0; i < HPG; i++) red[tg][i][dq] = acc[i];
-    __syncthreads();
+#pragma unroll
+    for (int x = 0; x < (HPG + 3) / 4; x++)
+        if (wv + 4 * x < HPG && lane == 0)
+            ml[size_t(g * HPG + wv + 4 * x) * nchunk + c] = make_float2(rm[x], rl[x]);
+    lds_barrier();
     for (int x = tid; x < HPG * NDQ; x += 256) {
         const int i = x / NDQ, col = x % NDQ;
         float4 a = red[0][i][col];
+#pragma unroll
         for (int u = 1; u < NTG; u++) {
-            const float4 b = red[u][i][col];
-            a.x += b.x;
-            a.y += b.y;
-            a.z += b.z;
-            a.w += b.w;
+            a.x += red[u][i][col].x;
+            a.y += red[u][i][col].y;
+            a.z += red[u][i][col].z;
+            a.w += red[u][i][col].w;
         }
-        float *po = part + (size_t(g * HPG + i) * nchunk + c) * (2 + D);
-        po[2 + 4 * col] = a.x;
-        po[3 + 4 * col] = a.y;
-        po[4 + 4 * col] = a.z;
-        po[5 + 4 * col] = a.w;
-        if (col == 0) {
-            po[0] = hm[i];
-            po[1] = hl[i];
-        }
+        reinterpret_cast<float4 *>(part + (size_t(g * HPG + i) * nchunk + c) * D)[col] = a;
     }
+}
+
+// the partials of n_heads heads of nchunk chunks: accumulators, then {m, l}
+size_t part_floats(int n_heads, int nchunk, int d) { return size_t(n_heads) * nchunk * (d + 2); }
+
+// chunks of the grouped-query kernel for at most `tokens` tokens
+int group_chunks(int64_t tokens) {
+    const int64_t tiles = (tokens + kTileTok - 1) / kTileTok;
+    return int(tiles < kMaxChunks ? (tiles > 0 ? tiles : 1) : kMaxChunks);
 }
 
 template <int D, class Lists>
 int launch_group(int hpg, Lists lists, const float *q, int G, float scale, int nchunk, int n_kv, int n_heads,
                  float *part, float *out, hipStream_t s) {
     const dim3 g(nchunk, n_kv);
+    float2 *ml = reinterpret_cast<float2 *>(part + size_t(n_heads) * nchunk * D);
     switch (hpg) {
-    case 1: hipLaunchKernelGGL((kv_attend_group_kernel<D, 1, Lists>), g, dim3(256), 0, s, lists, q, G, scale, nchunk, part); break;
-    case 2: hipLaunchKernelGGL((kv_attend_group_kernel<D, 2, Lists>), g, dim3(256), 0, s, lists, q, G, scale, nchunk, part); break;
-    case 4: hipLaunchKernelGGL((kv_attend_group_kernel<D, 4, Lists>), g, dim3(256), 0, s, lists, q, G, scale, nchunk, part); break;
-    default: hipLaunchKernelGGL((kv_attend_group_kernel<D, 8, Lists>), g, dim3(256), 0, s, lists, q, G, scale, nchunk, part); break;
+    case 1: hipLaunchKernelGGL((kv_attend_group_kernel<D, 1, Lists>), g, dim3(256), 0, s, lists, q, G, scale, nchunk, part, ml); break;
+    case 2: hipLaunchKernelGGL((kv_attend_group_kernel<D, 2, Lists>), g, dim3(256), 0, s, lists, q, G, scale, nchunk, part, ml); break;
+    case 4: hipLaunchKernelGGL((kv_attend_group_kernel<D, 4, Lists>), g, dim3(256), 0, s, lists, q, G, scale, nchunk, part, ml); break;
+    default: hipLaunchKernelGGL((kv_attend_group_kernel<D, 8, Lists>), g, dim3(256), 0, s, lists, q, G, scale, nchunk, part, ml); break;
     }
-    hipLaunchKernelGGL((kv_merge_kernel<D / 64, GroupCounts<Lists>>), dim3(n_heads), dim3(64), 0, s, part,
-                       GroupCounts<Lists>{lists, hpg}, nchunk, kGroupBlocks, out);
+    hipLaunchKernelGGL((kv_merge_kernel<D / 64, GroupCounts<Lists>>), dim3(n_heads), dim3(256), 0, s, part, ml,
+                       GroupCounts<Lists>{lists, hpg}, nchunk, out);
     return vh_check(hipGetLastError());
 }
 
@@ -439,20 +474,21 @@ __global__ void __launch_bounds__(256) kv_append_pos_kernel(float *__restrict__ 
                                                             int layer0, int max_blocks, int max_tokens,
                                                             const int *__restrict__ pos_p, const float *__restrict__ k,
                                                             const float *__restrict__ v, int d, int G) {
+    // a thread per column (kv_dim is 64, 128 or 256); the rows are requested with the position, not after it
+    const int i = blockIdx.x;
+    const float k0 = k[size_t(i) * d + threadIdx.x], v0 = v[size_t(i) * d + threadIdx.x];
     const int pos = *pos_p;
     if (pos < 0 || pos >= max_tokens) return;
-    const int i = blockIdx.x, b = pos / G, slot = pos % G;
+    const int b = pos / G, slot = pos % G;
     const size_t li = size_t(layer0 + i) * max_blocks + b;
     float *blk = base + li * size_t(2 * G * d);
     float *ks = ksum + li * size_t(d);
     const float inv = 1.0f / float(slot + 1);
-    for (int j = threadIdx.x; j < d; j += blockDim.x) {
-        const float kj = k[size_t(i) * d + j];
-        blk[size_t(slot) * d + j] = kj;
-        blk[size_t(G + slot) * d + j] = v[size_t(i) * d + j];
-        const float old = slot == 0 ? 0.0f : ks[j];  // a new block's mean starts at zero
-        ks[j] = add_rn(old, mul_rn(sub_rn(kj, old), inv));
-    }
+    const int j = threadIdx.x;
+    blk[size_t(slot) * d + j] = k0;
+    blk[size_t(G + slot) * d + j] = v0;
+    const float old = slot == 0 ? 0.0f : ks[j];  // a new block's mean starts at zero
+    ks[j] = add_rn(old, mul_rn(sub_rn(k0, old), inv));
 }
 
 int blocks_for(int tokens, int g) { return tokens > 0 ? (tokens + g - 1) / g : 0; }
@@ -706,10 +742,11 @@ void select_blocks(const VireoKV *S, int nb, const float *scores, std::vector<un
 template <int DPL>
 void launch_attend(const KvDesc *desc, const int *off, const int *cnt, const float *q, int G, float scale,
                    int nchunk, int heads, float *part, float *out, hipStream_t s) {
+    float2 *ml = reinterpret_cast<float2 *>(part + size_t(heads) * nchunk * 64 * DPL);
     hipLaunchKernelGGL((kv_attend_kernel<DPL>), dim3(nchunk, heads), dim3(256), 0, s, desc, off, cnt, q, G, scale,
-                       nchunk, part);
-    hipLaunchKernelGGL((kv_merge_kernel<DPL, HeadCounts>), dim3(heads), dim3(64), 0, s, part, HeadCounts{cnt}, nchunk,
-                       kChunkBlocks, out);
+                       nchunk, part, ml);
+    hipLaunchKernelGGL((kv_merge_kernel<DPL, HeadCounts>), dim3(heads), dim3(256), 0, s, part, ml, HeadCounts{cnt},
+                       nchunk, out);
 }
 
 // heads h < n_heads attend layer layer0 + h / kv_mul with q_h
@@ -770,7 +807,7 @@ int attend(VireoKV *S, int layer0, int n_heads, int kv_mul, const float *q, floa
     const bool grouped = S->strategy != VIREO_KV_SELECT_TOPK &&
                          (kv_mul == 1 || kv_mul == 2 || kv_mul == 4 || kv_mul == 8) &&
                          !(reinterpret_cast<uintptr_t>(q) & 15u);
-    const int n_lists = grouped ? n_heads / kv_mul : n_heads, cb = grouped ? kGroupBlocks : kChunkBlocks;
+    const int n_lists = grouped ? n_heads / kv_mul : n_heads;
     std::vector<KvDesc> desc;
     std::vector<int> off(static_cast<size_t>(n_lists)), cnt(static_cast<size_t>(n_heads));
     std::vector<KvBlock *> leased;
@@ -790,7 +827,7 @@ int attend(VireoKV *S, int layer0, int n_heads, int kv_mul, const float *q, floa
             got++;
         }
         cnt[h] = got;
-        const int nc = (got + cb - 1) / cb;
+        const int nc = grouped ? group_chunks(int64_t(got) * S->G) : (got + kChunkBlocks - 1) / kChunkBlocks;
         nchunk = nc > nchunk ? nc : nchunk;
     }
     if (!rc) {
@@ -800,7 +837,7 @@ int attend(VireoKV *S, int layer0, int n_heads, int kv_mul, const float *q, floa
             for (int g = 0; g < n_lists; g++) cnt_list.push_back(cnt[size_t(g) * kv_mul]);
         const size_t db = desc.size() * sizeof(KvDesc);
         const size_t ib = (size_t(n_lists) * (grouped ? 2 : 1) + size_t(n_heads)) * sizeof(int);
-        const size_t pb = size_t(n_heads) * nchunk * (2 + d) * sizeof(float);
+        const size_t pb = part_floats(n_heads, nchunk, d) * sizeof(float);
         void *dv = nullptr, *hv = nullptr;
         int slot = 0;
         rc = scratch(S, db + ib + 256, s, &dv);
@@ -822,7 +859,7 @@ int attend(VireoKV *S, int layer0, int n_heads, int kv_mul, const float *q, floa
             const int *dcnt_list = doff + n_lists, *dcnt = doff + n_lists * (grouped ? 2 : 1);
             const float scale = 1.0f / sqrtf(float(d));
             if (!rc && grouped) {
-                const ListedBlocks lb{dd, doff, dcnt_list};
+                const ListedBlocks lb{dd, doff, dcnt_list, S->G};
                 if (d == 64) rc = launch_group<64>(kv_mul, lb, q, S->G, scale, nchunk, n_lists, n_heads, S->part, out, s);
                 else if (d == 128) rc = launch_group<128>(kv_mul, lb, q, S->G, scale, nchunk, n_lists, n_heads, S->part, out, s);
                 else rc = launch_group<256>(kv_mul, lb, q, S->G, scale, nchunk, n_lists, n_heads, S->part, out, s);
@@ -915,7 +952,7 @@ extern "C" int vireo_kv_append_pos(VireoKV *S, int layer0, int n, const int32_t 
                                    void *stream) {
     if (!S || !S->contig || !pos || n < 1 || layer0 < 0 || layer0 + n > S->cfg.n_layers || !k || !v) return -EINVAL;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(kv_append_pos_kernel, dim3(n), dim3(S->d < 256 ? S->d : 256), 0, s, S->cbase, S->cksum, layer0,
+    hipLaunchKernelGGL(kv_append_pos_kernel, dim3(n), dim3(S->d), 0, s, S->cbase, S->cksum, layer0,
                        S->max_blocks, S->max_blocks * S->G, pos, k, v, S->d, S->G);
     return vh_finish(s, vh_check(hipGetLastError()));
 }
@@ -928,8 +965,8 @@ extern "C" int vireo_kv_attend_gqa_pos(VireoKV *S, int layer0, int n_heads, int 
     const int kv_mul = n_heads / n_kv_heads, d = S->d;
     if (kv_mul != 1 && kv_mul != 2 && kv_mul != 4 && kv_mul != 8) return -EINVAL;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const int nchunk = (S->max_blocks + kGroupBlocks - 1) / kGroupBlocks;
-    const size_t pb = size_t(n_heads) * nchunk * (2 + d) * sizeof(float);
+    const int nchunk = group_chunks(int64_t(S->max_blocks) * S->G);
+    const size_t pb = part_floats(n_heads, nchunk, d) * sizeof(float);
     if (int rc = grow(S, &S->part, &S->part_bytes, pb)) return rc;  // the first call sizes the partials
     const ContiguousBlocks cb{S->cbase, pos, layer0, S->max_blocks, S->G, d};
     const float scale = 1.0f / sqrtf(float(d));
