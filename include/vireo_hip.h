@@ -241,11 +241,11 @@ int vireo_hip_set_path(int path);
  * it. expert_store_packed_bytes reports the copies' bytes. A copy is made
  * from the pinned views and freed with the pin (expert_store_unpin_layer) or
  * the store; a caller that rewrites a pinned layer's expert bytes in place
- * must unpin and pin it again. Calls of 64 or more tokens on a pinned layer of Q8_0, Q4_K
- * or Q6_K experts make and read, the same way, a copy in matrix-operand
- * fragments (each lane's words of a 32-row, 64-column step together; 1.0, 1.1
- * and 1.07 times the expert bytes) for the prefill GEMMs. Results
- * are the same bit for bit either way. 0 turns both off for later calls
+ * must unpin and pin it again. Calls of 64 or more tokens on a pinned layer of
+ * Q8_0, Q4_K or Q6_K experts, and of 9 or more on Q8_0 experts, make and read,
+ * the same way, a copy in matrix-operand fragments (each lane's words of a
+ * 32-row, 64-column step together; 1.0, 1.1 and 1.07 times the expert bytes).
+ * Results are the same bit for bit either way. 0 turns both off for later calls
  * (existing copies stay until unpinned). No counterpart in the reference. */
 int vireo_hip_set_packed(int on);
 

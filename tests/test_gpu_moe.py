@@ -461,6 +461,45 @@ def test_grouped_plan_large_groups(cuda, oracle, path, name, T, zipf, plan):
     m.close()
 
 
+@pytest.mark.parametrize("E,k,d,fe", [(8, 2, 512, 384), (32, 4, 2048, 1152), (24, 11, 256, 128)])
+@pytest.mark.parametrize("T", [9, 16, 17, 40, 63])
+def test_q8_decode_batch(cuda, oracle, E, k, d, fe, T):
+    """The matrix-core decode batch of Q8_0 experts (9 to 63 tokens): groups of one
+    token to several tiles of 16 and passes of 32 (8 experts), more than 8
+    experts per token (24), down rows of an odd number of step pairs (384), two
+    unregistered experts, tokens whose inputs differ by 2^12; on the GGUF rows and
+    on the fragment copy (the same bits). A product's fp16 parts drop 2^-22 of an
+    input and the sums are fp32: 1e-5 of a token's largest contribution. Inputs are
+    scaled down only: a routing weight's relative error is its logits' absolute one,
+    d fp32 roundings of the inputs' size (1.5e-5 in every plan at inputs of 2^6)."""
+    lib = _lib.load()
+    shape = W.MoEShape("q8dec", d, E, k, fe, True, W.Q8_0, W.Q8_0, W.Q8_0)
+    bias = np.linspace(0.0, 2.0, E).astype(np.float32)
+    drop = {(0, 1), (0, E - 2)}
+    m = M.DeviceMoE(shape, 1, seed=73, logit_bias=bias, unregistered=drop)
+    m._unregistered = drop
+    x, hb = W.host_hidden(d, T, 73)
+    hb = hb * np.exp2(-(np.arange(T) % 13)).astype(np.float32)[:, None]
+    hbt = torch.from_numpy(hb).to(cuda)
+    outs = []
+    try:
+        for packed in (0, 1):
+            _lib.check(lib.vireo_hip_set_packed(packed), "vireo_hip_set_packed")
+            xt = torch.zeros((T, d), device=cuda)
+            idx, _ = m.forward(0, xt, hbt, return_routing=True)
+            outs.append(xt.cpu().numpy())
+    finally:
+        lib.vireo_hip_set_packed(1)
+    np.testing.assert_array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+    xo, io, _, _ = oracle_layer(oracle, m, 0, np.zeros_like(x), hb)
+    np.testing.assert_array_equal(idx.cpu().numpy(), io)
+    size = np.maximum(np.abs(xo).max(1), 1e-30)
+    rel = np.abs(outs[1] - xo).max(1) / size
+    print(f"E={E} T={T}: groups up to {np.bincount(io.ravel(), minlength=E).max()}, max rel {rel.max():.2e}")
+    assert rel.max() <= 1e-5
+    m.close()
+
+
 # gate/up and down types; fe = 1152 and 1280 take more than the 32 blocks of h
 # whose factors the down GEMM holds at a time
 EDGE_TYPES = [(W.Q4_K, W.Q6_K, 512), (W.Q8_0, W.Q8_0, 1152), (W.Q6_K, W.Q4_K, 1280)]

@@ -12,7 +12,8 @@
 // many tokens chose it. In calls of at least kMfmaMinCall tokens every group
 // runs as fp16 matrix-core GEMMs (moe_mfma.hip; 3 more kernels); calls of
 // kMdecMinTokens to kMfmaMinCall - 1 tokens with Q4_K_M experts run their
-// groups on the matrix cores with exact 16-bit operands (moe_mdec.hip), and
+// groups on the matrix cores with exact 16-bit operands (moe_mdec.hip), from
+// kQ8decMinTokens on with Q8_0 experts too (moe_q8dec.hip), and
 // smaller calls (or other types) on moe_gdec.hip's kernels, which keep a
 // group's inputs in registers and stream each weight row once; plan 4 runs
 // every call on the fp32 grouped kernels (moe_grouped.hip).
@@ -60,6 +61,14 @@ constexpr int kMdecMinTokens = 3;
 // B=8 108.4 / 131.1.
 constexpr int kDecodeBatchAuto = 4;
 
+// From this many tokens on, calls on Q8_0 layers run on the matrix cores
+// (moe_q8dec.hip), below on the decode plan for every token. Measured per layer
+// (decode plan / matrix cores): OLMoE Q8_0 4 tokens 84.6 / 87.5 us, 6 84.3 / 91.9, 8
+// 111 / 98.6; Qwen3 Q8_0 6 tokens 73.7 / 86.3, 8 90.7 / 91.8. Against the fp32
+// grouped kernels before: OLMoE 23 tokens 175 -> 117, 63 tokens 341 -> 171; Qwen3 12
+// tokens 157 -> 116, 40 tokens 288 -> 193.
+constexpr int kQ8decMinTokens = 9;
+
 bool type_ok(uint32_t t, int n) {
     // the expert formats of the MoE models (Q8_0, Q4_K gate/up, Q6_K down), and
     // the other types the reference's gguf_matmul computes (src/gguf_run.c:
@@ -98,6 +107,7 @@ struct Ws {
     void *xp;                // decode-batch matrix-core plan: split inputs [T x d x 4 bytes]
     float *xsc;              // either matrix-core plan's per-token scales [T]
     uint32_t *ctr;           // and the down kernel's arrival counters (vh_mdec_ctr_words)
+    float *hsc;              // Q8_0 decode batch: block scales of h [P x fe / 32]
     const void **tab;        // paged plan: [E + 1] expert tables [3 E] (one per batch, then the combine's)
     int32_t *act;            // paged plan: [E] active lists [E + 1] (one per batch)
     int32_t *pidx;           // paged plan: the next layer's guessed routing [T x k]
@@ -136,6 +146,7 @@ int get_ws(int T, int E, int k, int d, int fe, bool experts, bool grouped, Ws *w
     const bool small = experts && grouped && T < kMfmaMinCall;
     const size_t o_xp = small ? take(vh_mdec_xp_bytes(T, d)) : 0, o_xsc = small ? take(size_t(T) * 4) : 0;
     const size_t o_ctr = small ? take(size_t(vh_mdec_ctr_words(d)) * 4) : 0;
+    const size_t o_hsc = small ? take(P * (fe / 32) * 4) : 0;
     const size_t o_tab = paged ? take(size_t(E + 1) * 3 * E * sizeof(void *)) : 0,
                  o_act = paged ? take(size_t(E) * (E + 1) * 4) : 0;
     const size_t o_pidx = paged ? take(P * 4) : 0, o_pw = paged ? take(P * 4) : 0,
@@ -169,6 +180,7 @@ int get_ws(int T, int E, int k, int d, int fe, bool experts, bool grouped, Ws *w
               : mfma ? reinterpret_cast<float *>(b + o_parts + he_bytes)
                      : nullptr;
     ws->ctr = small ? reinterpret_cast<uint32_t *>(b + o_ctr) : nullptr;
+    ws->hsc = small ? reinterpret_cast<float *>(b + o_hsc) : nullptr;
     ws->tab = paged ? reinterpret_cast<const void **>(b + o_tab) : nullptr;
     ws->act = paged ? reinterpret_cast<int32_t *>(b + o_act) : nullptr;
     ws->pidx = paged ? reinterpret_cast<int32_t *>(b + o_pidx) : nullptr;
@@ -787,15 +799,18 @@ int ffn_forward(const vireo_moe_model *m, int layer, float *x, const float *hb, 
     const int P = n_tokens * k, slots = P < E ? P : E;
     const bool mdec = !mfma && n_tokens >= kMdecMinTokens && n_tokens < kMfmaMinCall && g_path != 4 &&
                       vh_mdec_supported(tg, td, d, fe);
+    const bool q8dec = !mfma && n_tokens >= kQ8decMinTokens && n_tokens < kMfmaMinCall && g_path != 4 &&
+                       vh_q8dec_supported(tg, td, d, fe, n_tokens);
     // the matrix-core decode batch's split inputs come with the router parts where the tiled kernel runs
-    rc = mdec ? vh_route_parts_tiled(R, hb, L.logit_bias, d, E, n_tokens, ws.parts, ws.xp, ws.xsc, s) : -EINVAL;
+    rc = mdec || q8dec ? vh_route_parts_tiled(R, hb, L.logit_bias, d, E, n_tokens, ws.parts, ws.xp, ws.xsc, s, q8dec)
+                       : -EINVAL;
     const bool prepped = rc == 0;
     if (rc == -EINVAL) rc = vh_route_parts(R, hb, L.logit_bias, d, E, n_tokens, exact, ws.parts, s);
     if (!rc) rc = vh_route_finish(ws.parts, R, hb, L.logit_bias, d, E, k, m->topk_renorm, exact, n_tokens, idx, w,
                                   ws.flags, nullptr, s);
-    // the matrix-core decode batch finds each expert's tokens itself
+    // the matrix-core decode batches find each expert's tokens themselves
     // (the matrix-core plan lists its groups itself: no active list)
-    if (!rc && !mdec) rc = vh_dispatch(idx, P, E, ws.counts, ws.offs, ws.perm, mfma ? nullptr : ws.active, s);
+    if (!rc && !mdec && !q8dec) rc = vh_dispatch(idx, P, E, ws.counts, ws.offs, ws.perm, mfma ? nullptr : ws.active, s);
     if (!rc && flags_out)
         rc = vh_check(hipMemcpyAsync(flags_out, ws.flags, size_t(n_tokens) * 4, hipMemcpyDeviceToDevice, s));
     if (mfma) {  // every group on the matrix cores
@@ -820,6 +835,12 @@ int ffn_forward(const vireo_moe_model *m, int layer, float *x, const float *hb, 
                                      n_tokens, d, fe, k, E, slots, n_tokens, ws.h, s, &sf);
         if (!rc) rc = vh_mdec_down(ws.counts, ws.offs, ws.perm, ws.active, tb, pt != nullptr, ws.h, d, fe, E, slots,
                                    n_tokens, ws.ybuf, s, &sf);
+    } else if (q8dec) {
+        if (!rc && !prepped) rc = vh_mdec_prep(hb, n_tokens, d, ws.xp, ws.xsc, s, true);
+        // the prefill GEMMs' fragment copy where the layer has it or can make it
+        const void *const *pt = rc ? nullptr : packed_table(m, layer, table, !src, s, 1);
+        const MdecSelf sf{idx, w, x, ws.ctr, vh_mdec_ctr_words(d), n_tokens, k};
+        if (!rc) rc = vh_q8dec(pt ? pt : table, pt != nullptr, ws.xp, ws.xsc, d, fe, E, ws.h, ws.hsc, ws.ybuf, sf, s);
     } else if (n_tokens < kMfmaMinCall && vh_gdec_supported(tg, td, d, fe, hb)) {
         // calls of a decode batch's size (a few tokens per group): inputs in registers
         if (!rc) rc = vh_gdec_gateup(tg, ws.counts, ws.offs, ws.perm, ws.active, table, hb, d, fe, k, E, slots, n_tokens, ws.h, s);
@@ -828,7 +849,7 @@ int ffn_forward(const vireo_moe_model *m, int layer, float *x, const float *hb, 
         if (!rc) rc = vh_grouped_gateup(tg, ws.counts, ws.offs, ws.perm, ws.active, table, hb, d, fe, k, E, slots, ws.h, s);
         if (!rc) rc = vh_grouped_down(td, ws.counts, ws.offs, ws.perm, ws.active, table, ws.h, d, fe, E, slots, ws.ybuf, s);
     }
-    if (!rc && !mdec) rc = vh_combine(idx, w, table, ws.ybuf, d, k, n_tokens, x, s);
+    if (!rc && !mdec && !q8dec) rc = vh_combine(idx, w, table, ws.ybuf, d, k, n_tokens, x, s);
     if (!rc && !src) rc = vh_store_note_routing(m->es, layer, idx, n_tokens, k, s);
     return vh_finish(s, rc);
 }

@@ -55,6 +55,7 @@
 #include <hip/hip_runtime.h>
 #include <vector>
 #include "common.h"
+#include "expert_group.h"
 #include "qdecode.h"
 #include "route.h"
 #include "route_kernels.h"
@@ -69,40 +70,6 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int kTok = 16;  // tokens per tile (the A operand's rows)
 constexpr int kDnTok = 8;  // tokens per down tile: its LDS holds their activations, and few experts of a
                            // decode call serve more (the MFMA rows past them are idle either way)
-constexpr int kGroupMax = 64;     // a call's tokens per expert (at most one pair per token; calls < 64 tokens)
-
-// The pairs p < P routed to expert e (idx[p] == e) in ascending order into
-// list (at most kGroupMax kept); returns their number. Called by every thread
-// of a workgroup of NT threads; the first two rounds' loads are issued
-// together, and the function ends with a barrier.
-template <int NT>
-VH_DEV int expert_group(const int32_t *__restrict__ idx, int P, int e, int *list, int *wc) {
-    constexpr int NW = NT / 64;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int v0 = tid < P ? idx[tid] : -1, v1 = tid + NT < P ? idx[tid + NT] : -1;
-    int base = 0;
-    for (int p0 = 0; p0 < P; p0 += NT) {
-        const int p = p0 + tid;
-        const int v = p0 == 0 ? v0 : p0 == NT ? v1 : (p < P ? idx[p] : -1);
-        const bool hit = v == e;
-        const uint64_t m = __ballot(hit);
-        if (lane == 0) wc[wv] = __popcll(m);
-        __syncthreads();
-        int before = base, tot = base;
-#pragma unroll
-        for (int w = 0; w < NW; w++) {
-            const int c = wc[w];
-            before += w < wv ? c : 0;
-            tot += c;
-        }
-        const int at = before + __popcll(m & ((1ull << lane) - 1ull));
-        if (hit && at < kGroupMax) list[at] = p;
-        base = tot;
-        __syncthreads();  // wc is written again by the next round
-    }
-    return min(base, kGroupMax);
-}
-
 VH_DEV f16x2 as_h2(uint32_t v) { return __builtin_bit_cast(f16x2, v); }
 VH_DEV uint32_t u4_at(const uint4 &v, int i) { return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w; }
 
@@ -171,6 +138,9 @@ VH_DEV int q6k_slot_of(int k) {
 // X_s of the scaled inputs over each 32-input sub-block, X_s / 32 split into
 // fp16 hi + lo at xsum + ((t * nb + b) * 4 + g) * 4: hi, lo of sub-block 2 g,
 // then of 2 g + 1 (the slots lane group g supplies to the min term).
+// NAT (the Q8_0 decode batch, moe_q8dec.hip): chunk c of a super-block holds
+// inputs 8 c .. 8 c + 7 in order, and there are no sums.
+template <bool NAT>
 __global__ void __launch_bounds__(256) mdec_prep_kernel(const float *__restrict__ hb, int d,
                                                         _Float16 *__restrict__ xp, float *__restrict__ xsc,
                                                         _Float16 *__restrict__ xsum) {
@@ -189,8 +159,8 @@ __global__ void __launch_bounds__(256) mdec_prep_kernel(const float *__restrict_
     const float up = ldexpf(1.0f, sh);
     if (tid == 0) xsc[t] = ldexpf(1.0f, -sh);
     _Float16 *o = xp + size_t(t) * d * 2;
-    int chunk;
-    const int j = q4k_slot_of(tid, chunk);
+    int chunk = tid >> 3;
+    const int j = NAT ? tid & 7 : q4k_slot_of(tid, chunk);
     for (int b = 0; b < nb; b++) {  // d % 256 == 0: every thread takes every step
         const float v = x[256 * b + tid] * up;
         const _Float16 hi = _Float16(v);
@@ -198,6 +168,7 @@ __global__ void __launch_bounds__(256) mdec_prep_kernel(const float *__restrict_
         const size_t c = (size_t(b) * 32 + chunk) * 16;
         o[c + j] = hi;
         o[c + 8 + j] = lo;
+        if (NAT) continue;
         float sv = v;  // sub-block tid / 32: lanes 32 s .. 32 s + 31 of the workgroup
 #pragma unroll
         for (int off = 16; off > 0; off >>= 1) sv += __shfl_xor(sv, off, 32);
@@ -223,6 +194,7 @@ __global__ void __launch_bounds__(256) mdec_prep_kernel(const float *__restrict_
 // sub-block l % 8 of super-block l / 8; its sum is taken in order in the lane).
 constexpr int kRpTile = 4, kRpLaneF = 36;  // 32 inputs per lane in LDS, plus 4 floats (no bank conflicts)
 
+template <bool NAT>
 __global__ void __launch_bounds__(256) mdec_route_prep_kernel(const float *__restrict__ R, const float *__restrict__ hb,
                                                               const float *__restrict__ bias, int E, int T,
                                                               RoutePart *__restrict__ parts, _Float16 *__restrict__ xp,
@@ -279,15 +251,23 @@ __global__ void __launch_bounds__(256) mdec_route_prep_kernel(const float *__res
             }
             // slots 4 hs .. 4 hs + 3 of chunk (b, u, g) hold positions 0, 2, 1, 3
             typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
-            f16x4 *c = reinterpret_cast<f16x4 *>(o + (size_t(b) * 32 + u * 4 + g) * 16 + 4 * hs);
-            c[0] = f16x4{hi[0], hi[2], hi[1], hi[3]};
-            c[2] = f16x4{lo[0], lo[2], lo[1], lo[3]};
+            if constexpr (NAT) {
+                f16x4 *c = reinterpret_cast<f16x4 *>(o + (size_t(b) * 32 + 4 * (lane & 7) + (u >> 1)) * 16 + 4 * (u & 1));
+                c[0] = f16x4{hi[0], hi[1], hi[2], hi[3]};
+                c[2] = f16x4{lo[0], lo[1], lo[2], lo[3]};
+            } else {
+                f16x4 *c = reinterpret_cast<f16x4 *>(o + (size_t(b) * 32 + u * 4 + g) * 16 + 4 * hs);
+                c[0] = f16x4{hi[0], hi[2], hi[1], hi[3]};
+                c[2] = f16x4{lo[0], lo[2], lo[1], lo[3]};
+            }
         }
-        const float q = sum * 0.03125f;  // |X_s| < 2^19
-        const _Float16 qh = _Float16(q);
-        _Float16 *xsp = xsum + ((size_t(t) * nb + b) * 4 + g) * 4 + 2 * hs;
-        xsp[0] = qh;
-        xsp[1] = _Float16(q - float(qh));
+        if constexpr (!NAT) {
+            const float q = sum * 0.03125f;  // |X_s| < 2^19
+            const _Float16 qh = _Float16(q);
+            _Float16 *xsp = xsum + ((size_t(t) * nb + b) * 4 + g) * 4 + 2 * hs;
+            xsp[0] = qh;
+            xsp[1] = _Float16(q - float(qh));
+        }
     }
     __syncthreads();
     if (e >= E) return;
@@ -861,20 +841,21 @@ bool vh_mdec_supported(uint32_t tg, uint32_t td, int d, int fe) {
 }
 
 int vh_route_parts_tiled(const float *R, const float *hb, const float *bias, int d, int E, int T, RoutePart *parts,
-                         void *xp, float *xsc, hipStream_t s) {
+                         void *xp, float *xsc, hipStream_t s, bool natural) {
     if (d != 2048 || T < 2 || E < 1 || ((reinterpret_cast<uintptr_t>(R) | reinterpret_cast<uintptr_t>(hb)) & 15u))
         return -EINVAL;
     const dim3 g((E + kRpTile - 1) / kRpTile, (T + kRpTile - 1) / kRpTile);
-    hipLaunchKernelGGL(mdec_route_prep_kernel, g, dim3(256), 0, s, R, hb, bias, E, T, parts,
-                       static_cast<_Float16 *>(xp), xsc,
-                       xp ? static_cast<_Float16 *>(vh_mdec_xsum(xp, T, d)) : nullptr);
+    _Float16 *x = static_cast<_Float16 *>(xp), *xsum = xp ? static_cast<_Float16 *>(vh_mdec_xsum(xp, T, d)) : nullptr;
+    if (natural) hipLaunchKernelGGL(mdec_route_prep_kernel<true>, g, dim3(256), 0, s, R, hb, bias, E, T, parts, x, xsc, xsum);
+    else hipLaunchKernelGGL(mdec_route_prep_kernel<false>, g, dim3(256), 0, s, R, hb, bias, E, T, parts, x, xsc, xsum);
     return vh_check(hipGetLastError());
 }
 
-int vh_mdec_prep(const float *hb, int T, int d, void *xp, float *xsc, hipStream_t s) {
+int vh_mdec_prep(const float *hb, int T, int d, void *xp, float *xsc, hipStream_t s, bool natural) {
     if (T < 1 || d % 256) return -EINVAL;
-    hipLaunchKernelGGL(mdec_prep_kernel, dim3(T), dim3(256), 0, s, hb, d, static_cast<_Float16 *>(xp), xsc,
-                       static_cast<_Float16 *>(vh_mdec_xsum(xp, T, d)));
+    _Float16 *x = static_cast<_Float16 *>(xp), *xsum = static_cast<_Float16 *>(vh_mdec_xsum(xp, T, d));
+    if (natural) hipLaunchKernelGGL(mdec_prep_kernel<true>, dim3(T), dim3(256), 0, s, hb, d, x, xsc, xsum);
+    else hipLaunchKernelGGL(mdec_prep_kernel<false>, dim3(T), dim3(256), 0, s, hb, d, x, xsc, xsum);
     return vh_check(hipGetLastError());
 }
 

@@ -1,0 +1,363 @@
+// Decode-batch projections of Q8_0 experts on the matrix cores, for calls of
+// kQ8decMinTokens to kMfmaMinCall - 1 tokens. The fp32 kernels (moe_gdec.hip)
+// convert and multiply every weight again for each token of its expert and are
+// bound by the vector ALUs (23 OLMoE tokens: 104 + 54 us per layer, where reading
+// the experts takes 80); here a weight becomes a matrix operand once for up to 32
+// tokens: 56 + 45 us, gate/up at 4.8 TB/s, down at 3 (its arrivals and the combine
+// are a tail of round trips).
+//
+// v_mfma_f32_16x16x32_f16: 16 tokens x 16 weight rows x one block of 32 weights.
+// The operand holds the quants themselves (exact in fp16) and each block's sum
+// is scaled by its d in fp32 (src/gguf_compute.c:112-120, the sums of :127-157).
+// Inputs are split into fp16 parts hi + lo (22 significant bits, under a power
+// of two per token: mdec_prep_kernel, natural order), one multiply each; the
+// activations h the same way under a power of two per (pair, 32 columns), which
+// enters the block's scale in the down projection. Products are exact in fp32, so
+// the results differ from the fp32 kernels' by the order of the sums and 2^-23 of
+// the inputs: 7.6e-8 of the output against 64 bits at 23 OLMoE tokens, as before.
+//
+// A wave owns two 32-row fragments (gate/up: 32 rows of gate and the same of
+// up; down: 64 rows) of the layout of mfma_frag.h - the copy the prefill GEMMs
+// read, or the GGUF rows: the same words, the same bits - whose lanes hold a
+// whole block of their row each. Four lane groups of 16 thus hold the blocks of
+// four (16 rows, block) operands, and a 4 x 4 transposition of 8-byte chunks over
+// the groups (eight v_permlane swaps) gives every group its quarter of each.
+//
+// Grid (128 columns of h, or 256 rows of down; expert), four waves; the
+// workgroup lists its expert's tokens itself (expert_group.h). The last of a
+// token's k experts to write a workgroup's rows adds them into x in selection
+// order, as mdec_down_kernel (moe_mdec.hip) does.
+#include <hip/hip_runtime.h>
+#include "common.h"
+#include "expert_group.h"
+#include "mfma_frag.h"
+#include "route.h"
+#include "route_kernels.h"
+
+namespace {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+constexpr int kTok = 16;                  // tokens per matrix tile; NT of them per pass over the weights
+
+struct Q8Lds {
+    int list[kGroupMax], wc[4], last[kGroupMax + 1];
+};
+
+VH_DEV void swap32(uint32_t &a, uint32_t &b) {  // a's upper 32 lanes with b's lower
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+}
+VH_DEV void swap16(uint32_t &a, uint32_t &b) {  // a's odd rows of 16 lanes with b's even ones
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+}
+
+// eight bytes q + 128 as fp16 q
+VH_DEV f16x8 q8_operand(uint32_t w0, uint32_t w1, uint32_t kb) {
+    f16x8 o;
+#pragma unroll
+    for (int p = 0; p < 4; p++) {
+        const uint32_t v = __builtin_amdgcn_perm(p < 2 ? w0 : w1, kb, (p & 1) ? 0x00070006u : 0x00050004u);
+        const f16x2 y = as_h2(v) - splat(_Float16(1152.0f));
+        o[2 * p] = y[0];
+        o[2 * p + 1] = y[1];
+    }
+    return o;
+}
+
+// acc[j][h][n]: rows 16 h .. + 15 of fragment j times the tokens 16 n .. of the
+// pass (lane l: row l % 16, tokens 4 (l / 16) .. + 3). A row of x is K x 4 bytes
+// (chunks of 8 inputs: hi parts, then lo); row_of(i) is the pass's token i's.
+// hs (down): the scales of h per row and block. Nothing passes through LDS: a
+// wave reads its inputs' operands itself, with its weights (the other waves'
+// reads of the same lines hit the L1), so no barrier ties its stream to theirs
+// (inputs staged for the workgroup: gate/up 75 us at 23 OLMoE tokens).
+template <bool PK, bool DOWN, int NT, class RowOf>
+VH_DEV void q8_stream(gbyte *F, gbyte *R0, gbyte *R1, const void *x, const float *hs, int K, int tn, RowOf row_of,
+                      f32x4 (&acc)[2][2][NT]) {
+    constexpr int SETS = NT == 1 ? 4 : 2;  // K steps in flight
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4, half = lane >> 5, nk = K / kBK;
+    uint32_t kb = 0x64646464u;
+    asm volatile("" : "+v"(kb));
+    gbyte *xr[NT], *sr[NT][4];
+#pragma unroll
+    for (int n = 0; n < NT; n++) {
+        xr[n] = gmem(x) + size_t(row_of(min(16 * n + r, tn - 1))) * K * 4 + 32 * g;
+        if constexpr (DOWN)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                sr[n][i] = gmem(hs) + size_t(row_of(min(16 * n + 4 * g + i, tn - 1))) * (K / 32) * 4;
+    }
+    struct Set {
+        uint32_t w[2][8], d[2];
+        uint4 xh[2][NT], xl[2][NT];
+        uint2 sc[DOWN ? NT : 1][4];
+    } st[SETS];
+    auto load = [&](Set &q, int s) {
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            if constexpr (PK) {
+                Frag<VT_Q8_0>::load(F + (size_t(s) * 2 + j) * Frag<VT_Q8_0>::bytes, lane, q.w[j], q.d[j]);
+            } else {
+                Rows<VT_Q8_0>::Raw w;
+                Rows<VT_Q8_0>::load(j ? R1 : R0, s, half, w);
+#pragma unroll
+                for (int i = 0; i < 8; i++) q.w[j][i] = u4_at(w.q[i >> 2], i & 3);
+                q.d[j] = w.d;
+            }
+        }
+#pragma unroll
+        for (int n = 0; n < NT; n++) {
+#pragma unroll
+            for (int k = 0; k < 2; k++) {  // block k of the step: chunk 4 k + g
+                q.xh[k][n] = ld_u128(xr[n] + 256 * s + 128 * k);
+                q.xl[k][n] = ld_u128(xr[n] + 256 * s + 128 * k + 16);
+            }
+            if constexpr (DOWN)
+#pragma unroll
+                for (int i = 0; i < 4; i++) q.sc[n][i] = ld_u64(sr[n][i] + 8 * s);
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < SETS; i++) load(st[i], min(i, nk - 1));
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int n = 0; n < NT; n++) acc[j][h][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto step = [&](int s, Set &t) {
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            uint32_t q[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) q[i] = PK ? t.w[j][i] : t.w[j][i] ^ 0x80808080u;
+            swap32(q[0], q[4]);
+            swap32(q[1], q[5]);
+            swap32(q[2], q[6]);
+            swap32(q[3], q[7]);
+            swap16(q[0], q[2]);
+            swap16(q[1], q[3]);
+            swap16(q[4], q[6]);
+            swap16(q[5], q[7]);
+            uint32_t d0 = t.d[j], d2 = t.d[j];
+            swap32(d0, d2);
+            uint32_t d1 = d0, d3 = d2;
+            swap16(d0, d1);
+            swap16(d2, d3);
+            const float d[4] = {h2f(d0), h2f(d1), h2f(d2), h2f(d3)};
+            // operand m: rows 16 (m % 2) .. of the fragment, block m / 2 of the step
+#pragma unroll
+            for (int m = 0; m < 4; m++) {
+                const f16x8 o = q8_operand(q[2 * m], q[2 * m + 1], kb);
+#pragma unroll
+                for (int n = 0; n < NT; n++) {
+                    f32x4 c = {0.f, 0.f, 0.f, 0.f};
+                    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, t.xh[m >> 1][n]), o, c, 0, 0, 0);
+                    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, t.xl[m >> 1][n]), o, c, 0, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const float f = DOWN ? d[m] * __uint_as_float(m >> 1 ? t.sc[DOWN ? n : 0][i].y : t.sc[DOWN ? n : 0][i].x) : d[m];
+                        acc[j][m & 1][n][i] = fmaf(f, c[i], acc[j][m & 1][n][i]);
+                    }
+                    // added here: left for later, every block's products would be held in registers
+                    asm volatile("" : "+v"(acc[j][m & 1][n]));
+                }
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        load(t, min(s + SETS, nk - 1));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    for (int s = 0; s < nk; s += 4) {  // nk is even
+        step(s, st[0]);
+        step(s + 1, st[1]);
+        if (s + 2 < nk) {
+            step(s + 2, st[SETS == 4 ? 2 : 0]);
+            step(s + 3, st[SETS == 4 ? 3 : 1]);
+        }
+    }
+}
+
+struct Q8Args {
+    const void *const *table;
+    const void *x;        // gate/up: the split inputs [T]; down: the split activations [pairs]
+    const float *xsc;     // gate/up: the tokens' scales
+    uint16_t *hp;         // gate/up: the activations [pairs x fe x 2]
+    float *hs;            // and their block scales [pairs x fe / 32]
+    float *y;             // down: [pairs x d]
+    int d, fe;
+    MdecSelf sf;
+};
+
+// the largest of v over the 16 lanes of a row of lanes
+VH_DEV float row_max(float v) {
+    v = fmaxf(v, dpp_keep<0xB1>(v));
+    v = fmaxf(v, dpp_keep<0x4E>(v));
+    v = fmaxf(v, dpp_keep<0x141>(v));
+    return fmaxf(v, dpp_keep<0x140>(v));
+}
+
+template <bool PK, int NT>
+VH_DEV void gateup_pass(const Q8Lds &L, const Q8Args &a, gbyte *G, gbyte *U, int c, int t0, int tn) {
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4, col = lane & 31, nk = a.d / kBK;
+    const int64_t rb = int64_t(a.d / 32) * 34;
+    gbyte *row = G + int64_t(32 * c + col) * rb, *row1 = U + int64_t(32 * c + col) * rb;
+    f32x4 acc[2][2][NT];
+    q8_stream<PK, false, NT>(G + size_t(c) * nk * 2 * Frag<VT_Q8_0>::bytes, row, row1, a.x, nullptr, a.d, tn,
+                             [&](int i) { return L.list[t0 + i] / a.sf.k; }, acc);
+    float rs[2][2] = {{1.0f, 1.0f}, {1.0f, 1.0f}};  // the rows' powers of two in the packed copy
+    if constexpr (PK) {
+        gbyte *p = G + size_t(2) * a.fe / 32 * nk * Frag<VT_Q8_0>::bytes;
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) rs[j][h] = __uint_as_float(ld_u32(p + 4 * (j * a.fe + 32 * c + 16 * h + r)));
+    }
+#pragma unroll
+    for (int n = 0; n < NT; n++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int tt = 16 * n + 4 * g + i, pair = L.list[t0 + min(tt, tn - 1)];
+            const float sc = a.xsc[pair / a.sf.k];
+            float h[2];
+#pragma unroll
+            for (int x = 0; x < 2; x++)
+                h[x] = swiglu(acc[0][x][n][i] * rs[0][x] * sc, acc[1][x][n][i] * rs[1][x] * sc);
+            // the block's power of two: |h| < 2^e, kept as h 2^(14 - e) in fp16 parts
+            const uint32_t m = __float_as_uint(row_max(fmaxf(fabsf(h[0]), fabsf(h[1]))));
+            const int e = m ? max(-100, min(127, int(m >> 23) - 126)) : 0;
+            if (tt >= tn) continue;
+            const float up = __uint_as_float(uint32_t(127 + 14 - e) << 23);
+            if (r == 0) a.hs[size_t(pair) * (a.fe / 32) + c] = ldexpf(1.0f, e - 14);
+#pragma unroll
+            for (int x = 0; x < 2; x++) {
+                const int o = 32 * c + 16 * x + r;
+                const float v = h[x] * up;
+                const _Float16 hi = _Float16(v);
+                uint16_t *p = a.hp + size_t(pair) * a.fe * 2 + (o >> 3) * 16 + (o & 7);
+                p[0] = __builtin_bit_cast(uint16_t, hi);
+                p[8] = __builtin_bit_cast(uint16_t, _Float16(v - float(hi)));
+            }
+        }
+}
+
+template <bool PK, int NT>
+__global__ void __launch_bounds__(256, 2) q8dec_gateup_kernel(Q8Args a) {
+    __shared__ Q8Lds L;
+    if (blockIdx.x == 0 && blockIdx.y == 0)  // the down kernel's counters start at 0
+        for (int i = threadIdx.x; i < a.sf.nctr; i += 256) a.sf.ctr[i] = 0u;
+    const int e = blockIdx.y, cnt = expert_group<256>(a.sf.idx, a.sf.T * a.sf.k, e, L.list, L.wc);
+    if (cnt == 0) return;
+    gbyte *G = gmem(a.table[3 * e]), *U = gmem(a.table[3 * e + 1]);
+    if (!G || !U) return;  // an unregistered expert: the down kernel writes zeros (src/gguf_run.c:201)
+    const int c = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (int t0 = 0; t0 < cnt; t0 += NT * kTok) gateup_pass<PK, NT>(L, a, G, U, c, t0, min(NT * kTok, cnt - t0));
+}
+
+template <bool PK, int NT>
+VH_DEV void down_pass(const Q8Lds &L, const Q8Args &a, gbyte *D, int c, int t0, int tn) {
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4, col = lane & 31, nk = a.fe / kBK;
+    const int64_t rb = int64_t(a.fe / 32) * 34;
+    f32x4 acc[2][2][NT];
+    if (D) {
+        q8_stream<PK, true, NT>(D + size_t(c) * nk * 2 * Frag<VT_Q8_0>::bytes, D + int64_t(64 * c + col) * rb,
+                                D + int64_t(64 * c + 32 + col) * rb, a.x, a.hs, a.fe, tn,
+                                [&](int i) { return L.list[t0 + i]; }, acc);
+    } else {  // an unregistered expert's rows are zeros, which the combine adds without changing a bit
+#pragma unroll
+        for (int x = 0; x < 4 * NT; x++) acc[x / 2 / NT][x / NT % 2][x % NT] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    gbyte *p = D + size_t(a.d) / 32 * nk * Frag<VT_Q8_0>::bytes;
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int o = 64 * c + 32 * j + 16 * h + r;
+            const float rs = PK && D ? __uint_as_float(ld_u32(p + 4 * o)) : 1.0f;
+#pragma unroll
+            for (int n = 0; n < NT; n++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const int tt = 16 * n + 4 * g + i;
+                    if (tt < tn)
+                        __hip_atomic_store(&a.y[size_t(L.list[t0 + tt]) * a.d + o], acc[j][h][n][i] * rs,
+                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+        }
+}
+
+template <bool PK, int NT>
+__global__ void __launch_bounds__(256, 2) q8dec_down_kernel(Q8Args a) {
+    __shared__ Q8Lds L;
+    constexpr int CR = 256;  // output rows of one workgroup
+    const MdecSelf &sf = a.sf;
+    const int tid = threadIdx.x, e = blockIdx.y, k = sf.k, d = a.d;
+    const int cnt = expert_group<256>(sf.idx, sf.T * k, e, L.list, L.wc);
+    if (cnt == 0) return;
+    gbyte *D = gmem(a.table[3 * e + 2]);
+    const int c = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(tid >> 6);
+    for (int t0 = 0; t0 < cnt; t0 += NT * kTok) down_pass<PK, NT>(L, a, D, c, t0, min(NT * kTok, cnt - t0));
+    // the combine (src/gguf_run.c:208-212; see mdec_down_kernel): rows out as
+    // agent-scope stores, one arrival per token once they are done, and the
+    // workgroup that brings a token's count to k reads its k rows past the L2
+    if (tid == 0) L.last[kGroupMax] = 0;
+    VH_WAIT_VMCNT(0);
+    __syncthreads();
+    if (tid < cnt) {
+        const int t = L.list[tid] / k;
+        const uint32_t n = __hip_atomic_fetch_add(&sf.ctr[blockIdx.x * kGroupMax + t], 1u, __ATOMIC_RELAXED,
+                                                  __HIP_MEMORY_SCOPE_AGENT);
+        if (n == uint32_t(k - 1)) L.last[atomicAdd(&L.last[kGroupMax], 1)] = t;
+    }
+    __syncthreads();
+    const int nl = L.last[kGroupMax], o = blockIdx.x * CR + tid;
+    constexpr int KB = 8;  // rows of y in flight per thread and token
+    for (int i = 0; i < nl; i++) {
+        const int t = L.last[i];
+        float s = 0.0f;
+        const float xo = sf.x[size_t(t) * d + o];
+        for (int j0 = 0; j0 < k; j0 += KB) {
+            float yv[KB];
+#pragma unroll
+            for (int j = 0; j < KB; j++)
+                yv[j] = __hip_atomic_load(&a.y[(size_t(t) * k + min(j0 + j, k - 1)) * d + o], __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for (int j = 0; j < KB; j++)
+                if (j0 + j < k) s = add_rn(s, mul_rn(sf.w[size_t(t) * k + j0 + j], yv[j]));
+        }
+        sf.x[size_t(t) * d + o] = add_rn(xo, s);
+    }
+}
+
+template <int NT>
+void q8dec_launch(Q8Args a, bool packed, int E, const void *hp, hipStream_t s) {
+    const dim3 gg(a.fe / 128, E), gd(a.d / 256, E), b(256);
+    if (packed) hipLaunchKernelGGL((q8dec_gateup_kernel<true, NT>), gg, b, 0, s, a);
+    else hipLaunchKernelGGL((q8dec_gateup_kernel<false, NT>), gg, b, 0, s, a);
+    a.x = hp;
+    if (packed) hipLaunchKernelGGL((q8dec_down_kernel<true, NT>), gd, b, 0, s, a);
+    else hipLaunchKernelGGL((q8dec_down_kernel<false, NT>), gd, b, 0, s, a);
+}
+
+}  // namespace
+
+bool vh_q8dec_supported(uint32_t tg, uint32_t td, int d, int fe, int T) {
+    return tg == VT_Q8_0 && td == VT_Q8_0 && d % 256 == 0 && fe % 128 == 0 && T <= kGroupMax;
+}
+
+int vh_q8dec(const void *const *table, bool packed, const void *xp, const float *xsc, int d, int fe, int E, void *hp,
+             float *hs, float *ybuf, const MdecSelf &self, hipStream_t s) {
+    if (!vh_q8dec_supported(VT_Q8_0, VT_Q8_0, d, fe, self.T) || self.T < 1 || self.k < 1 || !self.x || !self.w ||
+        self.nctr < vh_mdec_ctr_words(d))
+        return -EINVAL;
+    const Q8Args a{table, xp, xsc, static_cast<uint16_t *>(hp), hs, ybuf, d, fe, self};
+    // two token tiles per pass where the average expert has more than half a tile (its registers keep two waves
+    // per SIMD, one tile's four)
+    if (2 * self.T * self.k > kTok * E) q8dec_launch<2>(a, packed, E, hp, s);
+    else q8dec_launch<1>(a, packed, E, hp, s);
+    return vh_check(hipGetLastError());
+}

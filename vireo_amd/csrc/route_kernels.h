@@ -148,8 +148,8 @@ bool vh_mdec_supported(uint32_t tg, uint32_t td, int d, int fe);
 // bounded parts) by 4 x 4 tiles of (expert, token), d == 2048 and 16-byte
 // aligned R and hb, else -EINVAL; with xp given, also vh_mdec_prep's outputs.
 int vh_route_parts_tiled(const float *R, const float *hb, const float *bias, int d, int E, int T, RoutePart *parts,
-                         void *xp, float *xsc, hipStream_t s);
-int vh_mdec_prep(const float *hb, int T, int d, void *xp, float *xsc, hipStream_t s);
+                         void *xp, float *xsc, hipStream_t s, bool natural = false);
+int vh_mdec_prep(const float *hb, int T, int d, void *xp, float *xsc, hipStream_t s, bool natural = false);
 // A decode-batch call whose matrix-core kernels find each expert's pairs in
 // the routing themselves (no dispatch: workgroup column e takes expert e)
 // and whose down kernel also combines into x in selection order (no combine
@@ -180,6 +180,15 @@ int vh_mdec_down(const int32_t *counts, const int32_t *offs, const int32_t *perm
 // synchronizing read of the table; -EBUSY while s is being captured.
 uint64_t vh_mdec_pack_bytes(int E, int d, int fe);
 int vh_mdec_pack_layer(const void *const *table, int E, int d, int fe, void *buf, void **tab_out, hipStream_t s);
+
+// The decode batch of Q8_0 experts on the matrix cores (moe_q8dec.hip): gate/up,
+// down and the combine of the call `self` routes, T <= 64. xp, xsc: vh_mdec_prep's
+// split inputs in natural order (`natural` there and in vh_route_parts_tiled);
+// hp [pairs x fe x 4 bytes] and hs [pairs x fe / 32] take the activations.
+// `packed`: table points at vh_mfma_pack's fragments (the same bits either way).
+bool vh_q8dec_supported(uint32_t tg, uint32_t td, int d, int fe, int T);
+int vh_q8dec(const void *const *table, bool packed, const void *xp, const float *xsc, int d, int fe, int E, void *hp,
+             float *hs, float *ybuf, const MdecSelf &self, hipStream_t s);
 
 // Matrix-core grouped GEMMs (moe_mfma.hip) for the groups of calls of at
 // least kMfmaMinCall tokens. vh_mfma_plan lists the groups' token tiles (32,
