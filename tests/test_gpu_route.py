@@ -109,13 +109,14 @@ def test_route_zipf_bias(cuda, oracle):
 
 @pytest.mark.parametrize("T,k,E,skew", [(1, 8, 128, 0), (7, 8, 64, 0), (2048, 8, 128, 0), (300, 1, 256, 0),
                                          (33, 4, 8, 0), (256, 8, 64, 0), (257, 8, 64, 0), (4096, 8, 128, 1.1),
-                                         (1000, 3, 256, 1.1), (1001, 3, 256, 0), (16500, 8, 128, 1.1)])
+                                         (1000, 3, 256, 1.1), (1001, 3, 256, 0), (16500, 8, 128, 1.1),
+                                         (48, 8, 128, 0), (97, 4, 64, 0), (129, 3, 128, 0)])
 def test_dispatch_is_a_stable_sort(cuda, T, k, E, skew):
-    """One-workgroup form up to 2048 pairs (256 x 8 and 257 x 8 straddle the
-    switch); above, one launch with a workgroup per expert when the pair
-    count is a multiple of 4 and at most 131072 (2048 x 8, 4096 x 8,
-    1000 x 3), else the two-kernel form (1001 x 3, 16500 x 8); skew draws
-    experts with Zipf weights."""
+    """Above 384 pairs (48 x 8 and 97 x 4 straddle the switch) one launch with
+    a workgroup per expert when the pair count is a multiple of 4 and at most
+    131072 (256 x 8, 2048 x 8, 4096 x 8, 1000 x 3); else the one-workgroup form
+    up to 2048 pairs (33 x 4, 129 x 3) and the two-kernel form above (1001 x 3,
+    16500 x 8); skew draws experts with Zipf weights."""
     rng = np.random.default_rng(T * k + E)
     p = None
     if skew:
@@ -164,3 +165,26 @@ def test_router_logits_exact(cuda, oracle, lib, case):
     if case == "subnormal":
         assert np.count_nonzero(np.abs(want) < 1.1754944e-38) > 0
     np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("T,E,k,d", [(64, 7, 2, 128), (65, 7, 2, 160), (101, 128, 8, 2048), (512, 128, 8, 192),
+                                     (70, 9, 3, 320), (64, 256, 8, 256)])
+def test_few_tokens_sum_as_many(cuda, oracle, T, E, k, d):
+    """The exact router of calls of 64 tokens on that give at most 1024 waves of one
+    chain (512 x 128 is the last) takes one chain per lane, larger calls two: the
+    same in-order sums bit for bit, also where d is no multiple of the 64-column
+    chunk and where tokens (65, 70, 101) and experts (7, 9) end inside a workgroup."""
+    shape = W.MoEShape("few", d, E, k, 256, True, W.Q8_0, W.Q8_0, W.Q8_0)
+    bias = np.linspace(0.0, 0.5, E).astype(np.float32)
+    m = M.DeviceMoE(shape, 1, seed=57, logit_bias=bias)
+    _, hb = W.host_hidden(d, T, 57)
+    big = np.tile(hb, (64 * (1024 // E + 1) // T + 1, 1))
+    idx, w, _, probs = m.route(0, torch.from_numpy(hb).to(cuda), want_probs=True)
+    bi, bw, _, bp = m.route(0, torch.from_numpy(big).to(cuda), want_probs=True)
+    for few, many in ((idx, bi), (w, bw), (probs, bp)):
+        np.testing.assert_array_equal(few.cpu().numpy(), many[:T].cpu().numpy())
+        np.testing.assert_array_equal(few.cpu().numpy(), many[T * (len(big) // T - 1):].cpu().numpy()[:T])
+    oi, ow, _ = oracle_route(oracle, shape, m.host_router(0), hb, bias)
+    np.testing.assert_array_equal(idx.cpu().numpy(), oi)
+    np.testing.assert_allclose(w.cpu().numpy(), ow, rtol=1e-5)
+    m.close()

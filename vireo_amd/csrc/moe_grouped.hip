@@ -19,9 +19,12 @@
 namespace {
 
 constexpr int kDispWaves = 16;
-// up to this many pairs one workgroup dispatches (one launch, shorter); above,
-// the two-kernel form with a workgroup per expert
-constexpr int kDispatchOneBlock = 2048;
+// above this many pairs dispatch_fused_kernel's workgroup per expert, where it
+// takes the call; else up to kDispatchOneBlock pairs one workgroup dispatches
+// (one launch, shorter), above, the two-kernel form with a workgroup per expert.
+// Measured (128 experts, one workgroup / fused): 256 pairs 6.0 / 7.6 us, 512 8.6 /
+// 7.6, 1024 13.6 / 7.4, 2048 23.2 / 7.6.
+constexpr int kDispatchFusedMin = 384, kDispatchOneBlock = 2048;
 
 // One workgroup of 16 waves (see moe_dispatch in include/vireo_hip.h).
 __global__ void __launch_bounds__(1024) dispatch_kernel(const int32_t *__restrict__ idx, int P, int E,
@@ -658,12 +661,12 @@ int proj_launch(const int32_t *counts, const int32_t *offs, const int32_t *perm,
 
 int vh_dispatch(const int32_t *idx, int P, int E, int32_t *counts, int32_t *offs, int32_t *perm, int32_t *active,
                 hipStream_t s) {
-    if (P <= kDispatchOneBlock) {
-        hipLaunchKernelGGL(dispatch_kernel, dim3(1), dim3(1024), 0, s, idx, P, E, counts, offs, perm, active);
-    } else if (P % 4 == 0 && (reinterpret_cast<uintptr_t>(idx) & 15u) == 0 && P <= kFusedChunks * kFusedChunk &&
-               E <= kMaxExperts) {
+    if (P > kDispatchFusedMin && P % 4 == 0 && (reinterpret_cast<uintptr_t>(idx) & 15u) == 0 &&
+        P <= kFusedChunks * kFusedChunk && E <= kMaxExperts) {
         hipLaunchKernelGGL(dispatch_fused_kernel, dim3(E), dim3(kFusedThreads), 0, s, idx, P, E, counts, offs, perm,
                            active);
+    } else if (P <= kDispatchOneBlock) {
+        hipLaunchKernelGGL(dispatch_kernel, dim3(1), dim3(1024), 0, s, idx, P, E, counts, offs, perm, active);
     } else {
         hipLaunchKernelGGL(dispatch_count_kernel, dim3(E), dim3(256), 0, s, idx, P, counts);
         hipLaunchKernelGGL(dispatch_place_kernel, dim3(E), dim3(256), 0, s, idx, P, E, counts, offs, perm, active);

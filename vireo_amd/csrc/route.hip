@@ -250,6 +250,108 @@ __global__ void __launch_bounds__(256) route_exact_kernel(const float *__restric
     }
 }
 
+// route_exact_kernel for few tokens (one chain per lane, W experts per
+// workgroup): lane = token t0 + lane, wave g = expert e0 + g. Where the tokens
+// give less than a wave per SIMD, a call takes as long as one wave's chains, and
+// a lane with one chain instead of two takes half as long. An add of the chain
+// goes between two products of the columns ahead, so that neither waits.
+// Two LDS buffers (rows padded by 16 bytes: conflict-free) with one barrier per
+// chunk, loaded into registers two chunks ahead, read eight columns ahead of the
+// chain. Measured (d = 2048): 101 tokens x 128 experts 33.2 -> 21.7 us, 512 x 64
+// 33.5 -> 22.8 (four experts per workgroup 23.1 and 24.0, one 24.2 and 30.9); what is
+// left is the chain's 2048 dependent adds at 22 cycles per column.
+constexpr int kExFewExp = 2;
+// Up to this many waves of one chain per lane (one per SIMD: 256 CUs x 4); above,
+// route_exact_kernel's two chains share the LDS reads of a token's inputs: 2048
+// tokens x 128 experts 83.9 us with one chain, 46.2 with two.
+constexpr int kExFewWaves = 1024;
+template <int W>
+__global__ void __launch_bounds__(64 * W) route_exact_few_kernel(const float *__restrict__ R,
+                                                                 const float *__restrict__ hb,
+                                                                 const float *__restrict__ bias, int d, int E, int T,
+                                                                 RoutePart *__restrict__ parts) {
+    typedef float vf4 __attribute__((ext_vector_type(4)));
+    constexpr int CH = kExChunk, NX = 16 / W;  // 16-byte pieces of a chunk per thread
+    __shared__ __align__(16) float xs[2][kExTok][CH + 4];
+    __shared__ __align__(16) float rs[2][W][CH];
+    const int tid = threadIdx.x, lane = tid & 63, g = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int t0 = blockIdx.x * kExTok, e0 = blockIdx.y * W;
+    // rows and columns past the end repeat the last ones; their values are never used
+    const int cc = tid & 15, r0 = tid >> 4;
+    vf4 st[2][NX], sr[2];
+    auto load = [&](auto SET, int c0) {
+        constexpr int set = decltype(SET)::value;
+        const int c = min(c0 + 4 * cc, d - 4);
+#pragma unroll
+        for (int j = 0; j < NX; j++)
+            st[set][j] = *reinterpret_cast<const vf4 *>(hb + size_t(min(t0 + r0 + 4 * W * j, T - 1)) * d + c);
+        sr[set] = *reinterpret_cast<const vf4 *>(R + size_t(min(e0 + min(r0, W - 1), E - 1)) * d + c);
+    };
+    auto store = [&](auto SET, int buf) {
+        constexpr int set = decltype(SET)::value;
+#pragma unroll
+        for (int j = 0; j < NX; j++) *reinterpret_cast<vf4 *>(&xs[buf][r0 + 4 * W * j][4 * cc]) = st[set][j];
+        if (r0 < W) *reinterpret_cast<vf4 *>(&rs[buf][r0][4 * cc]) = sr[set];
+    };
+    vf4 xg[2][2], rg[2][2];
+    auto fetch = [&](int p, int buf, int i) {  // columns 8 i .. 8 i + 7 of the buffer
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            xg[p][u] = *reinterpret_cast<const vf4 *>(&xs[buf][lane][8 * i + 4 * u]);
+            rg[p][u] = *reinterpret_cast<const vf4 *>(&rs[buf][g][8 * i + 4 * u]);
+        }
+    };
+    float acc = 0.0f, pr[8];
+    // chunk c0 in buffer BUF, its first eight products in pr; SET holds the next chunk
+    auto chunk = [&](auto SET, auto BUF, int c0) {
+        constexpr int buf = decltype(BUF)::value;
+        store(SET, buf ^ 1);
+        load(SET, c0 + 3 * CH);
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            // group i + 1 was read a step ago; group i + 2 is read now. Before the
+            // next chunk's first: its stores are done, nobody reads this buffer any more
+            const int n = i + 2;
+            if (i == 6) lds_barrier();
+            fetch(n & 1, n < 8 ? buf : buf ^ 1, n & 7);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int v = 0; v < 8; v++) {
+                acc = add_rn(acc, pr[v]);
+                asm volatile("" : "+v"(acc));
+                pr[v] = mul_rn(rg[(i + 1) & 1][v >> 2][v & 3], xg[(i + 1) & 1][v >> 2][v & 3]);
+                asm volatile("" : "+v"(pr[v]));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    const std::integral_constant<int, 0> s0;
+    const std::integral_constant<int, 1> s1;
+    load(s0, 0);
+    load(s1, CH);
+    store(s0, 0);
+    load(s0, 2 * CH);
+    lds_barrier();
+    fetch(0, 0, 0);
+    fetch(1, 0, 1);
+#pragma unroll
+    for (int v = 0; v < 8; v++) pr[v] = mul_rn(rg[0][v >> 2][v & 3], xg[0][v >> 2][v & 3]);
+    int c0 = 0;
+    for (; c0 + 2 * CH <= d; c0 += 2 * CH) {
+        chunk(s1, s0, c0);
+        chunk(s0, s1, c0 + CH);
+    }
+    int rest = 0;  // the buffer of the columns left over
+    if (c0 + CH <= d) {
+        chunk(s1, s0, c0);
+        c0 += CH;
+        rest = 1;
+    }
+    for (int i = 0; i < d - c0; i++) acc = add_rn(acc, mul_rn(rs[rest][g][i], xs[rest][lane][i]));
+    const int t = t0 + lane, e = e0 + g;
+    if (t < T && e < E) parts[size_t(t) * E + e] = RoutePart{double(bias ? add_rn(acc, bias[e]) : acc), 0.0};
+}
+
 // One workgroup per token: 512 threads for certified parts (eight waves
 // share an uncertified token's contenders), 256 for exact ones. Dynamic LDS
 // (only where route_topk_block can stream the contenders' rows: d != 2048,
@@ -335,7 +437,10 @@ int vh_route_parts(const float *R, const float *hb, const float *bias, int d, in
         dim3 g((T + kExTok - 1) / kExTok, (E + kExExp - 1) / kExExp);
         const bool v4 = d % 4 == 0 && d >= 128 &&
                         ((reinterpret_cast<uintptr_t>(R) | reinterpret_cast<uintptr_t>(hb)) & 15u) == 0;
-        if (v4)
+        if (v4 && int(g.x) * E <= kExFewWaves)
+            hipLaunchKernelGGL(route_exact_few_kernel<kExFewExp>, dim3(g.x, (E + kExFewExp - 1) / kExFewExp),
+                               dim3(64 * kExFewExp), 0, s, R, hb, bias, d, E, T, parts);
+        else if (v4)
             hipLaunchKernelGGL((route_exact_kernel<kExChunk, true>), g, dim3(256), 0, s, R, hb, bias, d, E, T, parts);
         else
             hipLaunchKernelGGL((route_exact_kernel<kExChunk, false>), g, dim3(256), 0, s, R, hb, bias, d, E, T, parts);
