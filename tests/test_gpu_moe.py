@@ -3,7 +3,7 @@ src/gguf_run.c:185-214, restated) and against the golden vectors the
 reference itself wrote, on both execution plans.
 
 Bar: the routed experts bit-exact; the layer's contribution (x_out - x)
-within 2e-3 of its largest magnitude (1e-2 where groups run as bf16
+within 2e-3 of its largest magnitude (1e-2 where groups run as fp16
 matrix-core GEMMs); the mean absolute error is printed.
 """
 import numpy as np
@@ -17,7 +17,7 @@ from vireo_amd import workloads as W
 
 pytestmark = pytest.mark.gpu
 TOL = 2e-3
-TOL_BF16 = 1e-2  # calls of >= 64 tokens: every group as bf16 GEMMs
+TOL_BF16 = 1e-2  # calls of >= 64 tokens: every group as fp16 GEMMs
 
 
 @pytest.fixture
@@ -64,7 +64,7 @@ def test_moe_ffn_matches_oracle(cuda, oracle, path, name, T, plan):
     xt = torch.from_numpy(x).to(cuda)
     idx, w = m.forward(0, xt, torch.from_numpy(hb).to(cuda), return_routing=True)
     xo, io, wo, _ = oracle_layer(oracle, m, 0, x, hb)
-    # calls of >= 64 tokens run every group as bf16 matrix-core GEMMs under plans 0 and 2
+    # calls of >= 64 tokens run every group as fp16 matrix-core GEMMs under plans 0 and 2
     tol = TOL_BF16 if T >= 64 and plan in (0, 2) else TOL
     check(f"{name} T={T} plan={plan}", x, xt.cpu().numpy(), xo, idx.cpu().numpy(), io, tol=tol)
     np.testing.assert_allclose(w.cpu().numpy(), wo, rtol=1e-5)
@@ -319,7 +319,7 @@ def test_golden_moe_on_gpu(cuda, case):
 def test_unregistered_expert_is_skipped(cuda, oracle, path, name, plan, T):
     """An expert without slices contributes nothing: the one-token plan, the
     matrix-core decode batch, whose down kernel combines (its rows of y are
-    zeros), and the bf16 GEMMs on packed Q8_0 fragments (the expert's tiles
+    zeros), and the fp16 GEMMs on packed Q8_0 fragments (the expert's tiles
     write nothing; the combine kernel skips its rows)."""
     path(plan)
     shape = W.SHAPES[name]
@@ -392,7 +392,7 @@ def test_layers_are_independent(cuda, oracle):
 def test_prefill_2048_zipf(cuda, oracle):
     """Qwen3-30B-A3B Q8_0 prefill of 2048 tokens under a Zipf(1.1) router
     bias: every token's experts bit-exact with the oracle and every token's
-    output within the bf16 matrix-core tolerance (the oracle takes a few ms
+    output within the fp16 matrix-core tolerance (the oracle takes a few ms
     per token here, a few seconds for the call)."""
     shape = W.SHAPES["qwen3-30b-a3b-q8_0"]
     bias = W.zipf_bias(shape.E, 1.1, seed=7)
@@ -434,7 +434,7 @@ MFMA_CASES = [("qwen3-30b-a3b-q8_0", 512, True), ("olmoe-q4_k_m", 128, False), (
 @pytest.mark.parametrize("plan", [0, 4])
 def test_grouped_plan_large_groups(cuda, oracle, path, name, T, zipf, plan):
     """Calls of >= 64 tokens with groups of every size (1-15 tokens, and 16 to
-    over 128): under plan 0 every group runs as bf16 matrix-core GEMMs, one
+    over 128): under plan 0 every group runs as fp16 matrix-core GEMMs, one
     tile or several, ragged or not; plan 4 runs all of them on the fp32
     kernels. Every token's experts bit-exact and every token's output
     against the oracle; the same call twice gives the same bits."""
