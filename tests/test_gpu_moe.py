@@ -500,6 +500,44 @@ def test_q8_decode_batch(cuda, oracle, E, k, d, fe, T):
     m.close()
 
 
+def layer_64(m, hb, idx, w):
+    """The MoE contribution of layer 0 in 64 bits, on the routing (idx, w) that the library chose."""
+    s, (gs, us, ds) = m.shape, m.slices
+    o = s.E * (gs + us)
+    out, h = torch.zeros(hb.shape, dtype=torch.float64, device=hb.device), hb.double()
+    for e in range(s.E):
+        t, j = (idx == e).nonzero(as_tuple=True)
+        if t.numel() == 0:
+            continue
+        g = M.dequant_rows(s.gate_type, m.buf[e * gs:(e + 1) * gs].clone(), s.d, s.fe).double()
+        u = M.dequant_rows(s.up_type, m.buf[s.E * gs + e * us:s.E * gs + (e + 1) * us].clone(), s.d, s.fe).double()
+        dn = M.dequant_rows(s.down_type, m.buf[o + e * ds:o + (e + 1) * ds].clone(), s.fe, s.d).double()
+        a = h[t] @ g.t()
+        out.index_add_(0, t, (a * torch.sigmoid(a) * (h[t] @ u.t())) @ dn.t() * w[t, j].double()[:, None])
+    return out
+
+
+@pytest.mark.parametrize("E,k,d,fe,T", [(64, 8, 2048, 1024, 16), (128, 8, 2048, 768, 63), (8, 2, 2048, 768, 40)])
+def test_q8_decode_batch_rounding(cuda, E, k, d, fe, T):
+    """The matrix-core decode batch of Q8_0 experts rounds no more than the fp32
+    kernels, whose sums lie 1.86e-7 (2-norm) from 64 bits on these layers. An fp32
+    addition's relative rounding is 2^-24 / sqrt(3) = 3.4e-8 rms of the partial sum,
+    a chain of n grows it sqrt(n / 2) times: 1.4 for the chains of 4 of gate and
+    up, 2.8 for the two levels of down and 2 for the combine, with the inputs'
+    and activations' 2^-23: 1.8e-7 together, 2.0e-7 with a tenth to spare. (8
+    experts: two token tiles per pass.)"""
+    m = M.DeviceMoE(W.MoEShape("q8round", d, E, k, fe, True, W.Q8_0, W.Q8_0, W.Q8_0), 1, seed=79)
+    _, hb = W.host_hidden(d, T, 79)
+    hbt = torch.from_numpy(hb).to(cuda)
+    x = torch.zeros((T, d), device=cuda)
+    idx, w = m.forward(0, x, hbt, return_routing=True)
+    want = layer_64(m, hbt, idx, w)
+    rel = float((x.double() - want).norm() / want.norm())
+    print(f"E={E} T={T}: {rel:.3e}")
+    assert rel <= 2.0e-7
+    m.close()
+
+
 # gate/up and down types; fe = 1152 and 1280 take more than the 32 blocks of h
 # whose factors the down GEMM holds at a time
 EDGE_TYPES = [(W.Q4_K, W.Q6_K, 512), (W.Q8_0, W.Q8_0, 1152), (W.Q6_K, W.Q4_K, 1280)]

@@ -14,7 +14,7 @@
 // activations h the same way under a power of two per (pair, 32 columns), which
 // enters the block's scale in the down projection. Products are exact in fp32, so
 // the results differ from the fp32 kernels' by the order of the sums and 2^-23 of
-// the inputs: 7.6e-8 of the output against 64 bits at 23 OLMoE tokens, as before.
+// the inputs, which are no larger than theirs (q8_stream).
 //
 // A wave owns two 32-row fragments (gate/up: 32 rows of gate and the same of
 // up; down: 64 rows) of the layout of mfma_frag.h - the copy the prefill GEMMs
@@ -37,6 +37,7 @@
 namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef double f64x4 __attribute__((ext_vector_type(4)));
 constexpr int kTok = 16;                  // tokens per matrix tile; NT of them per pass over the weights
 
 struct Q8Lds {
@@ -77,24 +78,27 @@ VH_DEV f16x8 q8_operand(uint32_t w0, uint32_t w1, uint32_t kb) {
 template <bool PK, bool DOWN, int NT, class RowOf>
 VH_DEV void q8_stream(gbyte *F, gbyte *R0, gbyte *R1, const void *x, const float *hs, int K, int tn, RowOf row_of,
                       f32x4 (&acc)[2][2][NT]) {
-    constexpr int SETS = NT == 1 ? 4 : 2;  // K steps in flight
+    constexpr int SETS = NT == 1 ? 4 : 2;  // K steps of weights in flight; of inputs (from the L2), two
     const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4, half = lane >> 5, nk = K / kBK;
     uint32_t kb = 0x64646464u;
     asm volatile("" : "+v"(kb));
-    gbyte *xr[NT], *sr[NT][4];
+    gbyte *xb = gmem(x), *sb = gmem(hs);
+    uint32_t xr[NT], sr[NT][4];  // at most 63 x 64 rows of K x 4 bytes: 32-bit offsets
 #pragma unroll
     for (int n = 0; n < NT; n++) {
-        xr[n] = gmem(x) + size_t(row_of(min(16 * n + r, tn - 1))) * K * 4 + 32 * g;
+        xr[n] = uint32_t(row_of(min(16 * n + r, tn - 1))) * uint32_t(K) * 4u + 32u * uint32_t(g);
         if constexpr (DOWN)
 #pragma unroll
             for (int i = 0; i < 4; i++)
-                sr[n][i] = gmem(hs) + size_t(row_of(min(16 * n + 4 * g + i, tn - 1))) * (K / 32) * 4;
+                sr[n][i] = uint32_t(row_of(min(16 * n + 4 * g + i, tn - 1))) * uint32_t(K / 32) * 4u;
     }
     struct Set {
         uint32_t w[2][8], d[2];
-        uint4 xh[2][NT], xl[2][NT];
-        uint2 sc[DOWN ? NT : 1][4];
     } st[SETS];
+    struct In {
+        uint4 h[2][NT], l[2][NT];
+        uint2 sc[DOWN ? NT : 1][4];
+    } in[2];
     auto load = [&](Set &q, int s) {
 #pragma unroll
         for (int j = 0; j < 2; j++) {
@@ -108,27 +112,44 @@ VH_DEV void q8_stream(gbyte *F, gbyte *R0, gbyte *R1, const void *x, const float
                 q.d[j] = w.d;
             }
         }
+    };
+    auto load_in = [&](In &q, int s) {
 #pragma unroll
         for (int n = 0; n < NT; n++) {
 #pragma unroll
             for (int k = 0; k < 2; k++) {  // block k of the step: chunk 4 k + g
-                q.xh[k][n] = ld_u128(xr[n] + 256 * s + 128 * k);
-                q.xl[k][n] = ld_u128(xr[n] + 256 * s + 128 * k + 16);
+                q.h[k][n] = ld_u128(xb + 256 * s + 128 * k + xr[n]);
+                q.l[k][n] = ld_u128(xb + 256 * s + 128 * k + 16 + xr[n]);
             }
             if constexpr (DOWN)
 #pragma unroll
-                for (int i = 0; i < 4; i++) q.sc[n][i] = ld_u64(sr[n][i] + 8 * s);
+                for (int i = 0; i < 4; i++) q.sc[n][i] = ld_u64(sb + 8 * s + sr[n][i]);
         }
     };
 #pragma unroll
     for (int i = 0; i < SETS; i++) load(st[i], min(i, nk - 1));
+#pragma unroll
+    for (int i = 0; i < 2; i++) load_in(in[i], min(i, nk - 1));
 #pragma unroll
     for (int j = 0; j < 2; j++)
 #pragma unroll
         for (int h = 0; h < 2; h++)
 #pragma unroll
             for (int n = 0; n < NT; n++) acc[j][h][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-    auto step = [&](int s, Set &t) {
+    // Gate/up adds four blocks in fp32 and these sums in fp64, down eight blocks and
+    // these sums in fp32. In one fp32 chain of all 2 nk blocks the roundings left the
+    // layer 2.9e-7 (2-norm) from 64 bits, the fp32 kernels' many short chains
+    // (moe_gdec.hip) 1.86e-7; so it is 1.80e-7 (OLMoE and Qwen3, 9 to 63 tokens), at
+    // the same speed.
+    f32x4 sub[2][2][NT];
+    f64x4 tot[2][2][DOWN ? 1 : NT];
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int n = 0; n < (DOWN ? 1 : NT); n++) tot[j][h][n] = f64x4{0., 0., 0., 0.};
+    auto step = [&](int s, Set &t, In &x, bool first) {
 #pragma unroll
         for (int j = 0; j < 2; j++) {
             uint32_t q[8];
@@ -155,30 +176,52 @@ VH_DEV void q8_stream(gbyte *F, gbyte *R0, gbyte *R1, const void *x, const float
 #pragma unroll
                 for (int n = 0; n < NT; n++) {
                     f32x4 c = {0.f, 0.f, 0.f, 0.f};
-                    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, t.xh[m >> 1][n]), o, c, 0, 0, 0);
-                    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, t.xl[m >> 1][n]), o, c, 0, 0, 0);
+                    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, x.h[m >> 1][n]), o, c, 0, 0, 0);
+                    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, x.l[m >> 1][n]), o, c, 0, 0, 0);
 #pragma unroll
                     for (int i = 0; i < 4; i++) {
-                        const float f = DOWN ? d[m] * __uint_as_float(m >> 1 ? t.sc[DOWN ? n : 0][i].y : t.sc[DOWN ? n : 0][i].x) : d[m];
-                        acc[j][m & 1][n][i] = fmaf(f, c[i], acc[j][m & 1][n][i]);
+                        const float f = DOWN ? d[m] * __uint_as_float(m >> 1 ? x.sc[DOWN ? n : 0][i].y : x.sc[DOWN ? n : 0][i].x) : d[m];
+                        sub[j][m & 1][n][i] = first && m < 2 ? f * c[i] : fmaf(f, c[i], sub[j][m & 1][n][i]);
                     }
                     // added here: left for later, every block's products would be held in registers
-                    asm volatile("" : "+v"(acc[j][m & 1][n]));
+                    asm volatile("" : "+v"(sub[j][m & 1][n]));
                 }
             }
         }
         __builtin_amdgcn_sched_barrier(0);
         load(t, min(s + SETS, nk - 1));
+        load_in(x, min(s + 2, nk - 1));
         __builtin_amdgcn_sched_barrier(0);
     };
+    auto add = [&] {
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int n = 0; n < NT; n++) {
+                    if constexpr (DOWN) acc[j][h][n] += sub[j][h][n];
+                    else tot[j][h][n] += __builtin_convertvector(sub[j][h][n], f64x4);
+                }
+    };
     for (int s = 0; s < nk; s += 4) {  // nk is even
-        step(s, st[0]);
-        step(s + 1, st[1]);
+        step(s, st[0], in[0], true);
+        step(s + 1, st[1], in[1], false);
+        if (!DOWN) add();
         if (s + 2 < nk) {
-            step(s + 2, st[SETS == 4 ? 2 : 0]);
-            step(s + 3, st[SETS == 4 ? 3 : 1]);
+            step(s + 2, st[SETS == 4 ? 2 : 0], in[0], !DOWN);
+            step(s + 3, st[SETS == 4 ? 3 : 1], in[1], false);
+            if (!DOWN) add();
         }
+        if (DOWN) add();
     }
+    if constexpr (!DOWN)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int n = 0; n < NT; n++) acc[j][h][n] = __builtin_convertvector(tot[j][h][n], f32x4);
 }
 
 struct Q8Args {
