@@ -538,6 +538,32 @@ def test_q8_decode_batch_rounding(cuda, E, k, d, fe, T):
     m.close()
 
 
+def q8_blocks(m, scale, quant):
+    """Every gate, up and down block of a Q8_0 layer: (scale, quant) per projection."""
+    (gs, us, _), E = m.slices, m.shape.E
+    for i, (lo, hi) in enumerate(((0, E * gs), (E * gs, E * (gs + us)), (E * (gs + us), m.layer_bytes))):
+        b = m.buf[lo:hi].view(-1, 34)
+        b[:, :2] = torch.tensor([scale[i]], dtype=torch.float16).view(torch.uint8).to(b.device)
+        b[:, 2:] = torch.tensor([quant[i]], dtype=torch.int8).view(torch.uint8).to(b.device)
+
+
+@pytest.mark.parametrize("T", [5, 16])
+def test_q8_decode_batch_overflow(cuda, T):
+    """An activation beyond fp32 is an infinity in the output, as in the fp32
+    kernels (T = 5), not a NaN; the other tokens of its expert stay finite.
+    (One expert per token: a second one's weight of 0 would make it a NaN.)"""
+    m = M.DeviceMoE(W.MoEShape("q8inf", 512, 2, 1, 384, True, W.Q8_0, W.Q8_0, W.Q8_0), 1, seed=83)
+    q8_blocks(m, (1.0, 1.0, 0.5), (1, 1, 1))
+    hb = torch.full((T, 512), 0.001, device=cuda)
+    hb[3] = 2.0 ** 66
+    x = torch.zeros((T, 512), device=cuda)
+    m.forward(0, x, hb)
+    assert torch.isposinf(x[3]).all()
+    rest = x[[t for t in range(T) if t != 3]]
+    assert torch.isfinite(rest).all() and (rest > 0).all()
+    m.close()
+
+
 # gate/up and down types; fe = 1152 and 1280 take more than the 32 blocks of h
 # whose factors the down GEMM holds at a time
 EDGE_TYPES = [(W.Q4_K, W.Q6_K, 512), (W.Q8_0, W.Q8_0, 1152), (W.Q6_K, W.Q4_K, 1280)]

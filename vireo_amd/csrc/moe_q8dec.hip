@@ -282,7 +282,8 @@ VH_DEV void gateup_pass(const Q8Lds &L, const Q8Args &a, gbyte *G, gbyte *U, int
                 const _Float16 hi = _Float16(v);
                 uint16_t *p = a.hp + size_t(pair) * a.fe * 2 + (o >> 3) * 16 + (o & 7);
                 p[0] = __builtin_bit_cast(uint16_t, hi);
-                p[8] = __builtin_bit_cast(uint16_t, _Float16(v - float(hi)));
+                // no low part of an infinity (h overflowed): it would be a NaN
+                p[8] = __builtin_bit_cast(uint16_t, fabsf(v) < 65520.0f ? _Float16(v - float(hi)) : _Float16(0.0f));
             }
         }
 }
