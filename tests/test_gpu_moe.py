@@ -564,6 +564,20 @@ def test_q8_decode_batch_overflow(cuda, T):
     m.close()
 
 
+@pytest.mark.parametrize("T", [5, 16, 64])
+def test_large_finite_inputs(cuda, T):
+    """Inputs of 2^120: gate rows of -2^109 and up rows of 2^109 give activations of
+    -0 (silu of a large negative number) and a contribution of 0, in the fp32
+    kernels (T = 5), the decode batch and the fp16 GEMMs, whose scale has to bring
+    the inputs into fp16's range first. (An infinite gate row would be a NaN.)"""
+    m = M.DeviceMoE(W.MoEShape("q8big", 512, 2, 1, 384, True, W.Q8_0, W.Q8_0, W.Q8_0), 1, seed=89)
+    q8_blocks(m, (2.0 ** -20, 2.0 ** -20, 1.0), (-1, 1, 1))
+    x = torch.ones((T, 512), device=cuda)
+    m.forward(0, x, torch.full((T, 512), 2.0 ** 120, device=cuda))
+    assert (x == 1.0).all()
+    m.close()
+
+
 # gate/up and down types; fe = 1152 and 1280 take more than the 32 blocks of h
 # whose factors the down GEMM holds at a time
 EDGE_TYPES = [(W.Q4_K, W.Q6_K, 512), (W.Q8_0, W.Q8_0, 1152), (W.Q6_K, W.Q4_K, 1280)]

@@ -107,12 +107,13 @@ struct Op<VT_Q6_K> {  // src/gguf_compute.c:83-103: y = (d sc) (q - 32)
 
 // The power of two a weight row's scales are multiplied by, as its exponent:
 // bound * 2^e lies in [2^13, 2^14) for a bound on the row's magnitudes (0 for
-// a row of zeros or with a scale that is not finite).
+// a row of zeros or with a scale that is not finite). -114 takes the largest
+// fp32 number there; below 2^-86 the result is that much smaller.
 VH_DEV int exponent_for(float bound) {
     if (!(bound > 0.0f) || !(bound <= 3.4028234663852886e38f)) return 0;
     int ex;
     frexpf(bound, &ex);
-    return max(-100, min(100, 14 - ex));
+    return max(-114, min(100, 14 - ex));
 }
 
 // GGUF rows: the loads of one lane and step (raw), their rearrangement into
