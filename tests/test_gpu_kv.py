@@ -268,3 +268,39 @@ def test_attention_tile_edges(cuda, d, G, heads, kv_heads, ctx):
     print(f"d={d} G={G} {heads}/{kv_heads} ctx={ctx}: max rel {err:.2e}")
     assert err <= 2e-5
     assert torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("d,G,masked,ctx", [(64, 16, 32, 100), (128, 32, 96, 130), (128, 32, 64, 4200), (64, 8, 40, 40),
+                                            (256, 64, 31, 32)])
+def test_attention_scores_of_minus_infinity(cuda, d, G, masked, ctx):
+    """Tokens whose scores are -inf have no weight, also where they fill the first
+    tiles of 32 (32, 64, 96), whole chunks (96 of 130 tokens) or all of a chunk's
+    first tile (4200 tokens: two tiles per chunk), over listed and contiguous
+    blocks; where every score is -inf the output is a NaN, as the softmax is.
+    Same bound as test_attention_tile_edges."""
+    from vireo_amd import kv as KV
+    heads, kv_heads = 8, 2
+    gen = torch.Generator(device=cuda)
+    gen.manual_seed(ctx)
+    k, v = (torch.randn((ctx, kv_heads, d), generator=gen, device=cuda) for _ in range(2))
+    q = torch.randn((heads, d), generator=gen, device=cuda)
+    q[:, 0] = q[:, 0].abs() + 0.1
+    k[:masked, :, 0] = -float("inf")
+    s = torch.softmax((q.double().view(kv_heads, -1, d) @ k.double().permute(1, 2, 0).contiguous()) / d ** 0.5, -1)
+    want = (s @ v.double().permute(1, 0, 2).contiguous()).reshape(heads, d)
+    for max_tokens in (0, ctx + 70):
+        st = KV.DeviceKV(kv_heads, d, G, dense=True, max_tokens=max_tokens)
+        out = torch.empty((heads, d), device=cuda)
+        for t in range(ctx):
+            st.append(0, t, k[t], v[t])
+        if max_tokens:
+            pos = torch.full((1,), ctx - 1, dtype=torch.int32, device=cuda)
+            st.attend_gqa_pos(0, heads, kv_heads, pos, q, out)
+        else:
+            st.attend_gqa(0, heads, kv_heads, q, out)
+        if masked == ctx:
+            assert torch.isnan(out).all()
+        else:
+            assert float((out.double() - want).abs().max() / want.abs().max()) <= 2e-5
+        torch.cuda.synchronize()
+        st.close()

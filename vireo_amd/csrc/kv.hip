@@ -253,7 +253,8 @@ __global__ void __launch_bounds__(256) kv_merge_kernel(const float *__restrict__
             a.z += red[u][tid].z;
             a.w += red[u][tid].w;
         }
-        const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+        // no tokens: 0; every score -inf: a NaN, as the softmax of them is
+        const float inv = L > 0.0f ? 1.0f / L : nc > 0 && M == -INFINITY ? NAN : 0.0f;
         float *o = out + size_t(h) * D + 4 * tid;  // any 4-byte alignment
         o[0] = a.x * inv;
         o[1] = a.y * inv;
@@ -391,7 +392,10 @@ __global__ void __launch_bounds__(256, D <= 128 ? 3 : 2) kv_attend_group_kernel(
             const int i = wv + 4 * x;
             if (i >= HPG) break;
             const float a = lane < kTileTok ? ps[b][i][lane] : -INFINITY, mn = fmaxf(rm[x], wave_max_f(a));
-            const float corr = expf(rm[x] - mn), pa = lane < lim ? expf(a - mn) : 0.0f;
+            // a score of -inf has no weight, whatever the largest so far: a tile of
+            // such scores alone is as if it were empty
+            const float corr = rm[x] == mn ? 1.0f : expf(rm[x] - mn);
+            const float pa = lane < lim && a != -INFINITY ? expf(a - mn) : 0.0f;
             rl[x] = rl[x] * corr + wave_sum_f(pa);
             rm[x] = mn;
             if (lane < kTileTok) ps[b][i][lane] = pa;
