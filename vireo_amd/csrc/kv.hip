@@ -200,8 +200,17 @@ __global__ void __launch_bounds__(256) kv_merge_kernel(const float *__restrict__
     __shared__ float4 red[NG][NDQ];
     __shared__ float wm[4], wl[4];
     const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, dq = tid % NDQ, grp = tid / NDQ;
-    const int nc = counts.chunks(h);
     const float4 *p = reinterpret_cast<const float4 *>(part + size_t(h) * nchunk * D) + dq;
+    // Heads of 64: the first chunks' accumulators are requested before it is known
+    // how many chunks the head has (those past its own are in the buffer and not
+    // used): 16 heads at 1000 tokens 11.3 -> 10.6 us with the attention and the append.
+    // Of 128 the larger rows hold up the weights behind them: 60 tokens 10.8 -> 11.5 us.
+    constexpr bool EARLY = DPL == 1;
+    float4 v[U];
+    if (EARLY)
+#pragma unroll
+        for (int u = 0; u < U; u++) v[u] = p[size_t(min(grp + NG * u, nchunk - 1)) * NDQ];
+    const int nc = counts.chunks(h);
     ml += size_t(h) * nchunk;
     float M = -INFINITY;
     for (int c = tid; c < nc; c += 256) M = fmaxf(M, ml[c].x);
@@ -227,9 +236,9 @@ __global__ void __launch_bounds__(256) kv_merge_kernel(const float *__restrict__
         __syncthreads();
         L += (wl[0] + wl[1]) + (wl[2] + wl[3]);
         for (int u0 = grp; u0 < n; u0 += NG * U) {
-            float4 v[U];
+            if (!EARLY || c0 + u0 != grp)
 #pragma unroll
-            for (int u = 0; u < U; u++) v[u] = p[size_t(c0 + min(u0 + NG * u, n - 1)) * NDQ];
+                for (int u = 0; u < U; u++) v[u] = p[size_t(c0 + min(u0 + NG * u, n - 1)) * NDQ];
 #pragma unroll
             for (int u = 0; u < U; u++)
                 if (u0 + NG * u < n) {
