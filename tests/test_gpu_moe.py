@@ -617,6 +617,66 @@ def test_prefill_tiles_and_scales(cuda, oracle, tg, td, fe, T):
     m.close()
 
 
+def set_scales(raw, typ, K, factors):
+    """Multiply the scales of every row's blocks (of K weights a row) in the bytes `raw` by factors [period x
+    blocks]: row r takes line r % period, a block that is 0 there is all zeros."""
+    be, bb = W.BLOCK[typ]
+    at = {W.Q8_0: (0,), W.Q4_K: (0, 2), W.Q6_K: (208,)}[typ]
+    b = raw.view(-1, K // be, bb)
+    f = torch.as_tensor(factors, dtype=torch.float32, device=raw.device)
+    f = f[torch.arange(b.shape[0], device=raw.device) % f.shape[0]]
+    for o in at:
+        d = b[:, :, o:o + 2].contiguous().view(torch.float16)[..., 0].float()
+        b[:, :, o:o + 2] = (d * f).half().unsqueeze(-1).view(torch.uint8)
+
+
+def span_factors(n):
+    """Lines of n factors: scales up to 2^12 apart within a row."""
+    one = np.ones(n)
+    up = [one * 2.0 ** -12, one.copy(), one * 2.0 ** -12, np.zeros(n), one * 2.0 ** -6, one.copy(), one * 2.0 ** -12]
+    up[0][n // 2:] = 1.0                                     # small, then 2^12 times as large
+    up[1][n // 2:] = 2.0 ** -12                              # the other way round
+    up[2][[n // 3, (2 * n) // 3, n - 1]] = 2.0 ** -8, 2.0 ** -4, 1.0  # several jumps, the last at the end
+    up[3][1:] = 2.0 ** -5                                    # a first block of zeros
+    up[4][1 if n > 1 else 0] = 1.0                           # the second block alone (Q8_0: one half of a step)
+    up[6][n - 1] = 1.0                                       # the last block alone
+    return np.stack(up)
+
+
+@pytest.mark.parametrize("tg,td", [(W.Q4_K, W.Q6_K), (W.Q8_0, W.Q8_0), (W.Q6_K, W.Q4_K)])
+@pytest.mark.parametrize("T", [70, 600])
+def test_prefill_rows_with_wide_scales(cuda, tg, td, T):
+    """Rows whose blocks' scales lie up to 2^12 apart, or start with blocks of
+    zeros, in gate, up and down: the GEMMs on GGUF rows lower such a row's power
+    of two on the way and rescale what it has summed; the fragment copy knows
+    the row's largest. The same bits from both (no operand is subnormal in
+    fp16), and within test_prefill_tiles_and_scales' bound of a 64-bit evaluation;
+    both token tiles (64 and 128 rows)."""
+    lib = _lib.load()
+    shape = W.MoEShape("wide", 1536, 8, 2, 768, True, tg, tg, td)
+    m = M.DeviceMoE(shape, 1, seed=97)
+    (gs, us, ds), E = m.slices, shape.E
+    for at, nb, typ, K in ((0, E * (gs + us), tg, shape.d), (E * (gs + us), E * ds, td, shape.fe)):
+        set_scales(m.buf[at:at + nb], typ, K, span_factors(K // W.BLOCK[typ][0]))
+    _, hb = W.host_hidden(shape.d, T, 97)
+    hbt = torch.from_numpy(hb).to(cuda)
+    outs = []
+    try:
+        for packed in (0, 1):
+            _lib.check(lib.vireo_hip_set_packed(packed), "vireo_hip_set_packed")
+            xt = torch.zeros((T, shape.d), device=cuda)
+            idx, w = m.forward(0, xt, hbt, return_routing=True)
+            outs.append(xt.clone())
+    finally:
+        lib.vireo_hip_set_packed(1)
+    want = layer_64(m, hbt, idx, w)
+    rel = float(((outs[1].double() - want).abs().amax(1) / want.abs().amax(1)).max())
+    print(f"T={T}: max rel {rel:.2e}, bits differ in {int((outs[0] != outs[1]).sum())} of {outs[0].numel()}")
+    assert rel <= 4e-3
+    assert torch.equal(outs[0], outs[1])
+    m.close()
+
+
 def test_grouped_plan_large_groups_unregistered(cuda, oracle, path):
     """Unregistered experts among the matrix-core groups contribute nothing."""
     path(0)

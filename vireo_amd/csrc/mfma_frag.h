@@ -138,7 +138,6 @@ struct Rows<VT_Q8_0> {
     };
     static VH_DEV int blocks(int K) { return K / 32; }
     static VH_DEV float bound(gbyte *row, int b) { return fabsf(h2f(ld_u16(row + 34 * b))) * 128.0f; }
-    static VH_DEV float step_bound(const Raw &r) { return fabsf(h2f(r.d)) * 128.0f; }
     static VH_DEV void load(gbyte *row, int s, int half, Raw &r) {  // block 2 s + half
         gbyte *p = row + 68 * s + 34 * half;
         r.q[0] = ld_u128(p + 2);
@@ -162,7 +161,6 @@ struct Rows<VT_Q4_K> {
         return fmaxf(fabsf(h2f(h & 0xffffu)) * (63.0f * 15.0f), fabsf(h2f(h >> 16)) * 63.0f);
     }
     static VH_DEV float bound(gbyte *row, int b) { return bound_of(ld_u32(row + 144 * b)); }
-    static VH_DEV float step_bound(const Raw &r) { return bound_of(r.hdr.x); }
     // step s: the 32 bytes s % 4 of super-block s / 4, low nibbles (sub-block 2 (s % 4)) for half 0, high for 1
     static VH_DEV void load(gbyte *row, int s, int, Raw &r) {
         gbyte *p = row + 144 * (s >> 2);
@@ -192,7 +190,6 @@ struct Rows<VT_Q6_K> {
     };
     static VH_DEV int blocks(int K) { return K / 256; }
     static VH_DEV float bound(gbyte *row, int b) { return fabsf(h2f(ld_u16(row + 210 * b + 208))) * (128.0f * 32.0f); }
-    static VH_DEV float step_bound(const Raw &r) { return fabsf(h2f(r.d)) * (128.0f * 32.0f); }
     // step s: half h = (s % 4) / 2 of super-block s / 4, group g = 2 (s % 2) +
     // `half`: weight l has its low bits in ql[64 h + 32 (g % 2) + l] (low nibbles
     // for g < 2), its high bits 2 g of qh[32 h + l], its scale in scales[8 h + 2 g + l / 16]
@@ -259,6 +256,236 @@ struct Frag {
         if constexpr (NW == 6) *reinterpret_cast<uint2 *>(p + 1024 + 8 * lane) = make_uint2(w[4], w[5]);
         if constexpr (SB == 4) *reinterpret_cast<uint32_t *>(p + 256 * NW + 4 * lane) = sc;
         else *reinterpret_cast<uint16_t *>(p + 256 * NW + 2 * lane) = uint16_t(sc);
+    }
+};
+
+// ---- GGUF rows staged by a wave -----------------------------------------------
+// A wave reads its 64 rows (fragment 0's 32, then fragment 1's) a pair of K
+// steps (128 columns) at a time, in 16-byte pieces with neighbouring lanes on
+// neighbouring bytes of a row, through registers (Regs: the pair in flight) into
+// its own part of LDS (Lds: the pair being multiplied), where every lane finds the
+// words of its row. A lane per row touched 64 lines with every load instruction,
+// and rearranging what it read took more vector instructions than the multiplies
+// leave time for: Qwen3 Q4_K_M 2048 tokens gate/up 331 -> 206 us, down 372 -> 154
+// (from the packed copy 158 and 107); Q8_0 323 -> 247 and 166 -> 151 (170 and 107).
+// Q8_0's pieces are those of the row, 8-byte aligned, not of its 34-byte blocks:
+// loads at odd multiples of 2 bytes ran at half the rate.
+//   load(r, B, rb, t, lane)  requests pair t of the rows at B[0], B[1] (the
+//                            fragments' first rows), rb bytes apart
+//   bounds(r, b)             the rows' magnitude bounds in the pair
+//   put(l, r, up, lane)      the pair's pieces and its scales (those of Op<T>)
+//   fetch(l, p, i, j, ..)    step p's words 4 i .. 4 i + 3 of fragment j (sub-steps
+//                            2 i, 2 i + 1): a byte per weight
+//   get(w0, w1, sc, ks, c)   the operand of sub-step ks, Op<T>::get's bits
+// K-quants: the pieces are swizzled so that 16 lanes' reads and writes take 16 bank
+// groups, and a lane per row forms the pair's scales. Q8_0 (PER_STEP): the lanes
+// that multiply a row form its scale step by step.
+// A row's power of two follows from its first bound (below 2^11 under it) and is
+// lowered, with what the row has summed (lower_up), where a later bound would pass
+// 2^15 under it: no pass over the row's scales ahead. Powers of two are exact, so
+// the results are the packed copy's while no scale is subnormal in fp16 under
+// either power: while a row's scales lie within 2^12 of its largest.
+template <int T>
+struct Staged;
+
+// A lane's offset as a value of its own where it is used: added to a uniform
+// base by the load itself. (Hoisted out of the loop as a 64-bit pair, and LDS
+// addresses one per store, they take the registers of the loop's operands.)
+VH_DEV uint32_t here(uint32_t v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+template <int N>  // whether any lane's power was lowered (fix is set only then)
+VH_DEV bool lower_up(const float (&bound)[N], float (&up)[N], float (&fix)[N]) {
+    bool over = false;
+#pragma unroll
+    for (int i = 0; i < N; i++) over |= bound[i] * up[i] >= 32768.0f;
+    if (!__any(over)) return false;
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        const float to = bound[i] * up[i] >= 32768.0f ? ldexpf(1.0f, exponent_for(bound[i]) - 3) : up[i];
+        fix[i] = to / up[i];
+        up[i] = to;
+    }
+    return true;
+}
+VH_DEV float first_up(float bound) { return ldexpf(1.0f, bound > 0.0f ? exponent_for(bound) - 3 : 14); }
+VH_DEV float larger_bound(float a, float b) { return b > a || !(b <= 3.4028234663852886e38f) ? b : a; }
+
+// a byte of w per half of the operand: fp16 1024 + byte, less `zero`
+VH_DEV f16x2 byte_pair(uint32_t w, int odd, uint32_t b64, float zero) {
+    const uint32_t v = __builtin_amdgcn_perm(w, b64, odd ? 0x00070006u : 0x00050004u);
+    return as_h2(v) - splat(_Float16(zero));
+}
+
+template <>
+struct Staged<VT_Q8_0> {
+    // A row's 136 bytes of a pair are staged as they are: the scales lie in them, so
+    // the lanes that multiply a row (both halves) keep its power of two.
+    static constexpr bool PER_STEP = true;
+    static constexpr int NU = 2;  // of the lane's rows of the two fragments
+    struct Regs {
+        uint4 q[8];
+        uint2 tail;
+    };
+    struct Lds {
+        uint32_t q[64 * 34];
+    };
+    static VH_DEV void load(Regs &r, gbyte *const (&B)[2], int64_t rb, int t, int lane) {
+        const uint32_t o = here(uint32_t(lane >> 3) * uint32_t(rb) + 16u * uint32_t(lane & 7));
+#pragma unroll
+        for (int q = 0; q < 8; q++) r.q[q] = ld_u128(B[q >> 2] + (8 * (q & 3)) * rb + 136 * t + o);
+        r.tail = ld_u64((lane < 32 ? B[0] : B[1]) + 136 * t + 128 + uint32_t(lane & 31) * uint32_t(rb));
+    }
+    static VH_DEV void put(Lds &l, const Regs &r, int lane) {
+        // 8 bytes at a time: two in one store would reach 2 KB from its address register
+        typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+        auto *o = reinterpret_cast<volatile __attribute__((address_space(3))) u32x2 *>(
+            (__attribute__((address_space(3))) uint32_t *)l.q + 34 * (lane >> 3) + 4 * (lane & 7));
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            o[136 * q] = u32x2{r.q[q].x, r.q[q].y};
+            o[136 * q + 1] = u32x2{r.q[q].z, r.q[q].w};
+        }
+        *reinterpret_cast<uint2 *>(l.q + 34 * lane + 32) = r.tail;
+    }
+    // block `half` of the step lies at byte 34 `half` of its 68: words 0 .. 8, or 8 .. 16
+    // with the scale in the upper half of the first
+    static VH_DEV void fetch(const Lds &l, int p, int i, int j, int half, int col, uint32_t (&w)[4], uint32_t &d) {
+        const uint32_t *x = l.q + 34 * (32 * j + col) + 17 * p + 8 * half + 4 * i;
+        const uint32_t sel = half ? 0x07060504u : 0x05040302u;
+        uint32_t v[5];
+#pragma unroll
+        for (int k = 0; k < 5; k++) v[k] = x[k];
+#pragma unroll
+        for (int k = 0; k < 4; k++) w[k] = __builtin_amdgcn_perm(v[k + 1], v[k], sel) ^ 0x80808080u;
+        if (i == 0) d = half ? v[0] >> 16 : v[0] & 0xffffu;
+    }
+    static VH_DEV float step_bound(uint32_t d) {  // of the row's step: both halves'
+        const uint32_t b = __float_as_uint(fabsf(h2f(d)) * 128.0f);
+        const auto v = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+        return larger_bound(__uint_as_float(v[0]), __uint_as_float(v[1]));
+    }
+    static VH_DEV float of_row(const float (&v)[NU], int j, int) { return v[j]; }
+    static VH_DEV f16x8 get(uint32_t w0, uint32_t w1, uint32_t sc, int, const Consts &c) {
+        const f16x2 d = splat(as_h2(sc)[0]);
+        const f16x2 p0 = byte_pair(w0, 0, c.b, 1152.0f) * d, p1 = byte_pair(w0, 1, c.b, 1152.0f) * d;
+        const f16x2 p2 = byte_pair(w1, 0, c.b, 1152.0f) * d, p3 = byte_pair(w1, 1, c.b, 1152.0f) * d;
+        return f16x8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
+    }
+};
+
+template <>
+struct Staged<VT_Q4_K> {
+    static constexpr bool PER_STEP = false;
+    static constexpr int NU = 1;  // lane r holds row r's power
+    struct Regs {
+        uint4 q[4], hdr;
+        uint32_t t;  // the pair (uniform)
+    };
+    struct Lds {
+        uint4 q[256];
+        uint4 sc[64];
+    };
+    static VH_DEV void load(Regs &r, gbyte *const (&B)[2], int64_t rb, int t, int lane) {
+        const uint32_t oq = here(uint32_t(lane >> 2) * uint32_t(rb) + 16u * uint32_t(lane & 3));
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            r.q[q] = ld_u128(B[q >> 1] + (16 * (q & 1)) * rb + 144 * (t >> 1) + 16 + 64 * (t & 1) + oq);
+        r.hdr = ld_u128((lane < 32 ? B[0] : B[1]) + 144 * (t >> 1) + uint32_t(lane & 31) * uint32_t(rb));
+        r.t = uint32_t(t);
+    }
+    static VH_DEV void bounds(const Regs &r, float (&b)[NU]) { b[0] = Rows<VT_Q4_K>::bound_of(r.hdr.x); }
+    static VH_DEV float of_row(const float (&v)[NU], int j, int col) { return __shfl(v[0], 32 * j + col, 64); }
+    static VH_DEV void put(Lds &l, const Regs &r, const float (&up)[NU], int lane) {
+        const int a = 4 * (lane >> 2) + ((lane & 3) ^ (lane >> 4));
+#pragma unroll
+        for (int q = 0; q < 4; q++) l.q[64 * q + a] = r.q[q];
+        // the scales and minima of sub-blocks 4 (t % 2) .. + 3, a byte each (q4k_scale_min)
+        const uint32_t s = (r.t & 1) ? (r.hdr.w & 0x0f0f0f0fu) | ((r.hdr.y >> 2) & 0x30303030u) : r.hdr.y & 0x3f3f3f3fu;
+        const uint32_t m = (r.t & 1) ? ((r.hdr.w >> 4) & 0x0f0f0f0fu) | ((r.hdr.z >> 2) & 0x30303030u) : r.hdr.z & 0x3f3f3f3fu;
+        const float d = h2f(r.hdr.x & 0xffffu) * up[0], dm = h2f(r.hdr.x >> 16) * up[0];
+        uint32_t o[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            o[i] = h_bits(d * float((s >> (8 * i)) & 0xffu)) | h_bits(dm * float((m >> (8 * i)) & 0xffu)) << 16;
+        l.sc[lane] = make_uint4(o[0], o[1], o[2], o[3]);
+    }
+    static VH_DEV void fetch(const Lds &l, int p, int i, int j, int half, int col, uint32_t (&w)[4]) {
+        const uint4 v = l.q[128 * j + 4 * col + ((2 * p + i) ^ ((col >> 2) & 3))];
+        const int sh = 4 * half;
+        w[0] = (v.x >> sh) & 0x0f0f0f0fu;
+        w[1] = (v.y >> sh) & 0x0f0f0f0fu;
+        w[2] = (v.z >> sh) & 0x0f0f0f0fu;
+        w[3] = (v.w >> sh) & 0x0f0f0f0fu;
+    }
+    static VH_DEV f16x8 get(uint32_t w0, uint32_t w1, uint32_t sc, int, const Consts &c) {
+        const f16x2 s = as_h2(sc), d = splat(s[0]), m = -splat(s[1]);
+        const f16x2 p0 = __builtin_elementwise_fma(byte_pair(w0, 0, c.b, 1024.0f), d, m);
+        const f16x2 p1 = __builtin_elementwise_fma(byte_pair(w0, 1, c.b, 1024.0f), d, m);
+        const f16x2 p2 = __builtin_elementwise_fma(byte_pair(w1, 0, c.b, 1024.0f), d, m);
+        const f16x2 p3 = __builtin_elementwise_fma(byte_pair(w1, 1, c.b, 1024.0f), d, m);
+        return f16x8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
+    }
+};
+
+template <>
+struct Staged<VT_Q6_K> {
+    static constexpr bool PER_STEP = false;
+    static constexpr int NU = 1;
+    struct Regs {
+        uint4 ql[4], qh[2];
+        uint2 sc;
+        uint32_t d;
+    };
+    struct Lds {
+        uint4 ql[256], qh[128];
+        uint4 sc[64];
+    };
+    // pair t: half t % 2 of super-block t / 2 (Rows<VT_Q6_K>)
+    static VH_DEV void load(Regs &r, gbyte *const (&B)[2], int64_t rb, int t, int lane) {
+        const int sb = 210 * (t >> 1), h = t & 1;
+        const uint32_t ol = here(uint32_t(lane >> 2) * uint32_t(rb) + 16u * uint32_t(lane & 3)),
+                       oh = here(uint32_t(lane >> 1) * uint32_t(rb) + 16u * uint32_t(lane & 1));
+#pragma unroll
+        for (int q = 0; q < 4; q++) r.ql[q] = ld_u128(B[q >> 1] + (16 * (q & 1)) * rb + sb + 64 * h + ol);
+#pragma unroll
+        for (int q = 0; q < 2; q++) r.qh[q] = ld_u128(B[q] + sb + 128 + 32 * h + oh);
+        gbyte *p = (lane < 32 ? B[0] : B[1]) + sb + uint32_t(lane & 31) * uint32_t(rb);
+        r.sc = ld_u64(p + 192 + 8 * h);
+        r.d = ld_u16(p + 208);
+    }
+    static VH_DEV void bounds(const Regs &r, float (&b)[NU]) { b[0] = fabsf(h2f(r.d)) * (128.0f * 32.0f); }
+    static VH_DEV float of_row(const float (&v)[NU], int j, int col) { return __shfl(v[0], 32 * j + col, 64); }
+    static VH_DEV void put(Lds &l, const Regs &r, const float (&up)[NU], int lane) {
+        const int a = 4 * (lane >> 2) + ((lane & 3) ^ (lane >> 4)), b = 2 * (lane >> 1) + ((lane & 1) ^ ((lane >> 4) & 1));
+#pragma unroll
+        for (int q = 0; q < 4; q++) l.ql[64 * q + a] = r.ql[q];
+#pragma unroll
+        for (int q = 0; q < 2; q++) l.qh[64 * q + b] = r.qh[q];
+        const float d = h2f(r.d) * up[0];
+        uint32_t o[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint32_t v = i < 2 ? r.sc.x : r.sc.y;
+            o[i] = h_bits(d * float(int(int8_t(v >> (16 * (i & 1)))))) | h_bits(d * float(int(int8_t(v >> (16 * (i & 1) + 8))))) << 16;
+        }
+        l.sc[lane] = make_uint4(o[0], o[1], o[2], o[3]);
+    }
+    static VH_DEV void fetch(const Lds &l, int p, int i, int j, int half, int col, uint32_t (&w)[4]) {
+        const uint4 v = l.ql[128 * j + 4 * col + ((2 * half + i) ^ ((col >> 2) & 3))];
+        const uint4 h = l.qh[64 * j + 2 * col + (i ^ ((col >> 3) & 1))];
+        const int sl = 4 * p, sh = 4 * p + 2 * half;
+#pragma unroll
+        for (int x = 0; x < 4; x++)
+            w[x] = ((u4_at(v, x) >> sl) & 0x0f0f0f0fu) | (((u4_at(h, x) >> sh) & 0x03030303u) << 4);
+    }
+    static VH_DEV f16x8 get(uint32_t w0, uint32_t w1, uint32_t sc, int ks, const Consts &c) {
+        const f16x2 d = splat(as_h2(sc)[ks >> 1]);
+        const f16x2 p0 = byte_pair(w0, 0, c.b, 1056.0f) * d, p1 = byte_pair(w0, 1, c.b, 1056.0f) * d;
+        const f16x2 p2 = byte_pair(w1, 0, c.b, 1056.0f) * d, p3 = byte_pair(w1, 1, c.b, 1056.0f) * d;
+        return f16x8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
     }
 };
 

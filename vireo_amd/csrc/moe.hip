@@ -817,7 +817,8 @@ int ffn_forward(const vireo_moe_model *m, int layer, float *x, const float *hb, 
         // experts of a pinned layer: the fragment copy (made on the first such call that may allocate)
         const void *const *pt = rc ? nullptr : packed_table(m, layer, table, !src, s, 1);
         // the tile plan and the GEMMs' fp16 inputs in one launch
-        if (!rc) rc = vh_mfma_plan(ws.counts, ws.offs, E, n_tokens, k, tg, td, d, fe, ws.tiles, hb, ws.xb, ws.xsc, s);
+        if (!rc) rc = vh_mfma_plan(ws.counts, ws.offs, E, n_tokens, k, tg, td, d, fe, pt != nullptr, ws.tiles, hb, ws.xb,
+                                   ws.xsc, s);
         const void *const *tb = pt ? pt : table;
         if (!rc) rc = vh_mfma_gateup(tg, ws.tiles, P, E, ws.perm, tb, pt != nullptr, ws.xb, ws.xsc,
                                      d, fe, k, ws.hs, ws.he, s);

@@ -25,15 +25,18 @@
 // dequantizes its own 64 rows in registers and multiplies all of the tile's
 // rows by them, so a weight is converted once per workgroup and an input
 // fragment read from LDS feeds two multiplies (with 32 rows per wave the
-// operand reads alone took all of the LDS bandwidth). Only the inputs pass
-// through LDS, double buffered, as 16-byte chunks of 8 consecutive K values laid
-// out [K/8][row] (row index XOR-swizzled by the chunk), so a 32-lane group's
+// operand reads alone took all of the LDS bandwidth). The inputs pass through
+// LDS in three buffers (two: TileLds) as 16-byte chunks of 8 consecutive K values
+// laid out [K/8][row] (row index XOR-swizzled by the chunk), so a 32-lane group's
 // operand read is one contiguous 512-byte run. Two workgroups share a CU:
 // 256 registers, two waves per SIMD, one converting while the other multiplies.
 //
 // Weights: the experts of a pinned layer come from a copy in the operand order
-// (Frag, vh_mfma_pack); others are read from their GGUF rows and rearranged in
-// registers into the same words, so the results do not depend on the source.
+// (Frag, vh_mfma_pack); others are read from their GGUF rows, each wave's through
+// its own part of LDS (Staged), into the same operands, so the results do not
+// depend on the source. Per layer, GGUF rows / copy: Qwen3 Q4_K_M 101 tokens 233 /
+// 178 us, 2048 465 / 396; Q8_0 253 / 198 and 498 / 410 (2048 tokens through the
+// kernel that staged bf16 weights for the whole workgroup: 672 and 540).
 //
 // Order: the workgroups are numbered so that each XCD (hardware dispatch sends
 // workgroup b to XCD b mod 8) takes a contiguous run of (token tile, column
@@ -57,7 +60,6 @@ namespace {
 
 constexpr int kBRows = 256, kWaves = 4, kThreads = 64 * kWaves, kXcds = 8;
 constexpr int kChunks = kBK / 8;  // 16-byte chunks per row and K step
-constexpr int kBufs = 3;          // LDS buffers of the inputs: the step's, the next one's, and the one being written
 constexpr int kBigTile = 128, kSmallTile = 64;  // the largest token tile of the two kernels (tile_rows)
 
 struct GemmArgs {
@@ -83,14 +85,30 @@ VH_DEV void fold(float (&m)[16], bool hi) {
     }
 }
 
+// orders the lanes' LDS accesses within a wave (the hardware keeps their order)
+VH_DEV void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // 2^n as fp16 bits, n <= 0 (0 below 2^-24)
 VH_DEV uint32_t h_pow2(int n) { return n >= -14 ? uint32_t(15 + n) << 10 : n >= -24 ? 1u << (24 + n) : 0u; }
 
 constexpr int kFacBlocks = 32;  // blocks of h whose factors are in LDS at a time
 
-template <bool GATEUP, int LDB>
+// LDS of a workgroup. The inputs have three buffers (the step's, the next one's
+// and the one being written), or two where the staged rows (Staged) leave no room
+// for a third in half of a CU's 160 KB.
+template <int T, bool GATEUP, int LDB, bool PK>
+constexpr int input_bufs() { return !PK && (T == VT_Q8_0 || (LDB == kBigTile && T == VT_Q6_K && !GATEUP)) ? 2 : 3; }
+struct NoRows {};
+
+template <int T, bool GATEUP, int LDB, bool PK>
 struct TileLds {
-    f16x8 As[kBufs][kChunks][LDB];
+    static constexpr int NB = input_bufs<T, GATEUP, LDB, PK>();
+    f16x8 As[NB][kChunks][LDB];
+    std::conditional_t<PK, NoRows, typename Staged<T>::Lds> rows[kWaves];
     float rsc[LDB];                                  // the rows' scales in the epilogue
     float hsc[GATEUP ? kWaves : 1][32];              // gate/up: a wave's 32 row scales of h
     int prow[GATEUP ? 1 : LDB];                      // down: the rows' y rows
@@ -104,14 +122,14 @@ struct TileLds {
 // perm[i]. i runs over base + m0 .. + mcnt - 1 (mcnt <= BM) within the group;
 // rows of the tile past mcnt repeat the group's last row and are not stored.
 //
-// K step s: the inputs of step s + 2 go from registers into LDS and those of s
-// + 3 are requested; the wave multiplies step s, forming its operands from the
-// weights requested two steps ago, and requests those of step s + 2. Every load
-// is unconditional (steps past the end repeat the last one), so the waits count
-// exactly the loads issued after the one needed, and the barrier is LDS-only:
-// loads stay in flight across it.
+// K step s: the inputs of step s + 2 (s + 1 with two buffers) go from registers
+// into LDS and the next ones are requested; the wave multiplies step s, forming
+// its operands from the weights requested two steps ago (GGUF rows: a pair of steps)
+// and requests more. Every load is unconditional (steps past the end repeat
+// the last one), so the waits count exactly the loads issued after the one needed,
+// and the barrier is LDS-only: loads stay in flight across it.
 template <int T, bool GATEUP, int BM, int LDB, bool PK>
-VH_DEV void gemm_tile(TileLds<GATEUP, LDB> &L, const GemmArgs &a, gbyte *M0, gbyte *M1, int base, int m0, int mcnt,
+VH_DEV void gemm_tile(TileLds<T, GATEUP, LDB, PK> &L, const GemmArgs &a, gbyte *M0, gbyte *M1, int base, int m0, int mcnt,
                       int n0) {
     using O = Op<T>;
     constexpr int FI = BM / 32, AQ = BM * kChunks / kThreads;
@@ -165,7 +183,7 @@ VH_DEV void gemm_tile(TileLds<GATEUP, LDB> &L, const GemmArgs &a, gbyte *M0, gby
     uint4 av[AQ];
     auto loadA = [&](int step) {
 #pragma unroll
-        for (int q = 0; q < AQ; q++) av[q] = ld_u128(abase + 128 * step + aoff[q]);
+        for (int q = 0; q < AQ; q++) av[q] = ld_u128(abase + 128 * step + (PK ? aoff[q] : here(aoff[q])));
     };
     auto storeA = [&](int buf, int step) {
 #pragma unroll
@@ -182,34 +200,15 @@ VH_DEV void gemm_tile(TileLds<GATEUP, LDB> &L, const GemmArgs &a, gbyte *M0, gby
     // the wave's weights: fragment group c of the packed matrix, or the lane's two GGUF rows
     const int c = n0 / (GATEUP ? 32 : 64) + wv, col = lane & 31;
     gbyte *fb = M0 + size_t(c) * nk * 2 * Frag<T>::bytes;
-    gbyte *row[2];
-    float up[2], rs[2];  // the rows' powers of two (GGUF rows) and, for the epilogue, their inverses
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const int r = GATEUP ? 32 * c + col : 64 * c + 32 * j + col;
-        if constexpr (PK) {
-            const size_t frags = size_t(GATEUP ? 2 : 1) * a.rows / 32 * nk * Frag<T>::bytes;
-            rs[j] = __uint_as_float(ld_u32(M0 + frags + 4 * (GATEUP ? j * a.rows + r : r)));
-        } else {
-            row[j] = (GATEUP && j ? M1 : M0) + int64_t(r) * a.row_bytes;
-        }
-    }
-    struct Words {
-        uint32_t w[O::NW], sc;
-    };
-    struct Raw {
-        typename Rows<T>::Raw g;
-    };
-    using Set = std::conditional_t<PK, Words, Raw>;
-    // GGUF rows are rearranged into words a step ahead, so one set of them is in flight
-    Set st[PK ? 2 : 1][2];
-    auto loadB = [&](Set (&g)[2], int step) {
+    float rs[2];  // the inverses of the rows' powers of two, for the epilogue
+    if constexpr (PK) {
 #pragma unroll
         for (int j = 0; j < 2; j++) {
-            if constexpr (PK) Frag<T>::load(fb + (size_t(step) * 2 + j) * Frag<T>::bytes, lane, g[j].w, g[j].sc);
-            else Rows<T>::load(row[j], step, half, g[j].g);
+            const int r = GATEUP ? 32 * c + col : 64 * c + 32 * j + col;
+            const size_t frags = size_t(GATEUP ? 2 : 1) * a.rows / 32 * nk * Frag<T>::bytes;
+            rs[j] = __uint_as_float(ld_u32(M0 + frags + 4 * (GATEUP ? j * a.rows + r : r)));
         }
-    };
+    }
 
     f32x16 acc[FI][2];
 #pragma unroll
@@ -220,137 +219,230 @@ VH_DEV void gemm_tile(TileLds<GATEUP, LDB> &L, const GemmArgs &a, gbyte *M0, gby
             for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
 
     // The operands of sub-step ks + 1 are formed, and its input fragments read,
-    // between the multiplies of sub-step ks (across the step's barrier too: the
-    // inputs of step s + 1 have been in LDS since the barrier before), so a
-    // wave's vector instructions run in the shadow of its own multiplies.
+    // between the multiplies of sub-step ks (across the step's barrier too where
+    // there are three input buffers: the inputs of step s + 1 have been in LDS
+    // since the barrier before), so a wave's vector instructions run in the shadow
+    // of its own multiplies.
+    constexpr int NB = TileLds<T, GATEUP, LDB, PK>::NB, AHEAD = NB - 1;
     int rowe = 0;  // down, threads 2 r and 2 r + 1: row r's exponent
-    f16x8 af[FI], b[2];
-    Words wd[2];
-    auto words = [&](Set (&g)[2], int s) {
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            if constexpr (PK) wd[j] = g[j];
-            else Rows<T>::words(g[j].g, s, half, up[j], wd[j].w, wd[j].sc);
-        }
-    };
-    // GGUF rows: a row's power of two follows from its first step's bound (below
-    // 2^11 under it) and is lowered, with what the row has accumulated, where a
-    // later bound would pass 2^15 under it: no pass over the row's scales ahead.
-    // Powers of two are exact, so the results are those of the packed copy's.
-    float fix[2];
-    auto row_bound = [&](Set &g) {  // of the row's step: both halves' (a finite bound, or 0)
-        if constexpr (PK) {
-            return 0.0f;
-        } else {
-            const float b = Rows<T>::step_bound(g.g), o = T == VT_Q8_0 ? __shfl_xor(b, 32, 64) : b;
-            return fmaxf(b, o);
-        }
-    };
-    auto rescale = [&](Set (&g)[2]) {
-        if constexpr (!PK) {
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                const float bnd = row_bound(g[j]);
-                const float to = bnd * up[j] >= 32768.0f ? ldexpf(1.0f, exponent_for(bnd) - 3) : up[j];
-                fix[j] = to / up[j];
-                up[j] = to;
-            }
-        }
-    };
+    f16x8 af[FI], b[2], bn[2];
     auto readA = [&](int buf, int ks, int i) {
         const int kg = 4 * half + ks;
         af[i] = L.As[buf][kg][(col ^ kg) + 32 * i];
     };
-    auto step = [&](int s, int b0, int b1, int b2, Set (&cur)[2], Set (&nxt)[2]) {
+    // step s's start: the inputs of step s + AHEAD into buffer `buf`, the next ones requested
+    auto stage_inputs = [&](int s, int buf) {
         if constexpr (!GATEUP)
-            if ((s + 2) % (kFacBlocks / 2) == 0 && s + 2 < nk) {  // the next blocks' factors (every 16 steps)
+            if ((s + AHEAD) % (kFacBlocks / 2) == 0 && s + AHEAD < nk) {  // the next blocks' factors (every 16 steps)
                 lds_barrier();
-                factors(2 * (s + 2), rowe);
+                factors(2 * (s + AHEAD), rowe);
                 lds_barrier();
             }
-        storeA(b2, s + 2);
-        loadA(min(s + 3, nk - 1));
+        storeA(buf, s + AHEAD);
+        loadA(min(s + AHEAD + 1, nk - 1));
         __builtin_amdgcn_sched_barrier(0);  // the loads stay where they are issued
+    };
+    // sub-step ks of a step in buffer b0, the next step's in b1
+    auto multiply = [&](int ks, int b0, int b1) {
 #pragma unroll
-        for (int ks = 0; ks < 4; ks++) {
-            if (ks == 3) {
-                __builtin_amdgcn_sched_barrier(0);
-                if constexpr (PK) loadB(cur, min(s + 2, nk - 1));
-                __builtin_amdgcn_sched_barrier(0);
-                rescale(nxt);
-                words(nxt, min(s + 1, nk - 1));
-                if constexpr (!PK) {
+        for (int i = 0; i < FI; i++) {
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], b[j], acc[i][j], 0, 0, 0);
+            if (NB == 3 || ks < 3) readA(ks < 3 ? b0 : b1, (ks + 1) & 3, i);
+        }
+        b[0] = bn[0];
+        b[1] = bn[1];
+#pragma unroll
+        for (int i = 0; i < 2 * FI; i++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                    // a multiply
+            __builtin_amdgcn_sched_group_barrier(0x002, 20 / FI, 0);      // vector instructions
+            if (i & 1) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);         // an LDS read
+        }
+    };
+    auto end_step = [&](int b1) {
+        lds_barrier();
+        if constexpr (NB == 2)
+#pragma unroll
+            for (int i = 0; i < FI; i++) readA(b1, 0, i);
+    };
+    auto first_inputs = [&] {
+        loadA(0);
+        if constexpr (!GATEUP) {
+            rowe = factors(0, 0);
+            lds_barrier();
+        }
+        storeA(0, 0);
+        loadA(min(1, nk - 1));
+        if constexpr (NB == 3) {
+            storeA(1, 1);
+            loadA(min(2, nk - 1));
+        }
+        lds_barrier();
+#pragma unroll
+        for (int i = 0; i < FI; i++) readA(0, 0, i);
+    };
+    auto next = [](int buf) { return buf == NB - 1 ? 0 : buf + 1; };
+    // K is a multiple of 128 (vh_mfma_supported): an even number of steps
+    if constexpr (PK) {
+        struct Words {
+            uint32_t w[O::NW], sc;
+        } st[2][2], wd[2];
+        auto loadB = [&](Words (&g)[2], int step) {
+#pragma unroll
+            for (int j = 0; j < 2; j++) Frag<T>::load(fb + (size_t(step) * 2 + j) * Frag<T>::bytes, lane, g[j].w, g[j].sc);
+        };
+        auto step = [&](int s, int b0, int b1, int b2, Words (&cur)[2], Words (&nxt)[2]) {
+            stage_inputs(s, b2);
+#pragma unroll
+            for (int ks = 0; ks < 4; ks++) {
+                if (ks == 3) {
                     __builtin_amdgcn_sched_barrier(0);
-                    loadB(nxt, min(s + 2, nk - 1));
+                    loadB(cur, min(s + 2, nk - 1));
                     __builtin_amdgcn_sched_barrier(0);
+                    wd[0] = nxt[0];
+                    wd[1] = nxt[1];
+                }
+#pragma unroll
+                for (int j = 0; j < 2; j++) bn[j] = O::get(wd[j].w, wd[j].sc, (ks + 1) & 3, cst);
+                multiply(ks, b0, b1);
+            }
+            end_step(b1);
+        };
+        loadB(st[0], 0);
+        loadB(st[1], min(1, nk - 1));
+        first_inputs();
+        wd[0] = st[0][0];
+        wd[1] = st[0][1];
+#pragma unroll
+        for (int j = 0; j < 2; j++) b[j] = O::get(wd[j].w, wd[j].sc, 0, cst);
+        for (int s = 0, b0 = 0; s < nk; s += 2) {
+            const int b1 = next(b0), b2 = next(b1);
+            step(s, b0, b1, b2, st[0], st[1]);
+            step(s + 1, b1, b2, b0, st[1], st[0]);
+            b0 = b2;
+        }
+    } else {
+        using S = Staged<T>;
+        typename S::Lds &R = L.rows[wv];
+        typename S::Regs g;
+        float up[S::NU], fix[S::NU], bnd[S::NU];
+        const int64_t r0 = GATEUP ? 32 * c : 64 * c;
+        gbyte *const B[2] = {M0 + r0 * a.row_bytes, GATEUP ? M1 + r0 * a.row_bytes : M0 + (r0 + 32) * a.row_bytes};
+        uint32_t w[2][2][4], sc[2], d[2];  // [half of the step's words][fragment]; the scales (PER_STEP: of the next d)
+        auto put = [&] {  // other lanes' reads of the last pair lie before, those of this one after
+            wave_fence();
+            if constexpr (S::PER_STEP) S::put(R, g, lane);
+            else S::put(R, g, up, lane);
+            wave_fence();
+        };
+        auto fetch = [&](int p, int i) {
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                if constexpr (S::PER_STEP) S::fetch(R, p, i, j, half, col, w[i][j], d[j]);
+                else S::fetch(R, p, i, j, half, col, w[i][j]);
+            }
+        };
+        // the scales of step p, whose first words are there: under the rows' powers of two
+        auto scales = [&](int p, bool first) {
+            bool any = false;
+            if constexpr (S::PER_STEP) {
+                auto scale = [&](int j) { return h_bits(h2f(d[j]) * up[j]); };
+                if (first) {
+#pragma unroll
+                    for (int j = 0; j < 2; j++) up[j] = first_up(S::step_bound(d[j]));
+                }
+                sc[0] = scale(0);
+                sc[1] = scale(1);
+                // fp16 256 or more: 128 times it passes 2^15
+                if (!first && __any((sc[0] & 0x7fffu) >= 0x5c00u || (sc[1] & 0x7fffu) >= 0x5c00u)) {
+                    bnd[0] = S::step_bound(d[0]);
+                    bnd[1] = S::step_bound(d[1]);
+                    any = lower_up(bnd, up, fix);
+                    sc[0] = scale(0);
+                    sc[1] = scale(1);
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < 2; j++) sc[j] = reinterpret_cast<const uint32_t *>(R.sc)[4 * (32 * j + col) + 2 * p + half];
+            }
+            return any;
+        };
+        auto operands = [&](f16x8 (&o)[2], int ks) {
+#pragma unroll
+            for (int j = 0; j < 2; j++) o[j] = S::get(w[ks >> 1][j][2 * (ks & 1)], w[ks >> 1][j][2 * (ks & 1) + 1], sc[j], ks, cst);
+        };
+        // step s, step p of its unit: the next step's first words are read (after
+        // the next unit is put in place) once its own last operand is formed
+        constexpr int N = 2;
+        const int units = nk / N;
+        auto step = [&](int s, auto P, int b0, int b1, int b2) {
+            constexpr int p = decltype(P)::value, q = (p + 1) % N;  // the next step's place in its unit
+            stage_inputs(s, b2);
+            bool any = false;
+#pragma unroll
+            for (int ks = 0; ks < 4; ks++) {
+                if (ks == 0) fetch(p, 1);
+                if (ks < 3) operands(bn, ks + 1);
+                if (ks == 2) {
+                    if (q == 0) {
+                        if constexpr (!S::PER_STEP) {
+                            S::bounds(g, bnd);
+                            any = lower_up(bnd, up, fix);
+                        }
+                        put();
+                        __builtin_amdgcn_sched_barrier(0);
+                        S::load(g, B, a.row_bytes, min(s / N + 2, units - 1), lane);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    fetch(q, 0);
+                }
+                if (ks == 3) {
+                    any |= scales(q, false);
+                    operands(bn, 0);
+                }
+                multiply(ks, b0, b1);
+            }
+            if (any) {
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    const float f = S::of_row(fix, j, col);
+#pragma unroll
+                    for (int i = 0; i < FI; i++)
+#pragma unroll
+                        for (int r = 0; r < 16; r++) acc[i][j][r] *= f;
                 }
             }
-            f16x8 bn[2];
-#pragma unroll
-            for (int j = 0; j < 2; j++) bn[j] = O::get(wd[j].w, wd[j].sc, (ks + 1) & 3, cst);
-#pragma unroll
-            for (int i = 0; i < FI; i++) {
-#pragma unroll
-                for (int j = 0; j < 2; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], b[j], acc[i][j], 0, 0, 0);
-                readA(ks < 3 ? b0 : b1, (ks + 1) & 3, i);
+            end_step(b1);
+        };
+        S::load(g, B, a.row_bytes, 0, lane);
+        first_inputs();
+        if constexpr (!S::PER_STEP) {
+            S::bounds(g, bnd);
+            up[0] = first_up(bnd[0]);
+        }
+        put();
+        S::load(g, B, a.row_bytes, min(1, units - 1), lane);
+        fetch(0, 0);
+        scales(0, true);
+        operands(b, 0);
+        const std::integral_constant<int, 0> even;
+        const std::integral_constant<int, N - 1> odd;
+        for (int s = 0, b0 = 0; s < nk; s += 2) {
+            if constexpr (NB == 2) {
+                step(s, even, 0, 1, 1);
+                step(s + 1, odd, 1, 0, 0);
+            } else {
+                const int b1 = next(b0), b2 = next(b1);
+                step(s, even, b0, b1, b2);
+                step(s + 1, odd, b1, b2, b0);
+                b0 = b2;
             }
-            b[0] = bn[0];
-            b[1] = bn[1];
-#pragma unroll
-            for (int i = 0; i < 2 * FI; i++) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                    // a multiply
-                __builtin_amdgcn_sched_group_barrier(0x002, 20 / FI, 0);      // vector instructions
-                if (i & 1) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);         // an LDS read
-            }
         }
-        if constexpr (!PK) {
-            if (__any(fix[0] != 1.0f || fix[1] != 1.0f))
 #pragma unroll
-                for (int i = 0; i < FI; i++)
-#pragma unroll
-                    for (int j = 0; j < 2; j++)
-#pragma unroll
-                        for (int r = 0; r < 16; r++) acc[i][j][r] *= fix[j];
-        }
-        lds_barrier();
-    };
-    loadB(st[0], 0);
-    if constexpr (PK) loadB(st[1], min(1, nk - 1));
-    loadA(0);
-    if constexpr (!GATEUP) {
-        rowe = factors(0, 0);
-        lds_barrier();
-    }
-    storeA(0, 0);
-    loadA(min(1, nk - 1));
-    storeA(1, 1);
-    loadA(min(2, nk - 1));
-    lds_barrier();
-    if constexpr (!PK)
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const float bnd = row_bound(st[0][j]);
-            up[j] = ldexpf(1.0f, bnd > 0.0f ? exponent_for(bnd) - 3 : 14);
-        }
-    words(st[0], 0);
-    if constexpr (!PK) loadB(st[0], min(1, nk - 1));
-#pragma unroll
-    for (int i = 0; i < FI; i++) readA(0, 0, i);
-#pragma unroll
-    for (int j = 0; j < 2; j++) b[j] = O::get(wd[j].w, wd[j].sc, 0, cst);
-    // K is a multiple of 128 (vh_mfma_supported): an even number of steps
-    for (int s = 0, b0 = 0; s < nk; s += 2) {
-        const int b1 = b0 == 2 ? 0 : b0 + 1, b2 = b1 == 2 ? 0 : b1 + 1;
-        step(s, b0, b1, b2, st[0], st[PK ? 1 : 0]);
-        step(s + 1, b1, b2, b0, st[PK ? 1 : 0], st[0]);
-        b0 = b2;
+        for (int j = 0; j < 2; j++) rs[j] = 1.0f / S::of_row(up, j, col);
     }
 
-    if constexpr (!PK) {
-        rs[0] = 1.0f / up[0];
-        rs[1] = 1.0f / up[1];
-    }
     // epilogue: the lane holds column `col` of each fragment, rows 8 (r / 4) +
     // 4 half + r % 4 of each 32-row block
     const int r0 = base + m0;
@@ -388,9 +480,7 @@ VH_DEV void gemm_tile(TileLds<GATEUP, LDB> &L, const GemmArgs &a, gbyte *M0, gby
                 L.hsc[wv][rl] = __uint_as_float(uint32_t(127 + 14 - max(e, -100)) << 23);
                 if (32 * i + rl < mcnt) a.he[size_t(r0 + 32 * i + rl) * (a.rows / 32) + c] = int8_t(e);
             }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            wave_fence();
             auto *hs = (__attribute__((address_space(1))) char *)a.out + (size_t(r0 + 32 * i) * a.rows + 32 * c) * 2;
             const uint32_t ho = uint32_t(4 * half * a.rows + col) * 2u;
 #pragma unroll
@@ -428,7 +518,7 @@ VH_DEV void gemm_tile(TileLds<GATEUP, LDB> &L, const GemmArgs &a, gbyte *M0, gby
 template <int T, bool GATEUP, int BMAX, bool PK>
 __global__ void __launch_bounds__(kThreads, BMAX == kBigTile || !PK ? 2 : 3) mfma_gemm_kernel(GemmArgs a) {
     constexpr int NCOL = GATEUP ? kBRows / 2 : kBRows;  // output columns per workgroup
-    __shared__ TileLds<GATEUP, BMAX> lds;
+    __shared__ TileLds<T, GATEUP, BMAX, PK> lds;
     const int nct = a.rows / NCOL, xcd = blockIdx.x % kXcds, slot = blockIdx.x / kXcds;
     const int32_t *run = a.tiles + (GATEUP ? kPlanRunsGU : kPlanRunsDN);
     const int at = run[xcd] + slot;
@@ -616,8 +706,14 @@ __global__ void __launch_bounds__(256) mfma_plan_kernel(const int32_t *__restric
 // groups. Measured per layer with tiles of up to 64 / 128 rows: OLMoE Q4_K_M 512
 // tokens (64 per expert) 205 / 236 us, Qwen3 Q8_0 2048 tokens (128 per expert,
 // Zipf) 424 / 421 us, Qwen3 Q4_K_M 4093 tokens (256 per expert) 705 / 667 us.
-constexpr int kBigAverage = 100;
-int tile_rows(int P, int E) { return P >= kBigAverage * E ? kBigTile : kSmallTile; }
+// GGUF rows, whose weights cost more to form and whose kernels keep two waves
+// either way, from 70: Qwen3 Q8_0 1024 tokens (64 per expert) 382 / 384 us, 1200
+// (75) 437 / 420, 1500 (94) 468 / 396; OLMoE Q8_0 512 (64) 274 / 291.
+constexpr int kBigAverage = 100, kBigAverageRows = 70;
+int tile_rows(int P, int E, bool packed) {
+    return P >= (packed ? kBigAverage : kBigAverageRows) * E ? kBigTile : kSmallTile;
+}
+int max_tiles(int P, int E, bool packed) { return P / tile_rows(P, E, packed) + E; }
 
 // The column tiles, weight bytes per K step and workgroup slots per XCD of a
 // launch: an eighth more than an XCD's share of the most pairs there can be
@@ -626,11 +722,11 @@ int tile_rows(int P, int E) { return P >= kBigAverage * E ? kBigTile : kSmallTil
 struct TileCost {
     int nct, wb, slots;
 };
-TileCost tile_cost(uint32_t type, int K, int rows, bool gateup, int P, int E) {
+TileCost tile_cost(uint32_t type, int K, int rows, bool gateup, int P, int E, bool packed) {
     TileCost c;
     c.nct = rows / (gateup ? kBRows / 2 : kBRows);
     c.wb = int(int64_t(kBRows) * vh_row_bytes(type, K) * kBK / K);  // a multiple of 64 for these types
-    const int64_t per = (int64_t(vh_mfma_max_tiles(P, E)) * c.nct + kXcds - 1) / kXcds;
+    const int64_t per = (int64_t(max_tiles(P, E, packed)) * c.nct + kXcds - 1) / kXcds;
     c.slots = int(per + per / 8 + 1);
     return c;
 }
@@ -646,8 +742,8 @@ void launch_gemm(const GemmArgs &a, const dim3 &g, bool big, bool packed, hipStr
 
 template <bool GATEUP>
 int gemm(uint32_t type, int P, int E, bool packed, const GemmArgs &a, hipStream_t s) {
-    const dim3 g(unsigned(tile_cost(type, a.K, a.rows, GATEUP, P, E).slots) * kXcds);
-    const bool big = tile_rows(P, E) == kBigTile;
+    const dim3 g(unsigned(tile_cost(type, a.K, a.rows, GATEUP, P, E, packed).slots) * kXcds);
+    const bool big = tile_rows(P, E, packed) == kBigTile;
     switch (type) {
     case VT_Q8_0: launch_gemm<VT_Q8_0, GATEUP>(a, g, big, packed, s); break;
     case VT_Q4_K: launch_gemm<VT_Q4_K, GATEUP>(a, g, big, packed, s); break;
@@ -666,19 +762,17 @@ bool vh_mfma_supported(uint32_t tg, uint32_t td, int d, int fe, int E) {
            d % kBK == 0 && fe % kBK == 0 && E <= 256;
 }
 
-int vh_mfma_max_tiles(int P, int E) { return P / tile_rows(P, E) + E; }
+int vh_mfma_plan_words(int P, int E) { return kPlanHead + 4 * std::max(max_tiles(P, E, true), max_tiles(P, E, false)); }
 
-int vh_mfma_plan_words(int P, int E) { return kPlanHead + 4 * vh_mfma_max_tiles(P, E); }
-
-int vh_mfma_plan(const int32_t *counts, const int32_t *offs, int E, int T, int k, uint32_t tg, uint32_t td, int d, int fe, int32_t *tiles,
-                 const float *hb, void *xb, float *xsc, hipStream_t s) {
+int vh_mfma_plan(const int32_t *counts, const int32_t *offs, int E, int T, int k, uint32_t tg, uint32_t td, int d, int fe,
+                 bool packed, int32_t *tiles, const float *hb, void *xb, float *xsc, hipStream_t s) {
     if (E > 256 || d % 4 || ((reinterpret_cast<uintptr_t>(hb) | reinterpret_cast<uintptr_t>(xb)) & 15u)) return -EINVAL;
-    const int P = T * k, mt = vh_mfma_max_tiles(P, E);
-    const TileCost gu = tile_cost(tg, d, fe, true, P, E), dn = tile_cost(td, fe, d, false, P, E);
+    const int P = T * k, mt = max_tiles(P, E, packed);
+    const TileCost gu = tile_cost(tg, d, fe, true, P, E, packed), dn = tile_cost(td, fe, d, false, P, E, packed);
     // the plan's costs are 32-bit sums over every (tile, column tile) pair
     if (int64_t(mt) * std::max(gu.nct, dn.nct) * tile_step_cost(std::max(gu.wb, dn.wb), kBigTile) > INT32_MAX)
         return -E2BIG;
-    hipLaunchKernelGGL(mfma_plan_kernel, dim3(1 + unsigned((T + 3) / 4)), dim3(256), 0, s, counts, offs, E, tile_rows(P, E),
+    hipLaunchKernelGGL(mfma_plan_kernel, dim3(1 + unsigned((T + 3) / 4)), dim3(256), 0, s, counts, offs, E, tile_rows(P, E, packed),
                        gu.nct, gu.wb, gu.slots, dn.nct, dn.wb, dn.slots, tiles, hb, static_cast<_Float16 *>(xb), xsc,
                        T, d);
     return vh_check(hipGetLastError());

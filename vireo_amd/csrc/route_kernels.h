@@ -203,11 +203,11 @@ int vh_q8dec(const void *const *table, bool packed, const void *xp, const float 
 constexpr int kMfmaMinCall = 64;
 bool vh_mfma_supported(uint32_t tg, uint32_t td, int d, int fe, int E);
 constexpr int kPlanRunsGU = 1, kPlanRunsDN = 10, kPlanHead = 20;  // offsets in the tile plan
-int vh_mfma_max_tiles(int P, int E);
 int vh_mfma_plan_words(int P, int E);
-int vh_mfma_plan(const int32_t *counts, const int32_t *offs, int E, int T, int k, uint32_t tg, uint32_t td, int d, int fe, int32_t *tiles,
-                 const float *hb, void *xb, float *xsc, hipStream_t s);
-// `packed`: table points at vh_mfma_pack's fragments. P pairs, E experts as in the plan.
+// `packed`: the table points at vh_mfma_pack's fragments (for the plan and both launches).
+int vh_mfma_plan(const int32_t *counts, const int32_t *offs, int E, int T, int k, uint32_t tg, uint32_t td, int d, int fe,
+                 bool packed, int32_t *tiles, const float *hb, void *xb, float *xsc, hipStream_t s);
+// P pairs, E experts as in the plan.
 int vh_mfma_gateup(uint32_t type, const int32_t *tiles, int P, int E, const int32_t *perm,
                    const void *const *table, bool packed, const void *xb, const float *xsc, int d,
                    int fe, int k, void *hs, int8_t *he, hipStream_t s);
