@@ -214,6 +214,12 @@ VH_DEV void lds_barrier() {
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
+// Orders the lanes' LDS accesses within a wave (the hardware keeps their order).
+VH_DEV void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 // Sum over aligned groups of L lanes (L a power of two <= 64). The total is in
 // the last lane of each group (lane % L == L-1); for L <= 16 every lane of the
 // group holds it. Must be called with all 64 lanes active.

@@ -329,7 +329,7 @@ struct Staged<VT_Q8_0> {
         uint4 q[8];
         uint2 tail;
     };
-    struct Lds {
+    struct __align__(16) Lds {  // stores of 8 bytes that straddle them take eight times as long
         uint32_t q[64 * 34];
     };
     static VH_DEV void load(Regs &r, gbyte *const (&B)[2], int64_t rb, int t, int lane) {

@@ -62,11 +62,12 @@ constexpr int kMdecMinTokens = 3;
 constexpr int kDecodeBatchAuto = 4;
 
 // From this many tokens on, calls on Q8_0 layers run on the matrix cores
-// (moe_q8dec.hip), below on the decode plan for every token. Measured per layer
-// (decode plan / matrix cores): OLMoE Q8_0 4 tokens 84.6 / 87.5 us, 6 84.3 / 91.9, 8
-// 111 / 98.6; Qwen3 Q8_0 6 tokens 73.7 / 86.3, 8 90.7 / 91.8. Against the fp32
-// grouped kernels before: OLMoE 23 tokens 175 -> 117, 63 tokens 341 -> 171; Qwen3 12
-// tokens 157 -> 116, 40 tokens 288 -> 193.
+// (moe_q8dec.hip), below on the decode plan for every token, which ends at 8.
+// Measured per layer (decode plan / matrix cores on the fragment copy): OLMoE Q8_0 4
+// tokens 84.6 / 87.5 us, 6 84.3 / 91.9, 8 111 / 98.6; Qwen3 Q8_0 6 tokens 73.7 / 86.3,
+// 8 90.7 / 91.8. The fp32 grouped kernels / the matrix cores on the copy / on GGUF
+// rows: OLMoE 9 tokens 127 / 94 / 125 us, 23 169 / 111 / 139, 63 335 / 160 / 198; Qwen3 9
+// 118 / 84 / 111, 16 183 / 133 / 168, 32 237 / 165 / 212, 63 364 / 193 / 227.
 constexpr int kQ8decMinTokens = 9;
 
 bool type_ok(uint32_t t, int n) {

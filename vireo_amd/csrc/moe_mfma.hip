@@ -85,13 +85,6 @@ VH_DEV void fold(float (&m)[16], bool hi) {
     }
 }
 
-// orders the lanes' LDS accesses within a wave (the hardware keeps their order)
-VH_DEV void wave_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // 2^n as fp16 bits, n <= 0 (0 below 2^-24)
 VH_DEV uint32_t h_pow2(int n) { return n >= -14 ? uint32_t(15 + n) << 10 : n >= -24 ? 1u << (24 + n) : 0u; }
 

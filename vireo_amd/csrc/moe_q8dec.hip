@@ -3,7 +3,7 @@
 // convert and multiply every weight again for each token of its expert and are
 // bound by the vector ALUs (23 OLMoE tokens: 104 + 54 us per layer, where reading
 // the experts takes 80); here a weight becomes a matrix operand once for up to 32
-// tokens: 56 + 45 us, gate/up at 4.8 TB/s, down at 3 (its arrivals and the combine
+// tokens: 54 + 43 us, gate/up at 5 TB/s, down at 3 (its arrivals and the combine
 // are a tail of round trips).
 //
 // v_mfma_f32_16x16x32_f16: 16 tokens x 16 weight rows x one block of 32 weights.
@@ -28,6 +28,7 @@
 // token's k experts to write a workgroup's rows adds them into x in selection
 // order, as mdec_down_kernel (moe_mdec.hip) does.
 #include <hip/hip_runtime.h>
+#include <type_traits>
 #include "common.h"
 #include "expert_group.h"
 #include "mfma_frag.h"
@@ -40,8 +41,10 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 constexpr int kTok = 16;                  // tokens per matrix tile; NT of them per pass over the weights
 
+template <bool PK>
 struct Q8Lds {
     int list[kGroupMax], wc[4], last[kGroupMax + 1];
+    std::conditional_t<PK, int, Staged<VT_Q8_0>::Lds> rows[4];  // a wave's GGUF rows
 };
 
 VH_DEV void swap32(uint32_t &a, uint32_t &b) {  // a's upper 32 lanes with b's lower
@@ -71,13 +74,16 @@ VH_DEV f16x8 q8_operand(uint32_t w0, uint32_t w1, uint32_t kb) {
 // acc[j][h][n]: rows 16 h .. + 15 of fragment j times the tokens 16 n .. of the
 // pass (lane l: row l % 16, tokens 4 (l / 16) .. + 3). A row of x is K x 4 bytes
 // (chunks of 8 inputs: hi parts, then lo); row_of(i) is the pass's token i's.
-// hs (down): the scales of h per row and block. Nothing passes through LDS: a
-// wave reads its inputs' operands itself, with its weights (the other waves'
-// reads of the same lines hit the L1), so no barrier ties its stream to theirs
-// (inputs staged for the workgroup: gate/up 75 us at 23 OLMoE tokens).
-template <bool PK, bool DOWN, int NT, class RowOf>
-VH_DEV void q8_stream(gbyte *F, gbyte *R0, gbyte *R1, const void *x, const float *hs, int K, int tn, RowOf row_of,
-                      f32x4 (&acc)[2][2][NT]) {
+// hs (down): the scales of h per row and block. A wave reads its inputs' operands
+// itself, with its weights (the other waves' reads of the same lines hit the
+// L1), so no barrier ties its stream to theirs (inputs staged for the workgroup:
+// gate/up 75 us at 23 OLMoE tokens). GGUF rows (rows0, rows1: the fragments' first)
+// pass through the wave's own LDS: with a row per lane a load instruction touched
+// 64 lines, Qwen3 16 tokens gate/up 166 -> 95 us, down 78 -> 56 (the fp32 kernels
+// 101 and 61, from the copy 67 and 48).
+template <bool PK, bool DOWN, int NT, class Area, class RowOf>
+VH_DEV void q8_stream(gbyte *F, gbyte *rows0, gbyte *rows1, Area &lds, const void *x, const float *hs, int K, int tn,
+                      RowOf row_of, f32x4 (&acc)[2][2][NT]) {
     constexpr int SETS = NT == 1 ? 4 : 2;  // K steps of weights in flight; of inputs (from the L2), two
     const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4, half = lane >> 5, nk = K / kBK;
     uint32_t kb = 0x64646464u;
@@ -92,26 +98,21 @@ VH_DEV void q8_stream(gbyte *F, gbyte *R0, gbyte *R1, const void *x, const float
             for (int i = 0; i < 4; i++)
                 sr[n][i] = uint32_t(row_of(min(16 * n + 4 * g + i, tn - 1))) * uint32_t(K / 32) * 4u;
     }
+    using S = Staged<VT_Q8_0>;
     struct Set {
         uint32_t w[2][8], d[2];
-    } st[SETS];
+    } st[PK ? SETS : 1];
+    typename S::Regs rg[PK ? 1 : SETS / 2];  // pairs of steps in flight
+    gbyte *const B[2] = {rows0, rows1};
+    const int64_t rb = int64_t(K / 32) * 34;
     struct In {
         uint4 h[2][NT], l[2][NT];
         uint2 sc[DOWN ? NT : 1][4];
     } in[2];
     auto load = [&](Set &q, int s) {
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            if constexpr (PK) {
-                Frag<VT_Q8_0>::load(F + (size_t(s) * 2 + j) * Frag<VT_Q8_0>::bytes, lane, q.w[j], q.d[j]);
-            } else {
-                Rows<VT_Q8_0>::Raw w;
-                Rows<VT_Q8_0>::load(j ? R1 : R0, s, half, w);
-#pragma unroll
-                for (int i = 0; i < 8; i++) q.w[j][i] = u4_at(w.q[i >> 2], i & 3);
-                q.d[j] = w.d;
-            }
-        }
+        for (int j = 0; j < 2; j++)
+            Frag<VT_Q8_0>::load(F + (size_t(s) * 2 + j) * Frag<VT_Q8_0>::bytes, lane, q.w[j], q.d[j]);
     };
     auto load_in = [&](In &q, int s) {
 #pragma unroll
@@ -127,7 +128,10 @@ VH_DEV void q8_stream(gbyte *F, gbyte *R0, gbyte *R1, const void *x, const float
         }
     };
 #pragma unroll
-    for (int i = 0; i < SETS; i++) load(st[i], min(i, nk - 1));
+    for (int i = 0; i < (PK ? SETS : SETS / 2); i++) {
+        if constexpr (PK) load(st[i], min(i, nk - 1));
+        else S::load(rg[i], B, rb, min(i, nk / 2 - 1), lane);
+    }
 #pragma unroll
     for (int i = 0; i < 2; i++) load_in(in[i], min(i, nk - 1));
 #pragma unroll
@@ -149,12 +153,38 @@ VH_DEV void q8_stream(gbyte *F, gbyte *R0, gbyte *R1, const void *x, const float
         for (int h = 0; h < 2; h++)
 #pragma unroll
             for (int n = 0; n < (DOWN ? 1 : NT); n++) tot[j][h][n] = f64x4{0., 0., 0., 0.};
+    // pair s / 2 of GGUF rows into place; other lanes' reads of the last lie before, those of this one after
+    auto place = [&](int s, typename S::Regs &r) {
+        if constexpr (!PK) {
+            wave_fence();
+            S::put(lds, r, lane);
+            wave_fence();
+        }
+    };
+    auto request = [&](int s, typename S::Regs &r) {
+        if constexpr (!PK) {
+            __builtin_amdgcn_sched_barrier(0);
+            S::load(r, B, rb, min(s / 2 + SETS / 2, nk / 2 - 1), lane);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
     auto step = [&](int s, Set &t, In &x, bool first) {
 #pragma unroll
         for (int j = 0; j < 2; j++) {
-            uint32_t q[8];
+            uint32_t q[8], dj;
+            if constexpr (PK) {
 #pragma unroll
-            for (int i = 0; i < 8; i++) q[i] = PK ? t.w[j][i] : t.w[j][i] ^ 0x80808080u;
+                for (int i = 0; i < 8; i++) q[i] = t.w[j][i];
+                dj = t.d[j];
+            } else {
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    uint32_t w[4];
+                    S::fetch(lds, s & 1, i, j, half, lane & 31, w, dj);
+#pragma unroll
+                    for (int k = 0; k < 4; k++) q[4 * i + k] = w[k];
+                }
+            }
             swap32(q[0], q[4]);
             swap32(q[1], q[5]);
             swap32(q[2], q[6]);
@@ -163,7 +193,7 @@ VH_DEV void q8_stream(gbyte *F, gbyte *R0, gbyte *R1, const void *x, const float
             swap16(q[1], q[3]);
             swap16(q[4], q[6]);
             swap16(q[5], q[7]);
-            uint32_t d0 = t.d[j], d2 = t.d[j];
+            uint32_t d0 = dj, d2 = dj;
             swap32(d0, d2);
             uint32_t d1 = d0, d3 = d2;
             swap16(d0, d1);
@@ -189,8 +219,10 @@ VH_DEV void q8_stream(gbyte *F, gbyte *R0, gbyte *R1, const void *x, const float
             }
         }
         __builtin_amdgcn_sched_barrier(0);
-        load(t, min(s + SETS, nk - 1));
+        // the inputs first: loads arrive in order, so the wait for them in two steps
+        // would include every load of weights issued before them
         load_in(x, min(s + 2, nk - 1));
+        if constexpr (PK) load(t, min(s + SETS, nk - 1));
         __builtin_amdgcn_sched_barrier(0);
     };
     auto add = [&] {
@@ -204,15 +236,20 @@ VH_DEV void q8_stream(gbyte *F, gbyte *R0, gbyte *R1, const void *x, const float
                     else tot[j][h][n] += __builtin_convertvector(sub[j][h][n], f64x4);
                 }
     };
-    for (int s = 0; s < nk; s += 4) {  // nk is even
-        step(s, st[0], in[0], true);
-        step(s + 1, st[1], in[1], false);
+    // steps s, s + 1 from set 2 `i`: the first of the sum where `first`
+    auto pair = [&](int s, auto I, bool first) {
+        constexpr int i = SETS == 4 ? decltype(I)::value : 0;
+        place(s, rg[PK ? 0 : i]);
+        step(s, st[PK ? 2 * i : 0], in[0], first);
+        step(s + 1, st[PK ? 2 * i + 1 : 0], in[1], false);
+        request(s, rg[PK ? 0 : i]);
         if (!DOWN) add();
-        if (s + 2 < nk) {
-            step(s + 2, st[SETS == 4 ? 2 : 0], in[0], !DOWN);
-            step(s + 3, st[SETS == 4 ? 3 : 1], in[1], false);
-            if (!DOWN) add();
-        }
+    };
+    const std::integral_constant<int, 0> i0;
+    const std::integral_constant<int, 1> i1;
+    for (int s = 0; s < nk; s += 4) {  // nk is even
+        pair(s, i0, true);
+        if (s + 2 < nk) pair(s + 2, i1, !DOWN);
         if (DOWN) add();
     }
     if constexpr (!DOWN)
@@ -244,12 +281,12 @@ VH_DEV float row_max(float v) {
 }
 
 template <bool PK, int NT>
-VH_DEV void gateup_pass(const Q8Lds &L, const Q8Args &a, gbyte *G, gbyte *U, int c, int t0, int tn) {
-    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4, col = lane & 31, nk = a.d / kBK;
+VH_DEV void gateup_pass(Q8Lds<PK> &L, const Q8Args &a, gbyte *G, gbyte *U, int c, int t0, int tn) {
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4, nk = a.d / kBK;
     const int64_t rb = int64_t(a.d / 32) * 34;
-    gbyte *row = G + int64_t(32 * c + col) * rb, *row1 = U + int64_t(32 * c + col) * rb;
     f32x4 acc[2][2][NT];
-    q8_stream<PK, false, NT>(G + size_t(c) * nk * 2 * Frag<VT_Q8_0>::bytes, row, row1, a.x, nullptr, a.d, tn,
+    q8_stream<PK, false, NT>(G + size_t(c) * nk * 2 * Frag<VT_Q8_0>::bytes, G + 32 * c * rb, U + 32 * c * rb, L.rows[c & 3],
+                             a.x, nullptr, a.d, tn,
                              [&](int i) { return L.list[t0 + i] / a.sf.k; }, acc);
     float rs[2][2] = {{1.0f, 1.0f}, {1.0f, 1.0f}};  // the rows' powers of two in the packed copy
     if constexpr (PK) {
@@ -290,7 +327,7 @@ VH_DEV void gateup_pass(const Q8Lds &L, const Q8Args &a, gbyte *G, gbyte *U, int
 
 template <bool PK, int NT>
 __global__ void __launch_bounds__(256, 2) q8dec_gateup_kernel(Q8Args a) {
-    __shared__ Q8Lds L;
+    __shared__ Q8Lds<PK> L;
     if (blockIdx.x == 0 && blockIdx.y == 0)  // the down kernel's counters start at 0
         for (int i = threadIdx.x; i < a.sf.nctr; i += 256) a.sf.ctr[i] = 0u;
     const int e = blockIdx.y, cnt = expert_group<256>(a.sf.idx, a.sf.T * a.sf.k, e, L.list, L.wc);
@@ -302,13 +339,13 @@ __global__ void __launch_bounds__(256, 2) q8dec_gateup_kernel(Q8Args a) {
 }
 
 template <bool PK, int NT>
-VH_DEV void down_pass(const Q8Lds &L, const Q8Args &a, gbyte *D, int c, int t0, int tn) {
-    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4, col = lane & 31, nk = a.fe / kBK;
+VH_DEV void down_pass(Q8Lds<PK> &L, const Q8Args &a, gbyte *D, int c, int t0, int tn) {
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4, nk = a.fe / kBK;
     const int64_t rb = int64_t(a.fe / 32) * 34;
     f32x4 acc[2][2][NT];
     if (D) {
-        q8_stream<PK, true, NT>(D + size_t(c) * nk * 2 * Frag<VT_Q8_0>::bytes, D + int64_t(64 * c + col) * rb,
-                                D + int64_t(64 * c + 32 + col) * rb, a.x, a.hs, a.fe, tn,
+        q8_stream<PK, true, NT>(D + size_t(c) * nk * 2 * Frag<VT_Q8_0>::bytes, D + 64 * c * rb, D + (64 * c + 32) * rb,
+                                L.rows[c & 3], a.x, a.hs, a.fe, tn,
                                 [&](int i) { return L.list[t0 + i]; }, acc);
     } else {  // an unregistered expert's rows are zeros, which the combine adds without changing a bit
 #pragma unroll
@@ -335,7 +372,7 @@ VH_DEV void down_pass(const Q8Lds &L, const Q8Args &a, gbyte *D, int c, int t0, 
 
 template <bool PK, int NT>
 __global__ void __launch_bounds__(256, 2) q8dec_down_kernel(Q8Args a) {
-    __shared__ Q8Lds L;
+    __shared__ Q8Lds<PK> L;
     constexpr int CR = 256;  // output rows of one workgroup
     const MdecSelf &sf = a.sf;
     const int tid = threadIdx.x, e = blockIdx.y, k = sf.k, d = a.d;
