@@ -129,7 +129,7 @@ def test_gguf_stack_matches_oracle(cuda, oracle, tmp_path, name, untied, cap_exp
 
 @pytest.mark.parametrize("name,cap_experts,T,L", [("tiny-k", 3, 5, 2), ("tiny-q8", 1, 3, 2), ("qwen3-16e", 4, 1, 2),
                                                  ("qwen3-16e", 5, 6, 2), ("qwen3-16e", 24, 1, 3),
-                                                 ("tiny-k", 12, 4, 3)])
+                                                 ("tiny-k", 12, 4, 3), ("tiny-q8", 3, 20, 2), ("tiny-q8", 12, 63, 3)])
 def test_gguf_paged_store(cuda, oracle, tmp_path, name, cap_experts, T, L):
     """Stores smaller than the model (down to one expert, and about one and
     a half layers of a 3-layer model): the pool stays within its capacity,

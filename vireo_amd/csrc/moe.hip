@@ -592,7 +592,10 @@ int paged_forward(const vireo_moe_model *m, int layer, float *x, const float *hb
     const bool exact = n_tokens >= kExactRouteTokens;
     const bool mdec = n_tokens >= kMdecMinTokens && n_tokens < kMfmaMinCall && g_path != 4 &&
                       vh_mdec_supported(tg, td, d, fe);
-    int rc = mdec ? vh_route_parts_tiled(R, hb, L.logit_bias, d, E, n_tokens, ws.parts, ws.xp, ws.xsc, s) : -EINVAL;
+    const bool q8dec = n_tokens >= kQ8decMinTokens && n_tokens < kMfmaMinCall && g_path != 4 &&
+                       vh_q8dec_supported(tg, td, d, fe, n_tokens);
+    int rc = mdec || q8dec ? vh_route_parts_tiled(R, hb, L.logit_bias, d, E, n_tokens, ws.parts, ws.xp, ws.xsc, s, q8dec)
+                           : -EINVAL;
     const bool prepped = rc == 0;
     if (rc == -EINVAL) rc = vh_route_parts(R, hb, L.logit_bias, d, E, n_tokens, exact, ws.parts, s);
     if (!rc) rc = vh_route_finish(ws.parts, R, hb, L.logit_bias, d, E, k, m->topk_renorm, exact, n_tokens, idx, w,
@@ -650,8 +653,8 @@ int paged_forward(const vireo_moe_model *m, int layer, float *x, const float *hb
     vh_store_note_routing_host(m->es, layer, idx_h, n_tokens, k);
     const uint64_t cap = vh_store_capacity(m->es), leased = vh_store_leased_bytes(m->es);
     const uint64_t room = cap > leased ? cap - leased : 1;  // cap 0: unbounded (room unused)
-    const bool gdec = !mdec && n_tokens < kMfmaMinCall && vh_gdec_supported(tg, td, d, fe, hb);
-    if (mdec && !prepped) rc = vh_mdec_prep(hb, n_tokens, d, ws.xp, ws.xsc, s);
+    const bool gdec = !mdec && !q8dec && n_tokens < kMfmaMinCall && vh_gdec_supported(tg, td, d, fe, hb);
+    if ((mdec || q8dec) && !prepped) rc = vh_mdec_prep(hb, n_tokens, d, ws.xp, ws.xsc, s, q8dec);
     const void **present = tabs_h + size_t(E) * tab_n;  // the combine's table (the last one)
     memset(present, 0, tab_n * sizeof(void *));
     ExpertView views[kMaxExperts];
@@ -696,6 +699,9 @@ int paged_forward(const vireo_moe_model *m, int layer, float *x, const float *hb
                                              fe, k, E, slots, n_tokens, ws.h, s);
                 if (!rc) rc = vh_mdec_down(ws.counts, ws.offs, ws.perm, da, dt, false, ws.h, d, fe, E, slots,
                                            n_tokens, ws.ybuf, s);
+            } else if (q8dec) {
+                const MdecSelf sf{idx, w, x, ws.ctr, vh_mdec_ctr_words(d), n_tokens, k};
+                if (!rc) rc = vh_q8dec(dt, false, ws.xp, ws.xsc, d, fe, E, ws.h, ws.hsc, ws.ybuf, sf, false, s);
             } else if (gdec) {
                 if (!rc) rc = vh_gdec_gateup(tg, ws.counts, ws.offs, ws.perm, da, dt, hb, d, fe, k, E, slots, n_tokens, ws.h, s);
                 if (!rc) rc = vh_gdec_down(td, ws.counts, ws.offs, ws.perm, da, dt, ws.h, d, fe, E, slots, n_tokens, ws.ybuf, s);
@@ -842,7 +848,7 @@ int ffn_forward(const vireo_moe_model *m, int layer, float *x, const float *hb, 
         // the prefill GEMMs' fragment copy where the layer has it or can make it
         const void *const *pt = rc ? nullptr : packed_table(m, layer, table, !src, s, 1);
         const MdecSelf sf{idx, w, x, ws.ctr, vh_mdec_ctr_words(d), n_tokens, k};
-        if (!rc) rc = vh_q8dec(pt ? pt : table, pt != nullptr, ws.xp, ws.xsc, d, fe, E, ws.h, ws.hsc, ws.ybuf, sf, s);
+        if (!rc) rc = vh_q8dec(pt ? pt : table, pt != nullptr, ws.xp, ws.xsc, d, fe, E, ws.h, ws.hsc, ws.ybuf, sf, true, s);
     } else if (n_tokens < kMfmaMinCall && vh_gdec_supported(tg, td, d, fe, hb)) {
         // calls of a decode batch's size (a few tokens per group): inputs in registers
         if (!rc) rc = vh_gdec_gateup(tg, ws.counts, ws.offs, ws.perm, ws.active, table, hb, d, fe, k, E, slots, n_tokens, ws.h, s);

@@ -269,6 +269,7 @@ struct Q8Args {
     float *hs;            // and their block scales [pairs x fe / 32]
     float *y;             // down: [pairs x d]
     int d, fe;
+    bool combine;         // down: x += the weighted rows; else rows only, those of the table's experts
     MdecSelf sf;
 };
 
@@ -379,8 +380,10 @@ __global__ void __launch_bounds__(256, 2) q8dec_down_kernel(Q8Args a) {
     const int cnt = expert_group<256>(sf.idx, sf.T * k, e, L.list, L.wc);
     if (cnt == 0) return;
     gbyte *D = gmem(a.table[3 * e + 2]);
+    if (!D && !a.combine) return;
     const int c = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(tid >> 6);
     for (int t0 = 0; t0 < cnt; t0 += NT * kTok) down_pass<PK, NT>(L, a, D, c, t0, min(NT * kTok, cnt - t0));
+    if (!a.combine) return;
     // the combine (src/gguf_run.c:208-212; see mdec_down_kernel): rows out as
     // agent-scope stores, one arrival per token once they are done, and the
     // workgroup that brings a token's count to k reads its k rows past the L2
@@ -431,11 +434,11 @@ bool vh_q8dec_supported(uint32_t tg, uint32_t td, int d, int fe, int T) {
 }
 
 int vh_q8dec(const void *const *table, bool packed, const void *xp, const float *xsc, int d, int fe, int E, void *hp,
-             float *hs, float *ybuf, const MdecSelf &self, hipStream_t s) {
+             float *hs, float *ybuf, const MdecSelf &self, bool combine, hipStream_t s) {
     if (!vh_q8dec_supported(VT_Q8_0, VT_Q8_0, d, fe, self.T) || self.T < 1 || self.k < 1 || !self.x || !self.w ||
         self.nctr < vh_mdec_ctr_words(d))
         return -EINVAL;
-    const Q8Args a{table, xp, xsc, static_cast<uint16_t *>(hp), hs, ybuf, d, fe, self};
+    const Q8Args a{table, xp, xsc, static_cast<uint16_t *>(hp), hs, ybuf, d, fe, combine, self};
     // two token tiles per pass where the average expert has more than half a tile (its registers keep two waves
     // per SIMD, one tile's four)
     if (2 * self.T * self.k > kTok * E) q8dec_launch<2>(a, packed, E, hp, s);

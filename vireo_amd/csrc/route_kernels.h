@@ -186,9 +186,11 @@ int vh_mdec_pack_layer(const void *const *table, int E, int d, int fe, void *buf
 // split inputs in natural order (`natural` there and in vh_route_parts_tiled);
 // hp [pairs x fe x 4 bytes] and hs [pairs x fe / 32] take the activations.
 // `packed`: table points at vh_mfma_pack's fragments (the same bits either way).
+// Without `combine` only the table's experts run and their rows go to ybuf, for
+// vh_combine once every batch of a paged call has run (the same bits again).
 bool vh_q8dec_supported(uint32_t tg, uint32_t td, int d, int fe, int T);
 int vh_q8dec(const void *const *table, bool packed, const void *xp, const float *xsc, int d, int fe, int E, void *hp,
-             float *hs, float *ybuf, const MdecSelf &self, hipStream_t s);
+             float *hs, float *ybuf, const MdecSelf &self, bool combine, hipStream_t s);
 
 // Matrix-core grouped GEMMs (moe_mfma.hip) for the groups of calls of at
 // least kMfmaMinCall tokens. vh_mfma_plan lists the groups' token tiles (32,
