@@ -235,17 +235,26 @@ int vireo_hip_set_path(int path);
  * bytes reordered so that every load instruction reads 1 KB of consecutive
  * memory; later calls read the copy. The copy (as much again as the layer's
  * expert bytes) counts against the store's capacity like resident experts:
- * it is made only while the resident experts and the copies fit the capacity
- * with it (cut from the pool's own device block when that has room), else
- * the calls read the GGUF rows; an unbounded store (capacity 0) always makes
- * it. expert_store_packed_bytes reports the copies' bytes. A copy is made
+ * it is made only while it fits the capacity (cut from the pool's own device
+ * block when that has room) beside the other copies and the resident experts
+ * - all of the model's experts in a store that can hold them, so that no copy
+ * keeps a layer from being pinned -, else the calls read the GGUF rows; an
+ * unbounded store (capacity 0) always makes it. expert_store_packed_bytes
+ * reports the copies' bytes. A copy is made
  * from the pinned views and freed with the pin (expert_store_unpin_layer) or
  * the store; a caller that rewrites a pinned layer's expert bytes in place
  * must unpin and pin it again. Calls of 64 or more tokens on a pinned layer of
  * Q8_0, Q4_K or Q6_K experts, and of 9 or more on Q8_0 experts, make and read,
  * the same way, a copy in matrix-operand fragments (each lane's words of a
  * 32-row, 64-column step together; 1.0, 1.1 and 1.07 times the expert bytes).
- * Results are the same bit for bit either way. 0 turns both off for later calls
+ * In a bounded store a layer's fragments are made only beside the tiles of
+ * every layer that may still make them: a Q4_K_M model makes every copy from
+ * about 3.1 times its experts' bytes on (an unbounded store grows to that), the
+ * tiles from twice, a Q8_0 model from twice. The call that makes a copy waits
+ * for the work before it in its stream.
+ * Results are the same bit for bit either way, for Q4_K and Q6_K fragments as
+ * long as a row's scales lie within 2^12 of its largest (below that a weight is
+ * held to 2^-25 to 2^-28 of the row's largest). 0 turns both off for later calls
  * (existing copies stay until unpinned). No counterpart in the reference. */
 int vireo_hip_set_packed(int on);
 

@@ -196,6 +196,81 @@ def test_packed_copy_counts_against_capacity(cuda, lib):
         m.close()
 
 
+def fragment_bytes(shape):
+    """A layer's fragment copy: 32 rows x 64 columns a fragment, then the rows' scales."""
+    fb = {W.Q4_K: 1280, W.Q6_K: 1792, W.Q8_0: 2176}
+    up = lambda v: (v + 255) // 256 * 256  # noqa: E731
+    return shape.E * (up(2 * shape.fe // 32 * (shape.d // 64) * fb[shape.gate_type] + 8 * shape.fe) +
+                      up(shape.d // 32 * (shape.fe // 64) * fb[shape.down_type] + 4 * shape.d))
+
+
+def tile_bytes(shape):
+    """A Q4_K_M layer's decode-batch tiles."""
+    return shape.E * (2 * (shape.fe // 16) * (shape.d // 256) * 2368 + shape.d * (shape.fe // 256 * 210))
+
+
+@pytest.mark.parametrize("types,first", [((W.Q4_K, W.Q6_K), 70), ((W.Q4_K, W.Q6_K), 8), ((W.Q8_0, W.Q8_0), 70),
+                                         ((W.Q8_0, W.Q8_0), 16)])
+def test_copies_leave_room(cuda, lib, types, first):
+    """A two-layer model in stores of every size that matters, its first calls
+    of `first` tokens and then of both sizes: both layers are pinned whatever the
+    capacity (no copy takes the room of the other layer's experts), Q4_K_M
+    layers' tiles go before their fragments, and every call gives the unbounded
+    store's bits."""
+    tg, td = types
+    shape = W.MoEShape("room", 2048, 8, 2, 256, True, tg, tg, td)
+    L, k4 = 2, tg == W.Q4_K
+    m = M.DeviceMoE(shape, L, seed=73)
+    gs, us, ds = m.slices
+    layer, frag, tile = m.layer_bytes, fragment_bytes(shape), tile_bytes(shape) if k4 else 0
+    x, hb = W.host_hidden(shape.d, 70, 73)
+    hbt = torch.from_numpy(hb).to(cuda)
+
+    def calls():
+        outs = []
+        for T in (first, 70, 16, 8):
+            for l in range(L):
+                xt = torch.from_numpy(x[:T].copy()).to(cuda)
+                m.forward(l, xt, hbt[:T])
+                outs.append(xt.cpu().numpy().view(np.uint32))
+        return outs
+
+    want = calls()
+    fd, path = tempfile.mkstemp()
+    os.unlink(path)
+    try:
+        for l in range(L):
+            os.pwrite(fd, np.concatenate(m.device_layer_bytes(l)).tobytes(), l * layer)
+        base = L * layer
+        sizes = [(base, 0), (base + L * tile + frag - 1, L * tile), (base + L * (tile + frag), L * (tile + frag)),
+                 (0, L * (tile + frag))]
+        if k4:
+            sizes += [(base + tile - 1, 0), (base + L * tile, L * tile), (base + L * tile + frag, L * tile + frag)]
+        else:
+            sizes += [(base + frag, frag)]
+        for cap, copies in sizes:
+            s = lib.expert_store_create(fd, cap, L, shape.E)
+            for l in range(L):
+                for e in range(shape.E):
+                    o = l * layer
+                    sl = _lib.ExpertSlices(o + e * gs, o + shape.E * gs + e * us, o + shape.E * (gs + us) + e * ds, gs, us, ds)
+                    lib.expert_store_register(s, l, e, C.byref(sl))
+            m.model.es = s
+            for got, ref in zip(calls(), want):
+                np.testing.assert_array_equal(got, ref, err_msg=f"capacity {cap}")
+            st = _lib.ExpertStats()
+            lib.expert_store_hbm_stats(s, C.byref(st))
+            print(f"capacity {cap - base:+d}: copies {lib.expert_store_packed_bytes(s)}")
+            assert lib.expert_store_packed_bytes(s) == copies, cap - base
+            assert st.resident_bytes == base + copies
+            torch.cuda.synchronize()
+            lib.expert_store_destroy(s)
+    finally:
+        os.close(fd)
+        m.model.es = m.es
+        m.close()
+
+
 @pytest.mark.parametrize("case", ["tiny_q4km", "tiny_q8", "olmoe_q8_0", "qwen3_q4_k_m"])
 def test_golden_store_stats(cuda, lib, case):
     """The reference's own ExpertStore statistics after its moe_ffn over the

@@ -862,12 +862,15 @@ const void *const *vh_store_layer_table(const ExpertStore *s, int layer) {
 }
 
 /* A pinned layer's experts reordered for a kernel (kind 0: the matrix-core
- * decode batch's 16-row tiles, 1: the prefill GEMMs' Q8_0 row octets): their
- * device table, or NULL (never allocates). A copy counts against the
- * capacity like resident experts: vh_store_packed_begin gives a device
- * block of `bytes` for one only while resident experts and copies fit the
- * capacity with it (else NULL, and the caller reads the GGUF rows), cut
- * from the pool's arena when it has room; vh_store_set_packed then hands
+ * decode batch's 16-row tiles, 1: matrix-operand fragments for the prefill GEMMs
+ * and the Q8_0 decode batch): their device table, or NULL (never allocates). A
+ * copy counts against the capacity like resident experts: vh_store_packed_begin
+ * gives a device block of `bytes` for one only while it leaves room for the
+ * copies, for `reserve` bytes of copies that go before it and for the experts:
+ * the resident ones, or in a store that holds the whole model all of them, so
+ * that no copy keeps a layer from being pinned (else NULL, and the caller
+ * reads the GGUF rows). The block is cut from the pool's arena when it has
+ * room; vh_store_set_packed then hands
  * the store the copy's device [n_experts x 3] table, or vh_store_packed_abort
  * takes the block back. The store frees both when the layer is unpinned or
  * the store destroyed. */
@@ -876,13 +879,17 @@ const void *const *vh_store_packed_table(const ExpertStore *s, int layer, int ki
         return NULL;
     return (const void *const *)s->ptables[(size_t)kind * s->n_layers + layer];
 }
-void *vh_store_packed_begin(ExpertStore *s, int layer, int kind, uint64_t bytes) {
+void *vh_store_packed_begin(ExpertStore *s, int layer, int kind, uint64_t bytes, uint64_t reserve) {
     if (!store_ok(s) || layer < 0 || layer >= s->n_layers || kind < 0 || kind >= VH_PACK_KINDS || !s->tables[layer] ||
         !bytes)
         return NULL;
     const size_t i = (size_t)kind * s->n_layers + layer;
     if (s->ptables[i] || s->pbufs[i]) return NULL;
-    if (s->capacity_bytes && s->resident_bytes + s->packed_bytes + bytes > s->capacity_bytes) return NULL;
+    if (s->capacity_bytes) {
+        uint64_t experts = s->resident_bytes;
+        if (s->registered_bytes <= s->capacity_bytes && s->registered_bytes > experts) experts = s->registered_bytes;
+        if (experts + s->packed_bytes + bytes + reserve > s->capacity_bytes) return NULL;
+    }
     void *p = NULL;
     for (int j = 0; j < s->nfree && !p; j++)
         if (s->freel[j].size == bytes) {

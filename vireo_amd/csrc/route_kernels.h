@@ -32,7 +32,7 @@ uint64_t vh_store_capacity(const ExpertStore *s);
 int vh_store_valid(const ExpertStore *s);
 const void *const *vh_store_layer_table(const ExpertStore *s, int layer);
 const void *const *vh_store_packed_table(const ExpertStore *s, int layer, int kind);
-void *vh_store_packed_begin(ExpertStore *s, int layer, int kind, uint64_t bytes);
+void *vh_store_packed_begin(ExpertStore *s, int layer, int kind, uint64_t bytes, uint64_t reserve);
 int vh_store_set_packed(ExpertStore *s, int layer, int kind, void *tab);
 void vh_store_packed_abort(ExpertStore *s, int layer, int kind);
 int vh_store_fits_all(const ExpertStore *s);
