@@ -252,9 +252,9 @@ int vireo_hip_set_path(int path);
  * about 3.1 times its experts' bytes on (an unbounded store grows to that), the
  * tiles from twice, a Q8_0 model from twice. The call that makes a copy waits
  * for the work before it in its stream.
- * Results are the same bit for bit either way, for Q4_K and Q6_K fragments as
- * long as a row's scales lie within 2^12 of its largest (below that a weight is
- * held to 2^-25 to 2^-28 of the row's largest). 0 turns both off for later calls
+ * Results are the same bit for bit either way, with fragments as long as a
+ * row's scales lie within 2^12 of its largest (smaller weights are held to 2^-28
+ * of the row's largest). 0 turns both off for later calls
  * (existing copies stay until unpinned). No counterpart in the reference. */
 int vireo_hip_set_packed(int on);
 

@@ -3,8 +3,9 @@ src/gguf_run.c:185-214, restated) and against the golden vectors the
 reference itself wrote, on both execution plans.
 
 Bar: the routed experts bit-exact; the layer's contribution (x_out - x)
-within 2e-3 of its largest magnitude (1e-2 where groups run as fp16
-matrix-core GEMMs); the mean absolute error is printed.
+within 2e-3 of its largest magnitude (4e-3 where groups run as fp16
+matrix-core GEMMs: seven roundings to 11 bits); the mean absolute error is
+printed.
 """
 import numpy as np
 import pytest
@@ -17,7 +18,7 @@ from vireo_amd import workloads as W
 
 pytestmark = pytest.mark.gpu
 TOL = 2e-3
-TOL_BF16 = 1e-2  # calls of >= 64 tokens: every group as fp16 GEMMs
+TOL_FP16 = 4e-3  # calls of >= 64 tokens: every group as fp16 GEMMs (test_prefill_tiles_and_scales derives it)
 
 
 @pytest.fixture
@@ -65,7 +66,7 @@ def test_moe_ffn_matches_oracle(cuda, oracle, path, name, T, plan):
     idx, w = m.forward(0, xt, torch.from_numpy(hb).to(cuda), return_routing=True)
     xo, io, wo, _ = oracle_layer(oracle, m, 0, x, hb)
     # calls of >= 64 tokens run every group as fp16 matrix-core GEMMs under plans 0 and 2
-    tol = TOL_BF16 if T >= 64 and plan in (0, 2) else TOL
+    tol = TOL_FP16 if T >= 64 and plan in (0, 2) else TOL
     check(f"{name} T={T} plan={plan}", x, xt.cpu().numpy(), xo, idx.cpu().numpy(), io, tol=tol)
     np.testing.assert_allclose(w.cpu().numpy(), wo, rtol=1e-5)
     m.close()
@@ -334,7 +335,7 @@ def test_unregistered_expert_is_skipped(cuda, oracle, path, name, plan, T):
     idx, _ = m.forward(0, xt, torch.from_numpy(hb[:T]).to(cuda), return_routing=True)
     xo, io, _, _ = oracle_layer(oracle, m, 0, x[:T], hb[:T])
     check(f"unregistered {name} plan={plan} T={T}", x[:T], xt.cpu().numpy(), xo, idx.cpu().numpy(), io,
-          tol=TOL_BF16 if T >= 64 else TOL)
+          tol=TOL_FP16 if T >= 64 else TOL)
     m.close()
 
 
@@ -409,7 +410,7 @@ def test_prefill_2048_zipf(cuda, oracle):
         oi[t] = oracle.topk(oracle.softmax(lg), shape.k, shape.renorm)[0]
     np.testing.assert_array_equal(ig, oi)
     xo, io, _, _ = oracle_layer(oracle, m, 0, x, hb)
-    check("prefill, all 2048 tokens", x, xt.cpu().numpy(), xo, ig, io, tol=TOL_BF16)
+    check("prefill, all 2048 tokens", x, xt.cpu().numpy(), xo, ig, io, tol=TOL_FP16)
     m.close()
 
 
@@ -457,7 +458,7 @@ def test_grouped_plan_large_groups(cuda, oracle, path, name, T, zipf, plan):
     if zipf:
         assert counts.max() > 128, counts.max()
     xo, io, _, _ = oracle_layer(oracle, m, 0, x, hb)
-    check(f"{name} T={T} plan={plan}", x, outs[0], xo, ig, io, tol=TOL_BF16 if plan == 0 else TOL)
+    check(f"{name} T={T} plan={plan}", x, outs[0], xo, ig, io, tol=TOL_FP16 if plan == 0 else TOL)
     m.close()
 
 
@@ -695,7 +696,7 @@ def test_grouped_plan_large_groups_unregistered(cuda, oracle, path):
     idx, _ = m.forward(0, xt, torch.from_numpy(hb).to(cuda), return_routing=True)
     assert (ig == big[0]).any(axis=1).sum() >= 16  # the dropped expert had a matrix-core group
     xo, io, _, _ = oracle_layer(oracle, m, 0, x, hb)
-    check("unregistered large groups, all tokens", x, xt.cpu().numpy(), xo, idx.cpu().numpy(), io, tol=TOL_BF16)
+    check("unregistered large groups, all tokens", x, xt.cpu().numpy(), xo, idx.cpu().numpy(), io, tol=TOL_FP16)
     m.close()
 
 

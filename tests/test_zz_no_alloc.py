@@ -3,7 +3,7 @@
 moe_ffn_forward's bit for bit on the same inputs (the same kernels run), on
 consecutive calls whose second is smaller than the first, on every plan it
 takes (matrix-core GEMMs on GGUF rows and on packed Q8_0 fragments, the
-matrix-core decode batch on packed tiles, register-input groups, the decode
+matrix-core decode batch on packed tiles and on Q8_0 fragments, the decode
 plan for a batch of tokens and for one token);
 it refuses calls whose intermediates exceed the region (-E2BIG) and layers
 that are not pinned yet (-EINVAL), and it allocates no device memory."""
@@ -91,7 +91,8 @@ def test_noalloc_matches_moe_ffn_forward(cuda, lib):
 def test_noalloc_q8_fragments(cuda, lib):
     """Q8_0 experts: calls of 64+ tokens on the matrix-core GEMMs reading the
     packed operand fragments the first moe_ffn_forward made, 20 tokens on the
-    register-input groups and 6 on the decode plan for a batch."""
+    matrix-core decode batch, which reads them too, and 6 on the decode plan for a
+    batch."""
     shape = W.SHAPES["olmoe-q8_0"]
     m = M.DeviceMoE(shape, 1, seed=93)
     try:

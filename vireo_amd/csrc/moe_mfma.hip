@@ -14,7 +14,7 @@
 // per (pair, 32 columns) by the block's largest. A weight is formed from its
 // exact quant by packed fp16 operations: Q8_0 and Q6_K (q - 32) times the
 // rounded scale, Q4_K one fused d1 q - m1 on the rounded d1 and m1. On the
-// benchmark's shapes the layer's output lies 5 to 8 times closer to a 64-bit
+// benchmark's shapes the layer's output lies 4 to 8 times closer to a 64-bit
 // evaluation than with both operands rounded to bf16, and a weight costs 1.5
 // (Q8_0), 1.6 (Q4_K) or 2.4 (Q6_K) vector instructions where bf16 rounding
 // through fp32 took 2.8 to 4.
