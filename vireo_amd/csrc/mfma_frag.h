@@ -266,8 +266,8 @@ struct Frag {
 // its own part of LDS (Lds: the pair being multiplied), where every lane finds the
 // words of its row. A lane per row touched 64 lines with every load instruction,
 // and rearranging what it read took more vector instructions than the multiplies
-// leave time for: Qwen3 Q4_K_M 2048 tokens gate/up 331 -> 206 us, down 372 -> 154
-// (from the packed copy 158 and 107); Q8_0 323 -> 247 and 166 -> 151 (170 and 107).
+// leave time for: Qwen3 Q4_K_M 2048 tokens gate/up 330 -> 200 us, down 367 -> 151
+// (from the packed copy 154 and 107); Q8_0 329 -> 236 and 168 -> 147 (169 and 107).
 // Q8_0's pieces are those of the row, 8-byte aligned, not of its 34-byte blocks:
 // loads at odd multiples of 2 bytes ran at half the rate.
 //   load(r, B, rb, t, lane)  requests pair t of the rows at B[0], B[1] (the

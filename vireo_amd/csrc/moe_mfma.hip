@@ -506,7 +506,7 @@ VH_DEV void gemm_tile(TileLds<T, GATEUP, LDB, PK> &L, const GemmArgs &a, gbyte *
 // 128-row tiles): a K step takes 1.5 us of a CU's two workgroups where its
 // multiplies need 1.0 at the clock it runs at (2.0 GHz), and a workgroup spends
 // 6 us before its first step (a chain of four loads) and 8 (gate/up) or 6
-// (down) after its last; gate/up 514 -> 250 us, down 381 -> 180 us against the
+// (down) after its last; gate/up 514 -> 262 us, down 381 -> 182 us against the
 // kernel whose waves were split into staging and multiplying ones.
 template <int T, bool GATEUP, int BMAX, bool PK>
 __global__ void __launch_bounds__(kThreads, BMAX == kBigTile || !PK ? 2 : 3) mfma_gemm_kernel(GemmArgs a) {
