@@ -580,8 +580,9 @@ def test_large_finite_inputs(cuda, T):
 
 
 # gate/up and down types; fe = 1152 and 1280 take more than the 32 blocks of h
-# whose factors the down GEMM holds at a time
-EDGE_TYPES = [(W.Q4_K, W.Q6_K, 512), (W.Q8_0, W.Q8_0, 1152), (W.Q6_K, W.Q4_K, 1280)]
+# whose factors the down GEMM holds at a time, 128 and 256 are the fewest K steps
+EDGE_TYPES = [(W.Q4_K, W.Q6_K, 512), (W.Q8_0, W.Q8_0, 1152), (W.Q6_K, W.Q4_K, 1280), (W.Q8_0, W.Q8_0, 128),
+              (W.Q4_K, W.Q6_K, 256)]
 
 
 @pytest.mark.parametrize("tg,td,fe", EDGE_TYPES)
